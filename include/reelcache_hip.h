@@ -20,7 +20,7 @@
 extern "C" {
 #endif
 
-#define RCH_ABI_VERSION 12
+#define RCH_ABI_VERSION 13
 
 /* Status codes (mapped to reelcache errors by the host). */
 #define RCH_OK 0
@@ -182,6 +182,19 @@ int rch_basis_pack(const rch_pack* packs_dev, int n_packs, int64_t max_nblocks, 
  */
 int rch_coefficient_bound(const rch_job* jobs_dev, int n_jobs, const int32_t* tiles_dev, int n_tiles,
                           int max_rank, int32_t* scratch_dev, void* stream);
+
+/*
+ * Codes of picture sources (channel_tiles.v1, any segments) or uint8 rows of any strides into
+ * row-major uint8 rows: job j's token t, column k < rank goes to byte dst_ptr + t *
+ * dst_token_stride + k (dst_ptr and dst_token_stride multiples of 16, dst_token_stride >= rank
+ * rounded up to 16; columns up to that are written as zeros).  Of a job only tokens, rank, the grid,
+ * the source fields, dst_ptr, dst_token_stride and RCH_JF_PIC_VEC4 are read; pic_slots == 0 marks
+ * uint8 rows.  tiles_dev int32 [n_tiles, 2]: (job, first token) of every 128-token tile.
+ * Replaces _unpack_kernel's gather (reelcache/restore_kernels.py:1518-1554) for ranks whose
+ * restore kernel takes rows only.
+ */
+int rch_codes_unpack(const rch_job* jobs_dev, int n_jobs, const int32_t* tiles_dev, int n_tiles, int max_rank,
+                     void* stream);
 
 /*
  * The fused restore: gather / dequantize coefficients, rank-view product on

@@ -16,7 +16,7 @@ import numpy as np
 from .errors import ConfigurationError, UnsupportedError
 
 LIBRARY = Path(__file__).resolve().with_name("libreelcache_hip.so")
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 # Status codes (RCH_E_*).
 OK, E_CONFIG, E_UNSUPPORTED, E_LAUNCH = 0, 1, 2, 3
@@ -71,6 +71,7 @@ _SIGNATURES = {
     "rch_fragment_bytes": ([_i], _i),
     "rch_basis_pack": ([_p, _i, _i64, _i64, _i, _p], _i),
     "rch_coefficient_bound": ([_p, _i, _p, _i, _i, _p, _p], _i),
+    "rch_codes_unpack": ([_p, _i, _p, _i, _i, _p], _i),
     "rch_restore": ([_p, _i, _p, _i, _p, _i, _i, _i, _i, _i, _i, _i, _i, _p, _p], _i),
     "rch_restore_occupancy": ([_i, _i, _i, _i, _i, _i, ctypes.POINTER(_i)], _i),
     "rch_restore_pair": ([_p, _i, _p, _i, _i, _p, _i, _i, _i, _i, _i, _i, _i, _i, _p, _p], _i),

@@ -329,6 +329,112 @@ __global__ void __launch_bounds__(256) coefficient_bound_kernel(const rch_job* _
 }
 
 // ---------------------------------------------------------------------------------------------
+// Codes of picture (or unaligned uint8) sources -> 16-byte aligned uint8 rows
+// ---------------------------------------------------------------------------------------------
+
+typedef unsigned int u4_unaligned __attribute__((ext_vector_type(4), aligned(1)));
+
+// 4 x 4 byte transpose: out[t] holds byte t of d[0..3].
+__device__ __forceinline__ void transpose4(const uint32_t (&d)[4], uint32_t (&out)[4]) {
+    const uint32_t a = __builtin_amdgcn_perm(d[1], d[0], 0x05010400u);  // d0.0 d1.0 d0.1 d1.1
+    const uint32_t b = __builtin_amdgcn_perm(d[1], d[0], 0x07030602u);  // d0.2 d1.2 d0.3 d1.3
+    const uint32_t c = __builtin_amdgcn_perm(d[3], d[2], 0x05010400u);
+    const uint32_t e = __builtin_amdgcn_perm(d[3], d[2], 0x07030602u);
+    out[0] = __builtin_amdgcn_perm(c, a, 0x05040100u);
+    out[1] = __builtin_amdgcn_perm(c, a, 0x07060302u);
+    out[2] = __builtin_amdgcn_perm(e, b, 0x05040100u);
+    out[3] = __builtin_amdgcn_perm(e, b, 0x07060302u);
+}
+
+// Workgroup: 128 tokens x 128 rank columns of one job; thread = 16 columns of 4 tokens, so 16
+// loads are in flight and every store is a 16-byte piece of a row.  Columns past the rank inside a
+// 16-column group are written as zeros; groups past the rank are not written (nor read).
+// Latency-bound and a small share of a restore: the rows are 1 byte per coefficient against
+// 2 C bytes per token of output.
+__global__ void __launch_bounds__(256) codes_unpack_kernel(const rch_job* __restrict__ jobs,
+                                                           const int32_t* __restrict__ tiles) {
+    const rch_job* J = jobs + tiles[2 * blockIdx.x];
+    const int t0 = tiles[2 * blockIdx.x + 1];
+    const int c0 = 128 * blockIdx.y;
+    const int rank = static_cast<int>(J->rank);
+    if (c0 >= rank) return;  // whole workgroup
+    const int tokens = static_cast<int>(J->tokens);
+    const int lane = threadIdx.x & 31, g = threadIdx.x >> 5;  // token lane, 16-column group
+    const int k0 = c0 + 16 * g;
+    const int64_t pitch = J->dst_token_stride;
+    RCH_GLOBAL uint8_t* const rows = gout<uint8_t>(J->dst_ptr) + k0;
+    if (J->pic_slots == 0) {  // uint8 rows of any stride
+        const int64_t rs = J->src_row_stride, cs = J->src_col_stride;
+        if (k0 >= rank) return;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int token = t0 + 32 * t + lane;
+            if (token >= tokens) continue;
+            const RCH_GLOBAL uint8_t* from = gin<uint8_t>(J->src_ptr) + token * rs + k0 * cs;
+            u4 out = {0u, 0u, 0u, 0u};
+            if (cs == 1 && k0 + 16 <= rank) {
+                out = *reinterpret_cast<const RCH_GLOBAL u4_unaligned*>(from);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if (k0 + i < rank) out[i >> 2] |= static_cast<uint32_t>(from[i * cs]) << (8 * (i & 3));
+            }
+            *reinterpret_cast<RCH_GLOBAL u4*>(rows + token * pitch) = out;
+        }
+        return;
+    }
+    // Offset of every column's cell within its frame's picture, and its segment's first table entry.
+    __shared__ int64_t cell[128];
+    __shared__ int first[128];
+    if (threadIdx.x < 128) {
+        const int k = min(c0 + static_cast<int>(threadIdx.x), rank - 1);
+        const int slots = static_cast<int>(J->pic_slots), planes = static_cast<int>(J->pic_planes);
+        const int segment = k / slots, slot = k - segment * slots;
+        const int plane = slot % planes, index = slot / planes, cols = static_cast<int>(J->pic_grid_cols);
+        const int cell_row = index / cols, cell_col = index - cell_row * cols;
+        cell[threadIdx.x] = plane * J->pic_plane_stride + static_cast<int64_t>(cell_row) * J->grid_h * J->pic_row_stride +
+                            static_cast<int64_t>(cell_col) * J->grid_w;
+        first[threadIdx.x] = segment * static_cast<int>(J->frames);
+    }
+    __syncthreads();
+    if (k0 >= rank) return;
+    const RCH_GLOBAL uint8_t* const base = gin<uint8_t>(J->src_ptr);
+    const RCH_GLOBAL int64_t* const table = gin<int64_t>(J->pic_table_ptr);
+    if (J->flags & RCH_JF_PIC_VEC4) {  // 4 tokens of a cell row per 32-bit load (tokens % 4 == 0)
+        const int token = t0 + 4 * lane;
+        if (token >= tokens) return;
+        const Coords xy = coords(J, token);
+        const int64_t at = xy.y * J->pic_row_stride + xy.x;
+        uint32_t d[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {  // columns past the rank re-read the last one (clamped above)
+            const uint32_t v = *reinterpret_cast<const RCH_GLOBAL uint32_t*>(base + table[first[16 * g + i] + xy.f] + at + cell[16 * g + i]);
+            d[i] = k0 + i < rank ? v : 0u;
+        }
+        uint32_t out[4][4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) transpose4({d[4 * q], d[4 * q + 1], d[4 * q + 2], d[4 * q + 3]}, out[q]);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            *reinterpret_cast<RCH_GLOBAL u4*>(rows + (token + t) * pitch) = u4{out[0][t], out[1][t], out[2][t], out[3][t]};
+        return;
+    }
+    for (int t = 0; t < 4; ++t) {
+        const int token = t0 + 32 * t + lane;
+        if (token >= tokens) continue;
+        const Coords xy = coords(J, token);
+        const int64_t at = xy.y * J->pic_row_stride + xy.x;
+        u4 out = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const uint32_t v = base[table[first[16 * g + i] + xy.f] + at + cell[16 * g + i]];
+            out[i >> 2] |= (k0 + i < rank ? v : 0u) << (8 * (i & 3));
+        }
+        *reinterpret_cast<RCH_GLOBAL u4*>(rows + token * pitch) = out;
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
 // Dense rows -> RoPE -> cast -> store
 // ---------------------------------------------------------------------------------------------
 
@@ -509,6 +615,15 @@ int rch_coefficient_bound(const rch_job* jobs_dev, int n_jobs, const int32_t* ti
     hipLaunchKernelGGL(coefficient_bound_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, as_stream(stream),
                        jobs_dev, tiles_dev, k_tiles, scratch_dev);
     return check_launch("rch_coefficient_bound");
+}
+
+int rch_codes_unpack(const rch_job* jobs_dev, int n_jobs, const int32_t* tiles_dev, int n_tiles, int max_rank,
+                     void* stream) {
+    if (!jobs_dev || !tiles_dev || n_jobs <= 0 || n_tiles <= 0 || max_rank <= 0 || (max_rank + 127) / 128 > 65535)
+        return fail(RCH_E_CONFIG, "rch_codes_unpack: invalid arguments");
+    hipLaunchKernelGGL(codes_unpack_kernel, dim3(static_cast<unsigned>(n_tiles), static_cast<unsigned>((max_rank + 127) / 128)),
+                       dim3(256), 0, as_stream(stream), jobs_dev, tiles_dev);
+    return check_launch("rch_codes_unpack");
 }
 
 // The kernel an rch_restore launch group runs: the straight-line variant (restore_fast.h) when

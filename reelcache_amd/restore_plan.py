@@ -441,14 +441,16 @@ class _Layout:
                 self.picture_tables.append((index, at))
                 rows[index, _C_PIC_TABLE], relative[index, _C_PIC_TABLE] = at, 1
         self.staged_rows = np.zeros(len(descs), dtype=np.int64)
-        plans = self._launch_groups(descs, rows, arena, device, basis_groups)
+        kinds = [desc.kind for desc in descs]
+        rows, relative = self._unpack_layout(descs, kinds, rows, relative, arena)
+        plans = self._launch_groups(descs, kinds, rows, arena, device, basis_groups)
         self.staged_rows_offset = arena.add(self.staged_rows) if staged else None
         packs, pack_of = self._packs(descs, plans, basis_groups, arena)
         self._pack_layout(descs, rows, relative, plans, packs, pack_of)
         self.bound_tiles = _tiles(self.bound_jobs, descs) if self.bound_jobs else None
         self.bound_tile_offset = arena.add(self.bound_tiles) if self.bound_jobs else None
         self.packs_offset = arena.reserve(len(packs) * _lib.PACK_DTYPE.itemsize) if packs else None
-        self.desc_offset = arena.reserve(len(descs) * _N_FIELDS * 8)
+        self.desc_offset = arena.reserve(len(rows) * _N_FIELDS * 8)
         self.arena_bytes = (arena.size + 255) // 256 * 256
         if not self.static:
             for index, pack_index in pack_of.items():
@@ -458,7 +460,8 @@ class _Layout:
             self.template[offset:offset + array.nbytes] = array.reshape(-1).view(np.uint8)
         self.plans, self.jobs = plans, len(descs)
         self.scratch_words = self.exp_words + len(descs)
-        self.buffer_bytes = self.arena_bytes + self.pack_total + 4 * self.scratch_words + 256
+        self.codes_offset = (self.arena_bytes + self.pack_total + 4 * self.scratch_words + 255) // 256 * 256
+        self.buffer_bytes = self.codes_offset + self.codes_total + 256
         # Pack-table and pack-pointer offsets are relative to the buffer base.
         pack_rows = np.zeros((len(packs), len(_lib.PACK_FIELDS)), dtype=np.int64)
         pack_relative = np.zeros_like(pack_rows)
@@ -477,8 +480,60 @@ class _Layout:
             self.pack_sources.append(pack["member"])
         self.pack_rows, self.pack_relative = pack_rows, pack_relative
         self.rows, self.rows_relative = rows, relative
+        for position, (index, at) in enumerate(self.unpacked):
+            # The restore reads the rows the unpack row writes.
+            rows[index, _C_SRC_PTR] = rows[len(descs) + position, _C_DST_PTR] = self.codes_offset + at
         self.table_jobs = [i for i, d in enumerate(descs) if d.table is not None]
         self.host_bound_jobs = [i for i, d in enumerate(descs) if self.fp16_mode and d.host_bound is not None]
+
+    def _unpack_layout(self, descs, kinds, rows, relative, arena):
+        """Jobs whose codes are unpacked into aligned rows first (``rch_codes_unpack``): 16-bit modes'
+        ranks beyond one wave's registers, which the rank-halves kernel takes from uint8 rows only.
+        Without it they run the chunked general kernel, which converts (and gathers) a tile's codes
+        again for every 32-channel block: two chunks of K and V, 32 x 128 channels, ranks 256-512,
+        from pictures take 4.24 ms there and 0.19 ms here (MI355X).  Smaller ranks stay as they are: the straight-line kernels gather
+        pictures themselves.  Appends an unpack row per such job to the tables; its rows and
+        ``kinds`` entry become those of an aligned uint8 source."""
+        self.unpacked, self.codes_total, self.unpack_rank = [], 0, 0
+        config, precision = self.config, self.precision
+        limit = _FAST_MAX_KSTEPS[precision] if precision in _FAST_MAX_KSTEPS else 0
+        if (self.staged or self.static or not limit or not _config_value(config, "fast_variant")
+                or not _config_value(config, "split_rank")):
+            return rows, relative
+        extra, extra_relative, members = [], [], []
+        for index, desc in enumerate(descs):
+            row = rows[index]
+            if not (desc.kind == _lib.SRC_PICTURE or (desc.kind == _lib.SRC_U8 and not row[_C_FLAGS] & _lib.JF_SRC_VEC)):
+                continue
+            if not limit < (desc.rank + 15) // 16 <= _SPLIT_MAX_KSTEPS:
+                continue
+            aligned = row.copy()
+            aligned[_C_FLAGS] = (row[_C_FLAGS] | _lib.JF_SRC_VEC) & ~_lib.JF_PIC_VEC4
+            if not _fast_eligibility(_lib.SRC_U8, desc.head_dim, desc.table is not None, aligned, precision):
+                continue
+            pitch = (desc.rank + 15) // 16 * 16
+            unpack, shifts = row.copy(), relative[index].copy()
+            unpack[_C_DST_TOKEN] = pitch
+            shifts[_C_DST_PTR] = 1
+            extra.append(unpack)
+            extra_relative.append(shifts)
+            aligned[_C_SRC_ROW], aligned[_C_SRC_COL] = pitch, 1
+            aligned[[_C_PIC_SLOTS, _C_PIC_TABLE]] = 0
+            rows[index] = aligned
+            relative[index, _C_PIC_TABLE] = 0
+            relative[index, _C_SRC_PTR] = 1
+            kinds[index] = _lib.SRC_U8
+            members.append(index)
+            self.unpacked.append((index, self.codes_total))
+            self.unpack_rank = max(self.unpack_rank, desc.rank)
+            self.codes_total += (desc.tokens * pitch + 255) // 256 * 256
+        if not members:
+            return rows, relative
+        tiles = _tiles(members, descs)
+        positions = {index: len(descs) + position for position, index in enumerate(members)}
+        tiles[:, 0] = [positions[index] for index in tiles[:, 0].tolist()]
+        self.unpack_tiles = (arena.add(tiles), len(tiles))
+        return np.concatenate([rows, np.stack(extra)]), np.concatenate([relative, np.stack(extra_relative)])
 
     def _affine_layout(self, descs, rows, relative, arena):
         """One fp32 table of every job's (scale | offset) block, in job order; the rows' pointers."""
@@ -495,7 +550,7 @@ class _Layout:
             relative[index, _C_SCALE] = relative[index, _C_OFFSET] = 1
             first += size
 
-    def _launch_groups(self, descs, rows, arena, device, basis_groups):
+    def _launch_groups(self, descs, kinds, rows, arena, device, basis_groups):
         """Launch groups (source kind, dtypes, head geometry, rank class, straight-line eligibility)
         and the kernel variant, grid and work tables of each."""
         precision, config = self.precision, self.config
@@ -508,9 +563,9 @@ class _Layout:
         allow_stream = allow_fast and bool(_config_value(config, "stream_variant")) and precision == "fp16x2"
         groups: dict = {}
         for index, desc in enumerate(descs):
-            flags = (_fast_eligibility(desc.kind, desc.head_dim, desc.table is not None, rows[index], precision)
+            flags = (_fast_eligibility(kinds[index], desc.head_dim, desc.table is not None, rows[index], precision)
                      if allow_fast else 0)
-            key = (desc.kind, desc.dtype, desc.out_dtype, desc.head_dim, desc.channels,
+            key = (kinds[index], desc.dtype, desc.out_dtype, desc.head_dim, desc.channels,
                    _rank_steps_class(precision, desc.rank), None if desc.table is None else desc.rope_kind == "dense",
                    flags)
             groups.setdefault(key, []).append(index)
@@ -747,8 +802,16 @@ class _Layout:
         buffer = torch.empty(self.buffer_bytes, dtype=torch.uint8, device=device)
         base = buffer.data_ptr()
         rows = self.rows + self.rows_relative * base
-        rows[:, _C_DST_PTR] = dst
-        rows[:, _C_SRC_PTR] = src
+        count = len(descs)
+        if not self.unpacked:
+            rows[:, _C_DST_PTR] = dst
+            rows[:, _C_SRC_PTR] = src
+        else:  # unpacked jobs read the call buffer's rows, their unpack rows the source
+            codes = rows[:count, _C_SRC_PTR].copy()
+            rows[:count, _C_DST_PTR] = dst
+            rows[:count, _C_SRC_PTR] = src
+            for position, (index, _) in enumerate(self.unpacked):
+                rows[index, _C_SRC_PTR], rows[count + position, _C_SRC_PTR] = codes[index], src[index]
         tables: dict = {}
         for index in self.table_jobs:
             table = descs[index].table
@@ -804,6 +867,10 @@ class _Layout:
         if self.bound_jobs:
             _lib.call("rch_coefficient_bound", table, jobs, base + self.bound_tile_offset, len(self.bound_tiles),
                       int(max(self.rows[i, _C_RANK] for i in self.bound_jobs)), scratch_base, hip_stream)
+            launches += 1
+        if self.unpacked:
+            _lib.call("rch_codes_unpack", table, len(self.rows), base + self.unpack_tiles[0], self.unpack_tiles[1],
+                      self.unpack_rank, hip_stream)
             launches += 1
         for plan in self.plans:
             variant = plan["variant"]

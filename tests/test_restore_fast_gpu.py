@@ -198,3 +198,39 @@ def test_fast_picture_segments(device, grid, rank, heads):
     assert _run(cases[1], "fp16x2", "general") == ["general"]
     assert np.array_equal(written(cases[0]), written(cases[1]))
     _check_bound(cases[0], "fp16x2")
+
+
+# (grid, heads, head_dim, rank, rope, precision, source form): ranks beyond one wave's registers from
+# sources that are not aligned uint8 rows
+UNPACK_SHAPES = [
+    ((2, 12, 16), 4, 64, 208, "none", "fp16x2", "pictures"),         # word gather, 13 rank steps
+    ((2, 9, 13), 4, 128, 300, "separable", "fp16x2", "pictures"),    # byte gather, ragged columns and last tile
+    ((1, 1100, 3), 9, 32, 264, "none", "fp16", "pictures"),           # two segments of 210 cells
+    ((1, 11, 13), 5, 128, 512, "dense", "bf16", "pictures"),         # the largest rank, a part tile
+    ((2, 12, 14), 4, 64, 201, "separable", "fp16x2", 201),           # rows of 201 bytes
+    ((1, 16, 9), 3, 128, 257, "none", "fp16", 260),                  # one column past 16 rank steps
+]
+
+
+@pytest.mark.parametrize("shape", UNPACK_SHAPES)
+def test_unpacked_sources_match_aligned_rows(device, shape):
+    """High-rank pictures and unaligned rows are unpacked into aligned rows and run the rank-halves
+    kernel: bit for bit the restore of the same codes in aligned rows, within the oracle's bound;
+    with rank halves off they run the general kernel."""
+    grid, heads, head_dim, rank, rope, precision, form = shape
+    cases = []
+    for source, pitch, origin in (("uint8", -(-rank // 16) * 16, None),
+                                  ("pictures" if form == "pictures" else "uint8", None if form == "pictures" else form,
+                                   (0, 0) if grid[2] % 4 == 0 else (2, 3))):
+        rng = np.random.default_rng(71)
+        extra = {} if origin is None else {"picture_origin": origin, "picture_pad": (3, 4) if origin == (0, 0) else (3, 5)}
+        cases.append(make_case(rng, grid=grid, heads=heads, head_dim=head_dim, rank=rank, source=source, rope=rope,
+                               out_dtype="bfloat16", device=device, token_offset=3, code_pitch=pitch, **extra))
+    rows, other = cases
+    assert _run(rows, precision, "pairs") == ["split"] and _run(other, precision, "pairs") == ["split"]
+    assert np.array_equal(written(other), written(rows))
+    _check_bound(other, precision)
+    handle = rk.reconstruct([other.job], precision=precision, config={"split_rank": False})
+    handle.release()
+    assert handle.stats["variants"] == ["general"]
+    _check_bound(other, precision)
