@@ -438,16 +438,125 @@ __global__ void __launch_bounds__(256) codes_unpack_kernel(const rch_job* __rest
 // Dense rows -> RoPE -> cast -> store
 // ---------------------------------------------------------------------------------------------
 
+// Eight consecutive elements of a 16-byte aligned row as floats.
+template <int DT>
+struct Raw8 {
+    u4 w[DT == RCH_DT_F32 ? 2 : 1];
+};
+template <int DT>
+__device__ __forceinline__ Raw8<DT> load_raw8(const RCH_GLOBAL u4* p) {
+    Raw8<DT> r;
+    r.w[0] = p[0];
+    if constexpr (DT == RCH_DT_F32) r.w[1] = p[1];
+    return r;
+}
+template <int DT>
+__device__ __forceinline__ void unpack_raw8(const Raw8<DT>& r, float (&v)[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        if constexpr (DT == RCH_DT_F32) v[i] = __uint_as_float(r.w[i >> 2][i & 3]);
+        else if constexpr (DT == RCH_DT_F16) v[i] = static_cast<float>(__builtin_bit_cast(h8, r.w[0])[i]);
+        else v[i] = static_cast<float>(__builtin_bit_cast(bf8, r.w[0])[i]);
+    }
+}
+template <int OUT>
+__device__ __forceinline__ void store_raw8(RCH_GLOBAL u4* p, const float (&v)[8]) {
+    if constexpr (OUT == RCH_DT_F32) {
+        p[0] = __builtin_bit_cast(u4, (f4{v[0], v[1], v[2], v[3]}));
+        p[1] = __builtin_bit_cast(u4, (f4{v[4], v[5], v[6], v[7]}));
+    } else if constexpr (OUT == RCH_DT_F16) {
+        h8 out;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) out[i] = static_cast<_Float16>(v[i]);
+        p[0] = __builtin_bit_cast(u4, out);
+    } else {
+        bf8 out;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) out[i] = static_cast<__bf16>(v[i]);
+        p[0] = __builtin_bit_cast(u4, out);
+    }
+}
+
+// Aligned rows and slots: a work item is 8 channels (one dim chunk) of a token in up to four heads.
+// Lanes run over the dim chunks of a head and then over tokens, so a wave moves whole 16 * head_dim
+// byte runs, the four heads' loads are in flight together and one set of (cos, sin) serves them.
+template <int SRC, int OUT>
+__device__ __forceinline__ void rope_store_rows(const rch_job* J, int64_t t0, int block, int blocks, int channels,
+                                                int head_dim) {
+    constexpr int kHeads = 4;
+    constexpr int kSrcBytes = SRC == RCH_DT_F32 ? 4 : 2, kOutBytes = OUT == RCH_DT_F32 ? 4 : 2;
+    const int rope = static_cast<int>(J->rope);
+    const int chunks = head_dim >> 3, heads = channels / head_dim;
+    const int items = kTileTokens * chunks * ((heads + kHeads - 1) / kHeads);
+    for (int u = block * 256 + static_cast<int>(threadIdx.x); u < items; u += blocks * 256) {
+        const int rest = u / chunks, chunk = u - rest * chunks;
+        const int64_t t = t0 + rest % kTileTokens;
+        const int head = kHeads * (rest / kTileTokens);
+        if (t >= J->tokens) continue;
+        const int64_t src = J->src_ptr + (t * J->src_row_stride + static_cast<int64_t>(head) * head_dim + 8 * chunk) * kSrcBytes;
+        Raw8<SRC> raw[kHeads];
+#pragma unroll
+        for (int x = 0; x < kHeads; ++x)
+            if (head + x < heads) raw[x] = load_raw8<SRC>(gin<u4>(src + static_cast<int64_t>(x) * head_dim * kSrcBytes));
+        f4 cv, sv;
+        if (rope != RCH_ROPE_NONE) {
+            const Coords c = coords(J, static_cast<int>(t));
+            const int j0 = 4 * chunk;
+            const int64_t rs = J->rope_row_stride;
+            const RCH_GLOBAL float* cos_t = gin<float>(J->cos_ptr);
+            const RCH_GLOBAL float* sin_t = gin<float>(J->sin_ptr);
+            const int64_t s0 = J->sec_t, s1 = J->sec_t + J->sec_h;
+            const int first = (j0 >= s0) + (j0 >= s1), last = (j0 + 3 >= s0) + (j0 + 3 >= s1);
+            if ((J->flags & RCH_JF_ROPE_VEC) && (rope == RCH_ROPE_DENSE || first == last)) {
+                const int64_t at = rope_row(J, rope, j0, t, c.f, c.y, c.x) * rs + j0;
+                cv = *reinterpret_cast<const RCH_GLOBAL f4*>(cos_t + at);
+                sv = *reinterpret_cast<const RCH_GLOBAL f4*>(sin_t + at);
+            } else {
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    const int64_t at = rope_row(J, rope, j0 + p, t, c.f, c.y, c.x) * rs + j0 + p;
+                    cv[p] = cos_t[at];
+                    sv[p] = sin_t[at];
+                }
+            }
+        }
+        const int64_t dst = J->dst_ptr + (t * J->dst_token_stride + head * J->dst_head_stride + 8 * chunk) * kOutBytes;
+#pragma unroll
+        for (int x = 0; x < kHeads; ++x) {
+            if (head + x >= heads) continue;
+            float v[8];
+            unpack_raw8<SRC>(raw[x], v);
+            if (rope != RCH_ROPE_NONE) {
+#pragma unroll
+                for (int p = 0; p < 4; ++p) rotate(v[2 * p], v[2 * p + 1], cv[p], sv[p]);
+            }
+            store_raw8<OUT>(gout<u4>(dst + x * J->dst_head_stride * kOutBytes), v);
+        }
+    }
+}
+
+// HBM-bound: every value is read once and written once.  The c_tiles = ceil(channels / 64)
+// workgroups of a 128-token tile share its rows (aligned unit-stride rows and slots: one 16-byte
+// load per 8 values; three CausVid chunks of bf16 K, 43 MB in and 43 MB out, take 21 us against
+// 67 us through the element loads below, on MI355X), or each take 64 channels with element loads.
+template <int OUT>
 __global__ void __launch_bounds__(256) rope_store_kernel(const rch_job* __restrict__ jobs,
                                                          const int32_t* __restrict__ tiles, int c_tiles, int channels,
-                                                         int head_dim, int out_dtype) {
+                                                         int head_dim) {
     const int tile = blockIdx.x / c_tiles, ct = blockIdx.x - tile * c_tiles;
     const rch_job* J = jobs + tiles[2 * tile];
     const int64_t t0 = tiles[2 * tile + 1];
-    // 128 tokens x 64 channels per block: thread = (token pair of rows, 16 channels).
-    const int c0 = ct * 64 + (threadIdx.x & 3) * 16;
     const int rope = static_cast<int>(J->rope);
     const int dtype = static_cast<int>(J->src_dtype);
+    const int64_t row_bytes = J->src_row_stride * (dtype == RCH_DT_F32 ? 4 : 2);
+    if ((J->flags & RCH_JF_DST_VEC) && J->src_col_stride == 1 && ((J->src_ptr | row_bytes) & 15) == 0) {
+        if (dtype == RCH_DT_F32) rope_store_rows<RCH_DT_F32, OUT>(J, t0, ct, c_tiles, channels, head_dim);
+        else if (dtype == RCH_DT_F16) rope_store_rows<RCH_DT_F16, OUT>(J, t0, ct, c_tiles, channels, head_dim);
+        else rope_store_rows<RCH_DT_BF16, OUT>(J, t0, ct, c_tiles, channels, head_dim);
+        return;
+    }
+    // 128 tokens x 64 channels per block: thread = (token pair of rows, 16 channels).
+    const int c0 = ct * 64 + (threadIdx.x & 3) * 16;
     for (int rep = 0; rep < 2; ++rep) {
         const int64_t t = t0 + (threadIdx.x >> 2) + 64 * rep;
         if (t >= J->tokens || c0 >= channels) continue;
@@ -459,7 +568,7 @@ __global__ void __launch_bounds__(256) rope_store_kernel(const rch_job* __restri
             const Coords c = coords(J, static_cast<int>(t));
             apply_rope(J, rope, v, c0, channels, head_dim, t, c.f, c.y, c.x);
         }
-        store16(J, v, c0, channels, head_dim, t, out_dtype);
+        store16(J, v, c0, channels, head_dim, t, OUT);
     }
 }
 
@@ -815,8 +924,19 @@ int rch_rope_store(const rch_job* jobs_dev, int n_jobs, const int32_t* tiles_dev
     const int c_tiles = (channels + 63) / 64;
     const int64_t blocks = static_cast<int64_t>(n_tiles) * c_tiles;
     if (blocks > 0x7fffffff) return fail(RCH_E_CONFIG, "rch_rope_store: grid too large");
-    hipLaunchKernelGGL(rope_store_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, as_stream(stream),
-                       jobs_dev, tiles_dev, c_tiles, channels, head_dim, out_dtype);
+    const dim3 grid(static_cast<unsigned>(blocks));
+    hipStream_t s = as_stream(stream);
+    switch (out_dtype) {
+        case RCH_DT_F32:
+            hipLaunchKernelGGL(rope_store_kernel<RCH_DT_F32>, grid, dim3(256), 0, s, jobs_dev, tiles_dev, c_tiles, channels, head_dim);
+            break;
+        case RCH_DT_F16:
+            hipLaunchKernelGGL(rope_store_kernel<RCH_DT_F16>, grid, dim3(256), 0, s, jobs_dev, tiles_dev, c_tiles, channels, head_dim);
+            break;
+        default:
+            hipLaunchKernelGGL(rope_store_kernel<RCH_DT_BF16>, grid, dim3(256), 0, s, jobs_dev, tiles_dev, c_tiles, channels, head_dim);
+            break;
+    }
     return check_launch("rch_rope_store");
 }
 

@@ -253,3 +253,38 @@ def test_table_first_used_on_another_stream(device):
         for case in (first, second):
             values, bound = expected(case, "fp16x2")
             assert float((np.abs(written(case) - values) - bound).max()) <= 0
+
+
+@pytest.mark.parametrize("heads,head_dim,layout,rope_kind,grid", [(5, 80, "BHTD", "dense", (1, 11, 13)),
+                                                                  (4, 96, "BTHD", "separable", (2, 9, 15)),
+                                                                  (9, 32, "THD", "separable", (1, 16, 8)),
+                                                                  (1, 16, "BHTD", "none", (1, 1, 1))])
+@pytest.mark.parametrize("out_dtype", ["bfloat16", "float16", "float32"])
+def test_dense_rows_vector_and_element_paths_agree(device, heads, head_dim, layout, rope_kind, grid, out_dtype):
+    """Aligned dense rows (16-byte loads, four heads per work item) and the same values one element
+    off alignment (element loads) give the same bits: head counts beside multiples of four, section
+    boundaries inside a chunk's pairs, part tiles, one token."""
+    rng = np.random.default_rng(zlib.crc32(f"dense-vec/{heads}/{head_dim}/{out_dtype}".encode()))
+    tokens, channels = int(np.prod(grid)), heads * head_dim
+    positions, rope = None, None
+    if rope_kind != "none":
+        table, rows = _rope_table(rope_kind, head_dim, tokens, rng)
+        positions = rk.RopePositions(table, rows)
+        rope = orc.rope_cos_sin(table.cos.float().double().numpy(), table.sin.float().double().numpy(), table.sections,
+                                positions.rows, grid)
+    for source_dtype in (torch.float32, torch.bfloat16, torch.float16):
+        values = torch.from_numpy(rng.standard_normal((tokens, channels)).astype(np.float32) * 3).to(source_dtype)
+        shifted = torch.zeros((tokens, channels + 8), dtype=source_dtype, device=device)
+        shifted[:, 1:1 + channels] = values.to(device)
+        slots = []
+        for source in (values.to(device), shifted[:, 1:1 + channels]):
+            tensor = destination(layout, tokens, heads, head_dim, out_dtype, device, offset=2, extra=1, fill=-77.0)
+            job = rk.ReconstructionJob(rk.DenseSource(source), rk.NativeView(tensor, layout, token_offset=2), grid,
+                                       rope=positions)
+            rk.reconstruct([job]).synchronize()
+            slots.append(job.destination.slot(tokens).reshape(tokens, channels).double().cpu().numpy())
+            canonical = (tensor.transpose(1, 2) if layout == "BHTD" else tensor).reshape(-1, channels)
+            assert bool((canonical[:2] == -77.0).all()) and bool((canonical[2 + tokens:] == -77.0).all())
+        np.testing.assert_array_equal(slots[0], slots[1])
+        exact, bound = _rotation_bound(values.double().numpy(), heads, rope, out_dtype)
+        assert float((np.abs(slots[0] - exact) - bound).max()) <= 0
