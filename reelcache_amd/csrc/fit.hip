@@ -710,103 +710,173 @@ __global__ void __launch_bounds__(kThreads) quantize_batched_kernel(const rch_qu
 
 // ---------------------------------------------------------------------------------------------
 // Batched FP64 Cholesky factor and triangular inverse (the planner's CholeskyQR steps): one
-// 1024-thread workgroup per k x k matrix, whose upper triangle lives in LDS in packed row-major
-// form, with one workgroup barrier per factor column and one per inverse row.
+// 8-wave workgroup per k x k matrix, held in LDS (padded to whole 16-blocks with the identity).
+// Bound by the chain of dependent pivots, so the work is blocked by 16 to keep everything but that
+// chain off it: a column-at-a-time form with one workgroup barrier per factor column and per inverse
+// row took 202 us for 60 matrices of order 96 (44 for 32), this one 73 (19) us (MI355X).
 //
-// Factorization (right-looking): in step j every thread reads the pivot d = A[j][j], forms
-// 1 / sqrt(d) itself and applies the rank-1 update A[i][c] -= (A[j][i] / r)(A[j][c] / r) to its
-// share of the trailing triangle j < i <= c, reading row j unscaled (no thread writes row j in
-// step j).  The scaled row j = row j of R goes to a row buffer and is written back into the
-// triangle in step j + 1, when no thread reads row j.
+// Factorization, per 16-row panel: each wave holds the panel's diagonal block (lanes 0-15, one
+// column each; every wave factors it, so no barrier is needed inside a panel) and 48 further
+// columns (lanes 16-63); a step broadcasts the pivot and the pivot row's panel entries by readlane.
+// Two barriers per panel: before and after the trailing update A -= R_p^T R_p (16 x 16 tiles, four
+// elements per lane).
 //
-// Inverse X = R^-1, rows from the bottom: S[r][c] accumulates sum_{p > r} R[r][p] X[p][c] as rows
-// p are finished.  In step i, row i is final: X[i][c] = (delta_ic - S[i][c]) / R[i][i]; every
-// thread forms the values of row i it needs from S[i][c] and adds R[r][i] X[i][c] into S[r][c]
-// for its share of r < i <= c.  Row i of X goes to a row buffer and replaces row i of S in step
-// i - 1.  Lanes run over columns and waves over rows, so a wave's LDS accesses are one row of
-// consecutive doubles plus one broadcast word.
+// Inverse X = R^-1: wave J computes block column J from the bottom with no barrier.  Block (I, J)
+// sums S = sum_{I < P <= J} R_IP X_PJ (four rows per lane) and finishes by substitution in R_II (lane
+// = column).  X_PJ is kept in the unused lower triangle, at block (J, P).
+//
+// Every element's products are rounded, then added in one fixed order (factor: pivot rows
+// ascending; inverse: rows descending), whatever the blocking: no fused or matrix-unit products,
+// whose different rounding would move near-tied row signs of the planner's directions.
 // ---------------------------------------------------------------------------------------------
 
-constexpr int kCholThreads = 1024;
+constexpr int kCholThreads = 512;
 constexpr int kCholWaves = kCholThreads / 64;
-constexpr int kCholPacked = RCH_CHOLESKY_MAX_K * (RCH_CHOLESKY_MAX_K + 1) / 2;
+constexpr int kCholBlocks = RCH_CHOLESKY_MAX_K / 16;
+constexpr int kCholPitch = RCH_CHOLESKY_MAX_K + 1;
+static_assert(RCH_CHOLESKY_MAX_K % 16 == 0 && kCholBlocks <= kCholWaves, "one wave per block column");
 
-// Offset of (i, c), i <= c, in a packed upper triangle of order k (rows i = 0.. stored back to back).
-__device__ __forceinline__ int packed_at(int i, int c, int k) { return i * k - (i * (i - 1)) / 2 + (c - i); }
+__device__ __forceinline__ double broadcast_lane(double v, int lane) {
+    const u2 w = __builtin_bit_cast(u2, v);
+    return __builtin_bit_cast(double, (u2{static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(w[0]), lane)),
+                                          static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(w[1]), lane))}));
+}
 
 __global__ void __launch_bounds__(kCholThreads) cholesky_inverse_kernel(const double* __restrict__ a,
                                                                          double* __restrict__ x,
                                                                          int32_t* __restrict__ info, int k) {
-    __shared__ double m[kCholPacked];   // A, then R (off-diagonal; the diagonal keeps the pivots)
-    __shared__ double s[kCholPacked];   // S, then X
-    __shared__ double rowbuf[2][RCH_CHOLESKY_MAX_K];
-    __shared__ double diag[RCH_CHOLESKY_MAX_K];  // 1 / R[j][j]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int P = kCholPitch;
+    __shared__ double m[RCH_CHOLESKY_MAX_K * P];  // A, then R; below the diagonal blocks X transposed by blocks
+    __shared__ double inverse_diagonal[kCholBlocks][16 * 16];  // X_JJ
+    __shared__ double pivot_inverse[RCH_CHOLESKY_MAX_K];  // 1 / R[j][j]
+    __shared__ int failed_at;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i16 = lane & 15, g = lane >> 4;
+    const int blocks = (k + 15) >> 4, kp = 16 * blocks;
     const int64_t base = static_cast<int64_t>(blockIdx.x) * k * k;
     const RCH_GLOBAL double* A = gin<double>(reinterpret_cast<int64_t>(a)) + base;
     RCH_GLOBAL double* X = gout<double>(reinterpret_cast<int64_t>(x)) + base;
-    for (int i = wave; i < k; i += kCholWaves) {
-        for (int c = i + lane; c < k; c += 64) {
-            m[packed_at(i, c, k)] = A[i * k + c];
-            s[packed_at(i, c, k)] = 0.0;
-        }
-    }
+    if (tid == 0) failed_at = 0;
+    for (int i = wave; i < kp; i += kCholWaves)
+        for (int c = i + lane; c < kp; c += 64) m[i * P + c] = (i < k && c < k) ? A[i * k + c] : (i == c ? 1.0 : 0.0);
     __syncthreads();
-    int failed = 0;
-    for (int j = 0; j < k; ++j) {
-        const double d = m[packed_at(j, j, k)];  // every thread reads the same pivot: the branch is uniform
-        if (!(d > 0.0) || !(d < INFINITY)) {
-            failed = j + 1;
-            break;
-        }
-        const double inv = 1.0 / sqrt(d);
-        if (j > 0) {  // row j - 1 of R, scaled in the previous step
-            for (int c = j + tid; c < k; c += kCholThreads) m[packed_at(j - 1, c, k)] = rowbuf[(j - 1) & 1][c];
-        }
-        const int row_j = packed_at(j, j, k) - j;  // row j's entry c sits at row_j + c
-        for (int c = j + 1 + tid; c < k; c += kCholThreads) rowbuf[j & 1][c] = m[row_j + c] * inv;
-        if (tid == 0) diag[j] = inv;
-        for (int i = j + 1 + wave; i < k; i += kCholWaves) {
-            const double ri = m[row_j + i] * inv;
-            const int row_i = packed_at(i, i, k) - i;
-            for (int c = i + lane; c < k; c += 64) {
-                const double rc = m[row_j + c] * inv;
-                const double product = ri * rc;
-                m[row_i + c] = m[row_i + c] - product;
+    for (int J = 0; J < blocks; ++J) {
+        const int j0 = 16 * J;
+        const int right = kp - j0 - 16;  // columns beside the diagonal block
+        double v[16];
+        if (wave == 0 || 48 * wave < right) {
+            // Lower-triangle entries of the diagonal block's lanes are unset: they feed nothing and
+            // are not written back.
+            const int c = lane < 16 ? j0 + lane : j0 + 48 * wave + lane;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) v[r] = c < kp ? m[(j0 + r) * P + c] : 0.0;
+            int failed = 0;
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const double d = broadcast_lane(v[j], j);  // uniform
+                if (failed == 0 && (!(d > 0.0) || !(d < INFINITY))) failed = j0 + j + 1;
+                if (failed == 0) {
+                    const double inv = 1.0 / sqrt(d);
+                    v[j] *= inv;
+                    if (wave == 0 && lane == 0) pivot_inverse[j0 + j] = inv;
+#pragma unroll
+                    for (int i = j + 1; i < 16; ++i) v[i] = v[i] - broadcast_lane(v[j], i) * v[j];
+                }
+            }
+            if (wave == 0 && lane == 0) failed_at = failed;
+            if (c < kp && lane >= 16) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) m[(j0 + r) * P + c] = v[r];
             }
         }
         __syncthreads();
+        if (failed_at) break;  // uniform
+        // The diagonal block goes back only now: every panel wave has read it.
+        if (wave == 0 && lane < 16) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (r <= lane) m[(j0 + r) * P + j0 + lane] = v[r];
+        }
+        // Trailing tiles (ti <= tj) behind the panel, dealt to the waves.
+        const int left = blocks - J - 1, count = left * (left + 1) / 2;
+        for (int t = wave; t < count; t += kCholWaves) {
+            int tj = 0, rest = t;
+            while (rest > tj) {
+                rest -= tj + 1;
+                ++tj;
+            }
+            const int row = j0 + 16 + 16 * rest, col = j0 + 16 + 16 * tj;
+            double acc[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[v] = m[(row + g + 4 * v) * P + col + i16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const double rc = m[(j0 + r) * P + col + i16];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[v] = acc[v] - m[(j0 + r) * P + row + g + 4 * v] * rc;
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) m[(row + g + 4 * v) * P + col + i16] = acc[v];
+        }
+        __syncthreads();
     }
-    if (failed) {
+    if (failed_at) {
         for (int i = wave; i < k; i += kCholWaves)
             for (int c = lane; c < k; c += 64) X[i * k + c] = i == c ? 1.0 : 0.0;
-        if (tid == 0) info[blockIdx.x] = failed;
+        if (tid == 0) info[blockIdx.x] = failed_at;
         return;
     }
-    // Step k - 1 wrote row k - 2 back and row k - 1 has no off-diagonal entry: m holds R above
-    // the diagonal (the last step's barrier makes it visible).
-    for (int i = k - 1; i >= 0; --i) {
-        const double di = diag[i];
-        const int srow_i = packed_at(i, i, k) - i;
-        if (i + 1 < k) {  // row i + 1 of X, finished in the previous step
-            for (int c = i + 1 + tid; c < k; c += kCholThreads) s[packed_at(i + 1, c, k)] = rowbuf[(i + 1) & 1][c];
-        }
-        for (int c = i + tid; c < k; c += kCholThreads) rowbuf[i & 1][c] = ((c == i ? 1.0 : 0.0) - s[srow_i + c]) * di;
-        for (int r = wave; r < i; r += kCholWaves) {
-            const double rri = m[packed_at(r, i, k)];
-            const int srow_r = packed_at(r, r, k) - r;
-            for (int c = i + lane; c < k; c += 64) {
-                const double xic = ((c == i ? 1.0 : 0.0) - s[srow_i + c]) * di;
-                const double product = rri * xic;
-                s[srow_r + c] = s[srow_r + c] + product;
+    if (wave < blocks) {
+        const int J = wave;
+        for (int I = J; I >= 0; --I) {
+            double* const slot = m + 16 * J * P + 16 * I;  // block (J, I): holds S, then X_IJ
+            if (I < J) {
+                double sum[4] = {0.0, 0.0, 0.0, 0.0};  // rows g + 4v, column i16
+                for (int Q = J; Q > I; --Q) {
+                    const double* r_iq = m + (16 * I + g) * P + 16 * Q;
+                    const double* x_qj = Q == J ? inverse_diagonal[J] + i16 : m + 16 * J * P + 16 * Q + i16;
+                    const int pitch = Q == J ? 16 : P;
+#pragma unroll
+                    for (int p = 15; p >= 0; --p) {
+                        const double xv = x_qj[p * pitch];
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) sum[v] = sum[v] + r_iq[4 * v * P + p] * xv;
+                    }
+                }
+#pragma unroll
+                for (int v = 0; v < 4; ++v) slot[(g + 4 * v) * P + i16] = sum[v];
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // other lanes of this wave read it
             }
+            // Substitution: lane c holds column c of R_II and of S (the four lane groups repeat it).
+            double t[16], sum[16], y[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                t[r] = r <= i16 ? m[(16 * I + r) * P + 16 * I + i16] : 0.0;
+                sum[r] = I < J ? slot[r * P + i16] : 0.0;
+            }
+#pragma unroll
+            for (int i = 15; i >= 0; --i) {
+                const double value = ((I == J && i == i16 ? 1.0 : 0.0) - sum[i]) * pivot_inverse[16 * I + i];
+                y[i] = I == J && i > i16 ? 0.0 : value;
+#pragma unroll
+                for (int r = 0; r < i; ++r) sum[r] = sum[r] + broadcast_lane(t[r], i) * y[i];
+            }
+            if (lane < 16) {
+                double* const to = I == J ? inverse_diagonal[J] + i16 : slot + i16;
+                const int pitch = I == J ? 16 : P;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) to[r * pitch] = y[r];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const int col = 16 * J + i16;
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if ((r & 3) == g && 16 * I + r < k && col < k) X[(16 * I + r) * k + col] = y[r];
         }
-        __syncthreads();
+        for (int row = 16 * (J + 1) + g; row < k; row += 4)
+            if (16 * J + i16 < k) X[row * k + 16 * J + i16] = 0.0;
     }
-    for (int c = tid; c < k; c += kCholThreads) s[packed_at(0, c, k)] = rowbuf[0][c];
-    __syncthreads();
-    for (int i = wave; i < k; i += kCholWaves)
-        for (int c = lane; c < k; c += 64) X[i * k + c] = i <= c ? s[packed_at(i, c, k)] : 0.0;
     if (tid == 0) info[blockIdx.x] = 0;
 }
 

@@ -241,6 +241,33 @@ def test_batched_quantizer_matches_single_launches(device):
         np.testing.assert_array_equal(codes.cpu().numpy(), oq.quantize_with_affine(v.cpu().numpy(), affine[0], affine[1]))
 
 
+@pytest.mark.parametrize("k", [2, 15, 16, 17, 31, 33, 64, 65, 80, 81, 112, 127])
+def test_cholesky_inverse_block_edges(device, k):
+    """Orders around the kernel's 16-row blocks and 48-column panel waves: A = R^T R and X = R^-1 as
+    numpy computes them (relative 1e-12, condition <= 900), zeros below the diagonal; a member whose
+    leading minor of order k, or just past the first block, is negative is flagged there."""
+    from scipy.linalg import solve_triangular
+
+    rng = np.random.default_rng(57 + k)
+    q, _ = np.linalg.qr(rng.standard_normal((k, k)))
+    good = (q * rng.uniform(1.0, 30.0, k)) @ q.T
+    last = good.copy()
+    last[k - 1, k - 1] = -1.0
+    early = np.diag(np.arange(1.0, k + 1.0))
+    at = min(k, 17)
+    early[at - 1, at - 1] = -2.0
+    # The matrix's lower triangle is never read.
+    stored = np.stack([np.triu(member) + np.tril(np.full((k, k), np.nan), -1) for member in (good, last, early)])
+    inverse, info = fk.cholesky_inverse(torch.from_numpy(stored).to(device))
+    inverse = inverse.cpu().numpy()
+    assert info.cpu().tolist() == [0, k, at]
+    r = np.linalg.cholesky(good).T
+    want = solve_triangular(r, np.eye(k), lower=False)
+    assert np.abs(inverse[0] - want).max() <= 1e-12 * np.abs(want).max()
+    assert (np.tril(inverse[0], -1) == 0).all()
+    assert (inverse[1] == np.eye(k)).all() and (inverse[2] == np.eye(k)).all()
+
+
 @pytest.mark.parametrize("k", [1, 7, 96, 128])
 def test_cholesky_inverse_matches_fp64_factorization(device, k):
     """The batched factor-and-inverse launch of the planner's CholeskyQR steps against numpy's
