@@ -13,7 +13,7 @@
 //     exactly to FP64, products and sums on v_mfma_f64_16x16x4f64, P rounded once to fp32.
 //     The FP64 sum makes P the correctly rounded fp32 value of the exact dot product except
 //     within ~1e-13 relative of a rounding boundary, i.e. independent of summation order.
-//   * Energies: FP64 sums of (x - r)^2 and x^2, divided by s^2 per 64-row partial, fixed-order totals.
+//   * Energies: FP64 sums of (x - r)^2 and x^2, divided by s^2 per partial (16 or 32 rows), fixed-order totals.
 //   * Quantizer: FP64 (v - offset) / scale, round half to even, clamp to [0, 255].
 #include <type_traits>
 
@@ -75,29 +75,54 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t source_rows(const rch_fit_matr
 }
 
 // ---------------------------------------------------------------------------------------------
-// max|X|: workgroup (64-row tile, matrix); one unsigned atomic max of the fp32 bits per workgroup.
+// max|X|: workgroup (row tile, matrix), one unsigned atomic max of the fp32 bits per workgroup.
+// HBM-bound: the absolute values compare as integers in their own width (two 16-bit values per
+// v_pk_max_u16), only the maximum is widened; four rows per wave at a time, lanes along the row.  The
+// keys of a batch share cache lines, where the atomics queue at about 13 ns each, so a tile is as many
+// 16-row sets as leave about kAbsmaxGroups workgroups.
 // ---------------------------------------------------------------------------------------------
 
+constexpr int kAbsmaxRows = 16, kAbsmaxGroups = 600, kAbsmaxSets = 32;
+
 template <int DT>
-__global__ void __launch_bounds__(kThreads) absmax_kernel(const rch_fit_matrix* __restrict__ mats, int channels) {
+__global__ void __launch_bounds__(kThreads) absmax_kernel(const rch_fit_matrix* __restrict__ mats, int channels, int sets) {
     const rch_fit_matrix* M = mats + blockIdx.y;
-    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * 64;
-    if (r0 >= M->rows) return;
-    constexpr int E = esize<DT>();
-    const int rows = static_cast<int>(M->rows - r0 < 64 ? M->rows - r0 : 64);
-    const __amdgpu_buffer_rsrc_t src = source_rows<DT>(M, channels, r0);
-    const int groups = channels / 8;  // 8 elements per load
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * sets * kAbsmaxRows;
+    if (first >= M->rows) return;
+    constexpr int E = esize<DT>(), kLoads = DT == RCH_DT_F32 ? 2 : 1, kRows = kAbsmaxRows / (kThreads / 64);
+    const int groups = channels / 8;  // 8 elements per item
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint32_t row_bytes = static_cast<uint32_t>(M->src_stride * E);
+    typedef unsigned short us2 __attribute__((ext_vector_type(2)));
     uint32_t m = 0;
-    for (int i = threadIdx.x; i < rows * groups; i += kThreads) {
-        const int r = i / groups, g = i - r * groups;
-        double v[8];
-        load8<DT>(src, static_cast<uint32_t>((r * M->src_stride + 8 * g) * E), v);
+    us2 pair = {0, 0};
+    for (int set = 0; set < sets; ++set) {
+        // Rows past the end read zeros.
+        const __amdgpu_buffer_rsrc_t src = source_rows<DT>(M, channels, first + set * kAbsmaxRows);
+        for (int g = lane; g < groups; g += 64) {
+            u4 w[kRows][kLoads];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const uint32_t bits = __float_as_uint(static_cast<float>(v[j])) & 0x7fffffffu;  // exact: v is a float
-            m = bits > m ? bits : m;
+            for (int r = 0; r < kRows; ++r)
+#pragma unroll
+                for (int q = 0; q < kLoads; ++q)
+                    w[r][q] = __builtin_amdgcn_raw_buffer_load_b128(
+                        src, static_cast<uint32_t>(kRows * wave + r) * row_bytes + static_cast<uint32_t>(8 * g * E + 16 * q), 0, 0);
+#pragma unroll
+            for (int r = 0; r < kRows; ++r)
+#pragma unroll
+                for (int q = 0; q < kLoads; ++q)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        if constexpr (DT == RCH_DT_F32) {
+                            const uint32_t bits = w[r][q][j] & 0x7fffffffu;
+                            m = bits > m ? bits : m;
+                        } else {
+                            pair = __builtin_elementwise_max(pair, __builtin_bit_cast(us2, w[r][q][j] & 0x7fff7fffu));
+                        }
+                    }
         }
     }
+    if constexpr (DT != RCH_DT_F32) m = __float_as_uint(half_bits<DT>(pair[0] > pair[1] ? pair[0] : pair[1]));
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) {
         const uint32_t o = __shfl_xor(m, d);
@@ -362,64 +387,126 @@ __global__ void __launch_bounds__(kGramThreads) gram_kernel(const rch_fit_matrix
 
 // ---------------------------------------------------------------------------------------------
 // Projection P = X Q^T on v_mfma_f64_16x16x4f64: D[m = token][n = rank] = sum_c X[token][c] Q[rank][c].
-// Workgroup (64-token tile, 64-rank chunk, matrix); wave w owns tokens 16w .. 16w + 15 of the
-// tile and the chunk's 4 rank blocks of 16.  Per 32-channel step a lane (i = l % 16, group
-// g = l / 16) loads channels 8g .. 8g + 7 of its token row and of its basis row (16-byte loads,
-// no LDS), and MFMA step s takes channel 8g + s from every group.  The f64 accumulator holds
-// element v of lane l at row (l / 16) + 4v, column l % 16: token g + 4v, rank i of the block.
+// Per 32-channel step a lane (i = l % 16, group g = l / 16) holds channels 8g .. 8g + 7 of its token
+// rows and of its basis rows (16-byte loads, no LDS), and MFMA step s takes channel 8g + s from every
+// group.  The f64 accumulator holds element v of lane l at row (l / 16) + 4v, column l % 16: token
+// g + 4v, rank i of the block.
+//
+// Bound by the FP64 matrix rate; the next step's loads are issued before a step's products and the
+// step body has no branch, so their latency is covered.  Two shapes (project_kernel's TB, SPLIT):
+//   * TB = 2, SPLIT = 1: a wave owns 32 tokens, so each converted basis operand feeds two products;
+//     workgroup = 128 tokens x 64 ranks.
+//   * TB = 1, SPLIT = 4: for batches that would leave CUs idle, the four waves of a workgroup share 16
+//     tokens and split the channel steps; the partial sums are added through LDS in wave order.
+// One bf16 matrix [4680, 1536] at rank 96: 105 us with 64-token workgroups of one wave per 16 tokens and
+// loads in the step, 32 us now; 60 matrices at rank 96: 1563 -> 1396 us (59 of the 68 TFLOP/s that a
+// large library FP64 product reaches on this card).
 // ---------------------------------------------------------------------------------------------
 
+// Eight consecutive source elements as loaded, and as doubles.
 template <int DT>
-__global__ void __launch_bounds__(kThreads) project_kernel(const rch_fit_matrix* __restrict__ mats, int channels) {
-    const rch_fit_matrix* M = mats + blockIdx.z;
+struct Eight {
+    u4 w[DT == RCH_DT_F32 ? 2 : 1];
+};
+template <int DT>
+__device__ __forceinline__ Eight<DT> load_eight(__amdgpu_buffer_rsrc_t rsrc, uint32_t offset) {
+    Eight<DT> e;
+    e.w[0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset, 0, 0);
+    if constexpr (DT == RCH_DT_F32) e.w[1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset + 16, 0, 0);
+    return e;
+}
+template <int DT>
+__device__ __forceinline__ double eight_at(const Eight<DT>& e, int i) {
+    if constexpr (DT == RCH_DT_F32) return static_cast<double>(__uint_as_float(e.w[i >> 2][i & 3]));
+    else return static_cast<double>(half_bits<DT>((e.w[0][i >> 1] >> (16 * (i & 1))) & 0xffffu));
+}
+
+template <int DT, int TB, int SPLIT, int NB>
+__device__ __forceinline__ void project_ranks(const rch_fit_matrix* M, int channels, int r0, int64_t wt, int wave, int lane,
+                                              double* partial) {
+    constexpr int E = esize<DT>();
     const int64_t rows = M->rows;
     const int rank = static_cast<int>(M->rank);
-    const int64_t t0 = static_cast<int64_t>(blockIdx.x) * 64;
-    const int r0 = blockIdx.y * 64;
-    if (t0 >= rows || r0 >= rank) return;
-    constexpr int E = esize<DT>();
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int g = lane >> 4, i16 = lane & 15;
-    const int64_t wt = t0 + 16 * wave;  // first token of this wave
     const __amdgpu_buffer_rsrc_t xs = source_rows<DT>(M, channels, wt);
     const __amdgpu_buffer_rsrc_t qs = make_rsrc(M->basis_ptr, ((rank - 1) * M->basis_stride + channels) * 2);
-    const uint32_t x_row = static_cast<uint32_t>(i16 * M->src_stride * E);
-
-    d4 acc[4];
+    uint32_t x_row[TB], q_row[NB];
 #pragma unroll
-    for (int b = 0; b < 4; ++b) acc[b] = d4{};
-    for (int c0 = 0; c0 < channels; c0 += 32) {
-        const int c = c0 + 8 * g;
-        double xv[8];
-        load8<DT>(xs, c < channels ? x_row + static_cast<uint32_t>(c * E) : kOutOfRange, xv);
+    for (int t = 0; t < TB; ++t) x_row[t] = static_cast<uint32_t>((16 * t + i16) * M->src_stride * E);
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int k = r0 + 16 * b + i16;
-            const uint32_t q_off =
-                (k < rank && c < channels) ? static_cast<uint32_t>((k * M->basis_stride + c) * 2) : kOutOfRange;
-            if (r0 + 16 * b >= rank) continue;  // uniform: a 16-rank block past the rank adds zeros
-            double qv[8];
-            load8<RCH_DT_F16>(qs, q_off, qv);
+    for (int b = 0; b < NB; ++b)  // rows past the rank read zeros
+        q_row[b] = r0 + 16 * b + i16 < rank ? static_cast<uint32_t>((r0 + 16 * b + i16) * M->basis_stride * 2) : kOutOfRange;
+    Eight<DT> x_now[TB], x_next[TB];
+    Eight<RCH_DT_F16> q_now[NB], q_next[NB];
+    auto load = [&](int c0, Eight<DT> (&x)[TB], Eight<RCH_DT_F16> (&q)[NB]) __attribute__((always_inline)) {
+        const int c = c0 + 8 * g;  // channels % 8 == 0: a group is whole or past the end
+        const uint32_t past = c < channels ? 0u : kOutOfRange;
 #pragma unroll
-            for (int s = 0; s < 8; ++s) acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv[s], qv[s], acc[b], 0, 0, 0);
+        for (int t = 0; t < TB; ++t) x[t] = load_eight<DT>(xs, (x_row[t] + static_cast<uint32_t>(c * E)) | past);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) q[b] = load_eight<RCH_DT_F16>(qs, (q_row[b] + static_cast<uint32_t>(c * 2)) | past);
+    };
+    d4 acc[TB][NB];
+#pragma unroll
+    for (int t = 0; t < TB; ++t)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[t][b] = d4{};
+    const int first = SPLIT > 1 ? 32 * wave : 0;
+    load(first, x_now, q_now);
+    for (int c0 = first; c0 < channels; c0 += 32 * SPLIT) {
+        load(c0 + 32 * SPLIT, x_next, q_next);
+        double xv[TB][8];
+#pragma unroll
+        for (int t = 0; t < TB; ++t)
+#pragma unroll
+            for (int s = 0; s < 8; ++s) xv[t][s] = eight_at<DT>(x_now[t], s);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const double qv = eight_at<RCH_DT_F16>(q_now[b], s);
+#pragma unroll
+                for (int t = 0; t < TB; ++t)
+                    acc[t][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv[t][s], qv, acc[t][b], 0, 0, 0);
+            }
         }
+#pragma unroll
+        for (int t = 0; t < TB; ++t) x_now[t] = x_next[t];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) q_now[b] = q_next[b];
     }
-
+    if constexpr (SPLIT > 1) {  // block b of every wave is added, in wave order, by wave b
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) partial[((b * SPLIT + wave) * 4 + v) * 64 + lane] = acc[0][b][v];
+        __syncthreads();
+        if (wave >= NB) return;
+        d4 sum = d4{};
+#pragma unroll
+        for (int w = 0; w < SPLIT; ++w)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) sum[v] += partial[((wave * SPLIT + w) * 4 + v) * 64 + lane];
+        acc[0][0] = sum;
+    }
     RCH_GLOBAL float* out = gout<float>(M->coef_ptr);
     unsigned int* ext = reinterpret_cast<unsigned int*>(M->extrema_ptr);
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        const int k = r0 + 16 * b + i16;  // this lane's rank
+    for (int b = 0; b < (SPLIT > 1 ? 1 : NB); ++b) {
+        const int k = r0 + 16 * (SPLIT > 1 ? wave : b) + i16;  // this lane's rank
         uint32_t lo = 0u, hi = 0u;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int64_t t = wt + g + 4 * v;
-            const float value = static_cast<float>(acc[b][v]);
-            if (t < rows) {
-                if (k < rank) out[t * M->coef_stride + k] = value;  // 16 lanes: 64 contiguous bytes of a row
-                const uint32_t key = order_key(value);
-                lo = ~key > lo ? ~key : lo;
-                hi = key > hi ? key : hi;
+        for (int t = 0; t < TB; ++t) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int64_t token = wt + 16 * t + g + 4 * v;
+                const float value = static_cast<float>(acc[t][b][v]);
+                if (token < rows) {
+                    if (k < rank) out[token * M->coef_stride + k] = value;  // 16 lanes: 64 contiguous bytes of a row
+                    const uint32_t key = order_key(value);
+                    lo = ~key > lo ? ~key : lo;
+                    hi = key > hi ? key : hi;
+                }
             }
         }
         if (ext) {
@@ -437,174 +524,169 @@ __global__ void __launch_bounds__(kThreads) project_kernel(const rch_fit_matrix*
     }
 }
 
+// Tokens of a project_kernel workgroup.
+template <int TB, int SPLIT>
+constexpr int kProjectTokens = 16 * TB * (SPLIT > 1 ? 1 : kThreads / 64);
+
+template <int DT, int TB, int SPLIT>
+__global__ void __launch_bounds__(kThreads, 2) project_kernel(const rch_fit_matrix* __restrict__ mats, int channels,
+                                                              int chunk) {
+    static_assert(SPLIT == 1 || (SPLIT == kThreads / 64 && TB == 1), "all waves split the channels, or none");
+    __shared__ double partial[SPLIT > 1 ? 4 * SPLIT * 4 * 64 : 1];
+    const rch_fit_matrix* M = mats + blockIdx.z;
+    const int rank = static_cast<int>(M->rank);
+    const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kProjectTokens<TB, SPLIT>;
+    const int r0 = blockIdx.y * chunk;  // chunk: 16, 32, 48 or 64 ranks
+    if (t0 >= M->rows || r0 >= rank) return;  // whole workgroup
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int64_t wt = SPLIT > 1 ? t0 : t0 + 16 * TB * wave;  // first token of this wave
+    switch (min(chunk >> 4, (rank - r0 + 15) >> 4)) {  // 16-rank blocks of this chunk (uniform)
+        case 1: project_ranks<DT, TB, SPLIT, 1>(M, channels, r0, wt, wave, lane, partial); break;
+        case 2: project_ranks<DT, TB, SPLIT, 2>(M, channels, r0, wt, wave, lane, partial); break;
+        case 3: project_ranks<DT, TB, SPLIT, 3>(M, channels, r0, wt, wave, lane, partial); break;
+        default: project_ranks<DT, TB, SPLIT, 4>(M, channels, r0, wt, wave, lane, partial); break;
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Residual energies on v_mfma_f64_16x16x4f64: D[m = token][n = channel] = sum_k P[token][k] Q[k][c].
+// Workgroup = 16 TB tokens of one matrix and every gridDim.z-th set of four 64-channel groups, one
+// group per wave.  A group
+// is four 16 x 16 blocks per 16 tokens whose columns interleave: column i of block b is channel
+// 4i + b of the group, so after the four blocks lane l (i = l % 16, g = l / 16) holds channels 4i ..
+// 4i + 3 of tokens g + 4v (v = 0..3, the f64 accumulator's row (l / 16) + 4v): X and the residual move
+// as 4-channel vectors, 16 lanes covering 64 contiguous channels of a row.  Per 16-rank step a lane
+// takes P[token i][4g .. 4g + 3] (the A operand; MFMA step j takes rank 4g + j) and, for each j,
+// Q[4g + j][4i .. 4i + 3] (one 8-byte load: the B operands of the four blocks).
+//
+// Bound by the FP64 matrix rate (rank 0, the source energy alone: by HBM): the next step's operands
+// and the next group's source elements are loaded before a step's products.  TB = 2 lets each
+// converted basis operand feed two products; small batches take TB = 1 and split the channels over
+// workgroups (grid z) until they fill the chip.  One bf16 matrix [4680, 1536] at rank 96: 137 -> 41 us;
+// 60 matrices: 1808 -> 1527 us (54 TFLOP/s); source energy of one: 29 -> 18 us.
+// ---------------------------------------------------------------------------------------------
+
 // The 4 channels of tokens g + 4v (v = 0..3) of a lane's 64-channel group, as raw 16-bit pairs
-// (or fp32 words), loaded ahead of their use.
+// (or fp32 words).
 template <int DT>
 struct SourceQuad {
     using word = std::conditional_t<DT == RCH_DT_F32, u4, u2>;
     word w[4];
 };
 
-template <int DT>
-__device__ __forceinline__ void load_quad(__amdgpu_buffer_rsrc_t xs, const rch_fit_matrix* M, int c, bool c_ok,
-                                          SourceQuad<DT>& q) {
+template <int DT, int TB>
+__global__ void __launch_bounds__(kThreads, 2) residual_kernel(const rch_fit_matrix* __restrict__ mats, int channels) {
     constexpr int E = esize<DT>();
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        const int token = (threadIdx.x & 63) / 16 + 4 * v;
-        const uint32_t offset = c_ok ? static_cast<uint32_t>((token * M->src_stride + c) * E) : kOutOfRange;
-        if constexpr (DT == RCH_DT_F32) {
-            q.w[v] = __builtin_amdgcn_raw_buffer_load_b128(xs, offset, 0, 0);
-        } else {
-            q.w[v] = __builtin_amdgcn_raw_buffer_load_b64(xs, offset, 0, 0);
-        }
-    }
-}
-
-// Residual of one 64-channel group: e = x - r per element, FP64 sums of x^2 and e^2, optional fp32 store.
-template <int DT>
-__device__ __forceinline__ void residual_group(const SourceQuad<DT>& q, const d4 (&acc)[4], int c, bool c_ok,
-                                               int64_t wt, int64_t left, int channels, RCH_GLOBAL float* resid,
-                                               double& src, double& err) {
-    const int g = (threadIdx.x & 63) >> 4;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        const int token = g + 4 * v;
-        double a[4];
-        if constexpr (DT == RCH_DT_F32) {
-#pragma unroll
-            for (int b = 0; b < 4; ++b) a[b] = static_cast<double>(__uint_as_float(q.w[v][b]));
-        } else {
-#pragma unroll
-            for (int b = 0; b < 4; ++b) a[b] = static_cast<double>(half_bits<DT>((q.w[v][b >> 1] >> (16 * (b & 1))) & 0xffffu));
-        }
-        double e[4];
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            e[b] = a[b] - acc[b][v];
-            // The scale s is applied once per tile: sum (a / s)^2 = (sum a^2) / s^2 up to the rounding
-            // of the FP64 sums (relative 1e-16), without two FP64 divisions per element.
-            src += a[b] * a[b];
-            err += e[b] * e[b];
-        }
-        if (resid && c_ok && token < left) {
-            const f4 out = {static_cast<float>(e[0]), static_cast<float>(e[1]), static_cast<float>(e[2]),
-                            static_cast<float>(e[3])};
-            *reinterpret_cast<RCH_GLOBAL f4*>(resid + (wt + token) * channels + c) = out;
-        }
-    }
-}
-
-// The four B operands (channels 4i .. 4i + 3 of basis row k) from one 8-byte load, as doubles.
-__device__ __forceinline__ double basis_operand(const u2& w, int b) {
-    return static_cast<double>(half_bits<RCH_DT_F16>((w[b >> 1] >> (16 * (b & 1))) & 0xffffu));
-}
-
-// ---------------------------------------------------------------------------------------------
-// Residual energies on v_mfma_f64_16x16x4f64: D[m = token][n = channel] = sum_k P[token][k] Q[k][c].
-// Workgroup = 64-token tile of one matrix, wave w = tokens 16w .. 16w + 15, looping over
-// 64-channel groups.  A group is four 16 x 16 blocks whose columns interleave: column i of
-// block b is channel 4i + b of the group, so after the four blocks lane l (i = l % 16,
-// g = l / 16) holds channels 4i .. 4i + 3 of tokens g + 4v (v = 0..3, the f64 accumulator's row
-// (l / 16) + 4v): X and the residual move as 4-channel vectors, 16 lanes covering 64 contiguous
-// channels of a row.  Per 16-rank step a lane takes P[token i][4g .. 4g + 3] (the A operand; MFMA
-// step j takes rank 4g + j) and, for each j, Q[4g + j][4i .. 4i + 3] (one 8-byte load: the B
-// operands of the four blocks).
-//
-// Ranks up to 64 (the common fit ranks) keep the wave's P block in registers for the whole
-// channel loop (loaded once instead of once per channel group) and load a group's source
-// elements before its MFMAs; larger ranks stream P per step.  Both paths add the products in the same
-// order (rank ascending within each block), so their results are identical.
-// ---------------------------------------------------------------------------------------------
-
-template <int DT>
-__global__ void __launch_bounds__(kThreads) residual_kernel(const rch_fit_matrix* __restrict__ mats, int channels) {
+    constexpr int kTokens = 16 * TB, kWaves = kThreads / 64;
     const rch_fit_matrix* M = mats + blockIdx.y;
     const int64_t rows = M->rows;
     const int rank = static_cast<int>(M->rank);
-    const int64_t t0 = static_cast<int64_t>(blockIdx.x) * 64;
+    const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kTokens;
     if (t0 >= rows) return;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int g = lane >> 4, i16 = lane & 15;
-    const int64_t wt = t0 + 16 * wave;
-    const int64_t left = rows - wt;
-    const __amdgpu_buffer_rsrc_t xs = source_rows<DT>(M, channels, wt);
-    const __amdgpu_buffer_rsrc_t ps = make_rsrc(M->coef_ptr + wt * M->coef_stride * 4,
-                                                (rank > 0 && left > 0) ? ((left - 1) * M->coef_stride + rank) * 4 : 0);
+    const int64_t left = rows - t0;
+    const __amdgpu_buffer_rsrc_t xs = source_rows<DT>(M, channels, t0);
+    const __amdgpu_buffer_rsrc_t ps = make_rsrc(M->coef_ptr + t0 * M->coef_stride * 4,
+                                                rank > 0 ? ((left - 1) * M->coef_stride + rank) * 4 : 0);
     const __amdgpu_buffer_rsrc_t qs = make_rsrc(M->basis_ptr, rank > 0 ? ((rank - 1) * M->basis_stride + channels) * 2 : 0);
-    const float smax = __uint_as_float(*gin<unsigned int>(M->absmax_ptr));
-    const double s = static_cast<double>(smax);
-    const bool scaled = smax != 0.0f;
-    const uint32_t p_row = static_cast<uint32_t>(i16 * M->coef_stride * 4);
     const uint32_t q_stride = static_cast<uint32_t>(M->basis_stride * 2);
     RCH_GLOBAL float* resid = M->resid_ptr ? gout<float>(M->resid_ptr) : nullptr;
+    uint32_t p_row[TB], x_row[TB][4];
+#pragma unroll
+    for (int t = 0; t < TB; ++t) {
+        p_row[t] = static_cast<uint32_t>((16 * t + i16) * M->coef_stride * 4);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) x_row[t][v] = static_cast<uint32_t>((16 * t + g + 4 * v) * M->src_stride * E);
+    }
+    auto load_source = [&](int c64, SourceQuad<DT> (&q)[TB]) __attribute__((always_inline)) {
+        const int c = c64 + 4 * i16;  // this lane's 4 channels (channels % 8 == 0: all or none in range)
+        const uint32_t past = c < channels ? 0u : kOutOfRange;
+#pragma unroll
+        for (int t = 0; t < TB; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const uint32_t offset = (x_row[t][v] + static_cast<uint32_t>(c * E)) | past;
+                if constexpr (DT == RCH_DT_F32) q[t].w[v] = __builtin_amdgcn_raw_buffer_load_b128(xs, offset, 0, 0);
+                else q[t].w[v] = __builtin_amdgcn_raw_buffer_load_b64(xs, offset, 0, 0);
+            }
+    };
+    struct Operands {
+        u2 q[4];   // Q[k + j][4 channels], j = 0..3
+        u4 p[TB];  // P[token][k .. k + 3]
+    };
+    auto load_operands = [&](int c64, int k0, Operands& o) __attribute__((always_inline)) {
+        const int c = c64 + 4 * i16, k = k0 + 4 * g;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t offset = (k + j < rank && c < channels) ? static_cast<uint32_t>(k + j) * q_stride + 2u * c : kOutOfRange;
+            o.q[j] = __builtin_amdgcn_raw_buffer_load_b64(qs, offset, 0, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < TB; ++t)
+            o.p[t] = __builtin_amdgcn_raw_buffer_load_b128(ps, k < rank ? p_row[t] + static_cast<uint32_t>(k * 4) : kOutOfRange, 0, 0);
+    };
 
     double src = 0.0, err = 0.0;
-    if (rank <= 64) {
-        const int steps = (rank + 15) >> 4;  // uniform
-        u4 pw[4];
+    SourceQuad<DT> x_now[TB], x_next[TB];
+    Operands now, next;
+    const int first = 64 * (wave + kWaves * static_cast<int>(blockIdx.z));
+    const int stride = 64 * kWaves * static_cast<int>(gridDim.z);
+    load_source(first, x_now);
+    if (rank > 0) load_operands(first, 0, now);
+    for (int c64 = first; c64 < channels; c64 += stride) {
+        load_source(c64 + stride, x_next);
+        d4 acc[TB][4];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const int k = 16 * t + 4 * g;
-            pw[t] = __builtin_amdgcn_raw_buffer_load_b128(ps, (t < steps && k < rank) ? p_row + static_cast<uint32_t>(k * 4)
-                                                                                     : kOutOfRange, 0, 0);
-        }
-        for (int c64 = 0; c64 < channels; c64 += 64) {
-            const int c = c64 + 4 * i16;  // this lane's 4 channels (channels % 8 == 0: all or none in range)
-            const bool c_ok = c < channels;
-            SourceQuad<DT> xq;
-            load_quad<DT>(xs, M, c, c_ok, xq);
-            d4 acc[4] = {d4{}, d4{}, d4{}, d4{}};
-#pragma unroll 1
-            for (int t = 0; t < steps; ++t) {
-                const int k = 16 * t + 4 * g;
-                u2 qw[4];
+        for (int t = 0; t < TB; ++t)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t q_off =
-                        (k + j < rank && c_ok) ? static_cast<uint32_t>(k + j) * q_stride + 2u * c : kOutOfRange;
-                    qw[j] = __builtin_amdgcn_raw_buffer_load_b64(qs, q_off, 0, 0);
-                }
-                const u4 p = t == 0 ? pw[0] : t == 1 ? pw[1] : t == 2 ? pw[2] : pw[3];
+            for (int b = 0; b < 4; ++b) acc[t][b] = d4{};
+        for (int k0 = 0; k0 < rank; k0 += 16) {
+            const bool last = k0 + 16 >= rank;
+            load_operands(last ? c64 + stride : c64, last ? 0 : k0 + 16, next);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    // P rows may hold padding beyond the rank; its basis rows read as zero.
-                    const double pa = k + j < rank ? static_cast<double>(__uint_as_float(p[j])) : 0.0;
+            for (int j = 0; j < 4; ++j) {
+                // P rows may hold padding beyond the rank; its basis rows read as zero.
+                double pa[TB];
 #pragma unroll
-                    for (int b = 0; b < 4; ++b)
-                        acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(pa, basis_operand(qw[j], b), acc[b], 0, 0, 0);
+                for (int t = 0; t < TB; ++t)
+                    pa[t] = k0 + 4 * g + j < rank ? static_cast<double>(__uint_as_float(now.p[t][j])) : 0.0;
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const double qb = static_cast<double>(half_bits<RCH_DT_F16>((now.q[j][b >> 1] >> (16 * (b & 1))) & 0xffffu));
+#pragma unroll
+                    for (int t = 0; t < TB; ++t) acc[t][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(pa[t], qb, acc[t][b], 0, 0, 0);
                 }
             }
-            residual_group<DT>(xq, acc, c, c_ok, wt, left, channels, resid, src, err);
+            now = next;
         }
-    } else {
-        for (int c64 = 0; c64 < channels; c64 += 64) {
-            const int c = c64 + 4 * i16;
-            const bool c_ok = c < channels;
-            d4 acc[4] = {d4{}, d4{}, d4{}, d4{}};
-            for (int k0 = 0; k0 < rank; k0 += 16) {
-                const int k = k0 + 4 * g;
-                const u4 pw = __builtin_amdgcn_raw_buffer_load_b128(
-                    ps, k < rank ? p_row + static_cast<uint32_t>(k * 4) : kOutOfRange, 0, 0);
-                u2 qw[4];
+        // e = x - r per element: FP64 sums of x^2 and e^2, optional fp32 store.
+        const int c = c64 + 4 * i16;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t q_off =
-                        (k + j < rank && c_ok) ? static_cast<uint32_t>(k + j) * q_stride + 2u * c : kOutOfRange;
-                    qw[j] = __builtin_amdgcn_raw_buffer_load_b64(qs, q_off, 0, 0);
+        for (int t = 0; t < TB; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                double e[4];
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    double a;
+                    if constexpr (DT == RCH_DT_F32) a = static_cast<double>(__uint_as_float(x_now[t].w[v][b]));
+                    else a = static_cast<double>(half_bits<DT>((x_now[t].w[v][b >> 1] >> (16 * (b & 1))) & 0xffffu));
+                    e[b] = a - acc[t][b][v];
+                    // The scale s is applied once per tile: sum (a / s)^2 = (sum a^2) / s^2 up to the
+                    // rounding of the FP64 sums (relative 1e-16), without two FP64 divisions per element.
+                    src = fma(a, a, src);
+                    err = fma(e[b], e[b], err);
                 }
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const double pa = k + j < rank ? static_cast<double>(__uint_as_float(pw[j])) : 0.0;
-#pragma unroll
-                    for (int b = 0; b < 4; ++b)
-                        acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(pa, basis_operand(qw[j], b), acc[b], 0, 0, 0);
+                const int token = 16 * t + g + 4 * v;
+                if (resid && c < channels && token < left) {
+                    const f4 out = {static_cast<float>(e[0]), static_cast<float>(e[1]), static_cast<float>(e[2]),
+                                    static_cast<float>(e[3])};
+                    *reinterpret_cast<RCH_GLOBAL f4*>(resid + (t0 + token) * channels + c) = out;
                 }
             }
-            SourceQuad<DT> xq;
-            load_quad<DT>(xs, M, c, c_ok, xq);
-            residual_group<DT>(xq, acc, c, c_ok, wt, left, channels, resid, src, err);
-        }
+#pragma unroll
+        for (int t = 0; t < TB; ++t) x_now[t] = x_next[t];
     }
     // Fixed-order reduction: butterfly within the wave, then waves 0..3 in order.
 #pragma unroll
@@ -612,7 +694,7 @@ __global__ void __launch_bounds__(kThreads) residual_kernel(const rch_fit_matrix
         src += __shfl_xor(src, d);
         err += __shfl_xor(err, d);
     }
-    __shared__ double part[2][kThreads / 64];
+    __shared__ double part[2][kWaves];
     if (lane == 0) {
         part[0][wave] = src;
         part[1][wave] = err;
@@ -620,34 +702,44 @@ __global__ void __launch_bounds__(kThreads) residual_kernel(const rch_fit_matrix
     __syncthreads();
     if (threadIdx.x == 0) {
         double a = 0.0, b = 0.0;
-        for (int w = 0; w < kThreads / 64; ++w) {
+        for (int w = 0; w < kWaves; ++w) {
             a += part[0][w];
             b += part[1][w];
         }
-        if (scaled) {
+        const float smax = __uint_as_float(*gin<unsigned int>(M->absmax_ptr));
+        if (smax != 0.0f) {
+            const double s = static_cast<double>(smax);
             a = a / s / s;
             b = b / s / s;
         }
-        RCH_GLOBAL double* out = gout<double>(M->partial_ptr) + 2 * blockIdx.x;
+        RCH_GLOBAL double* out = gout<double>(M->partial_ptr) + 2 * (gridDim.z * blockIdx.x + blockIdx.z);
         out[0] = a;
         out[1] = b;
     }
 }
 
-// Sum of the per-tile partials of each matrix in tile order (one workgroup per matrix).
-__global__ void __launch_bounds__(64) energy_total_kernel(const rch_fit_matrix* __restrict__ mats) {
+// Sum of the partials of each matrix (`splits` per `tokens` rows): one wave per matrix, lane l takes
+// partials l, l + 64, ... in order, then a butterfly -- the same order whatever the launch.
+__global__ void __launch_bounds__(64) energy_total_kernel(const rch_fit_matrix* __restrict__ mats, int tokens,
+                                                          int splits) {
     const rch_fit_matrix* M = mats + blockIdx.x;
-    if (threadIdx.x != 0) return;
-    const int64_t tiles = (M->rows + 63) / 64;
+    const int64_t tiles = (M->rows + tokens - 1) / tokens * splits;
     const RCH_GLOBAL double* p = gin<double>(M->partial_ptr);
     double a = 0.0, b = 0.0;
-    for (int64_t t = 0; t < tiles; ++t) {
+    for (int64_t t = threadIdx.x; t < tiles; t += 64) {
         a += p[2 * t];
         b += p[2 * t + 1];
     }
-    RCH_GLOBAL double* out = gout<double>(M->energy_ptr);
-    out[0] = a;
-    out[1] = b;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        a += __shfl_xor(a, d);
+        b += __shfl_xor(b, d);
+    }
+    if (threadIdx.x == 0) {
+        RCH_GLOBAL double* out = gout<double>(M->energy_ptr);
+        out[0] = a;
+        out[1] = b;
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -933,6 +1025,14 @@ __global__ void __launch_bounds__(256) gaussian_kernel(const rch_gauss_job* __re
     }
 }
 
+// Measured on [n x 4680, 1536] bf16 (MI355X, host-side upload included): the projection's 128-token
+// workgroups beat the channel-split ones at 2220 workgroups (60 matrices, rank 32: 514 / 533 us) and lose
+// at 592 (8 matrices, rank 96: 254 / 224 us); the residual's 32-token workgroups win at 1176 (8
+// matrices: 242 / 269 us) and lose at 588 (4 matrices, rank 96: 156 / 134 us).
+constexpr int64_t kProjectWholeGroups = 2000;
+constexpr int64_t kResidualPairGroups = 1000;
+constexpr int64_t kResidualSplitGroups = 2000;  // workgroups that the channel splits aim at
+
 int check_matrices(const rch_fit_matrix* mats, int n, int channels, const char* what) {
     if (!mats || n <= 0 || n > 65535) return fail(RCH_E_CONFIG, "%s: 1 <= n_mats <= 65535 required", what);
     if (channels <= 0 || channels % 8 != 0 || channels > (1 << 20))
@@ -952,8 +1052,6 @@ using namespace rch;
         case RCH_DT_F32: hipLaunchKernelGGL(KERNEL<RCH_DT_F32>, GRID, dim3(BLOCK), 0, s, __VA_ARGS__); break;       \
         default: return fail(RCH_E_CONFIG, "%s: source dtype must be bf16, f16 or f32", what);                      \
     }
-#define RCH_DISPATCH_DTYPE(dtype, what, KERNEL, GRID, ...) \
-    RCH_DISPATCH_DTYPE_BLOCK(dtype, what, KERNEL, GRID, kThreads, __VA_ARGS__)
 
 extern "C" {
 
@@ -962,10 +1060,14 @@ int rch_fit_matrix_size(void) { return static_cast<int>(sizeof(rch_fit_matrix));
 int rch_fit_absmax(const rch_fit_matrix* mats_dev, int n_mats, int channels, int64_t max_rows, int src_dtype,
                    void* stream) {
     if (int status = check_matrices(mats_dev, n_mats, channels, "rch_fit_absmax")) return status;
-    if (max_rows <= 0 || (max_rows + 63) / 64 > 0x7fffffff) return fail(RCH_E_CONFIG, "rch_fit_absmax: invalid max_rows");
-    const dim3 grid(static_cast<unsigned>((max_rows + 63) / 64), static_cast<unsigned>(n_mats));
+    if (max_rows <= 0 || (max_rows + kAbsmaxRows - 1) / kAbsmaxRows > 0x7fffffff)
+        return fail(RCH_E_CONFIG, "rch_fit_absmax: invalid max_rows");
+    const int64_t tiles = (max_rows + kAbsmaxRows - 1) / kAbsmaxRows;
+    const int64_t wanted = tiles * n_mats / kAbsmaxGroups;
+    const int sets = static_cast<int>(wanted < 1 ? 1 : (wanted > kAbsmaxSets ? kAbsmaxSets : wanted));
+    const dim3 grid(static_cast<unsigned>((tiles + sets - 1) / sets), static_cast<unsigned>(n_mats));
     hipStream_t s = as_stream(stream);
-    RCH_DISPATCH_DTYPE(src_dtype, "rch_fit_absmax", absmax_kernel, grid, mats_dev, channels);
+    RCH_DISPATCH_DTYPE_BLOCK(src_dtype, "rch_fit_absmax", absmax_kernel, grid, kThreads, mats_dev, channels, sets);
     return check_launch("rch_fit_absmax");
 }
 
@@ -986,22 +1088,69 @@ int rch_fit_project(const rch_fit_matrix* mats_dev, int n_mats, int channels, in
     if (int status = check_matrices(mats_dev, n_mats, channels, "rch_fit_project")) return status;
     if (max_rows <= 0 || max_rank <= 0 || (max_rows + 63) / 64 > 0x7fffffff || max_rank > channels)
         return fail(RCH_E_CONFIG, "rch_fit_project: invalid max_rows / max_rank");
-    const dim3 grid(static_cast<unsigned>((max_rows + 63) / 64), static_cast<unsigned>((max_rank + 63) / 64),
-                    static_cast<unsigned>(n_mats));
     hipStream_t s = as_stream(stream);
-    RCH_DISPATCH_DTYPE(src_dtype, "rch_fit_project", project_kernel, grid, mats_dev, channels);
+    const unsigned z = static_cast<unsigned>(n_mats);
+    // The fewest rank chunks of at most 64 ranks, as equal as 16-rank blocks allow.
+    const int blocks = (max_rank + 15) / 16;
+    int chunks = (blocks + 3) / 4, chunk = 16 * ((blocks + chunks - 1) / chunks);
+    // 128-token workgroups while they fill the chip several times over; fewer leave CUs idle for most
+    // of the launch (one matrix [4680, 1536] at rank 96 is 74 of them), so the channel-split shape
+    // runs, in chunks of 32 ranks.
+    if ((max_rows + 127) / 128 * chunks * n_mats >= kProjectWholeGroups) {
+        const dim3 grid(static_cast<unsigned>((max_rows + 127) / 128), static_cast<unsigned>(chunks), z);
+        switch (src_dtype) {
+            case RCH_DT_BF16: hipLaunchKernelGGL((project_kernel<RCH_DT_BF16, 2, 1>), grid, dim3(kThreads), 0, s, mats_dev, channels, chunk); break;
+            case RCH_DT_F16: hipLaunchKernelGGL((project_kernel<RCH_DT_F16, 2, 1>), grid, dim3(kThreads), 0, s, mats_dev, channels, chunk); break;
+            case RCH_DT_F32: hipLaunchKernelGGL((project_kernel<RCH_DT_F32, 2, 1>), grid, dim3(kThreads), 0, s, mats_dev, channels, chunk); break;
+            default: return fail(RCH_E_CONFIG, "rch_fit_project: source dtype must be bf16, f16 or f32");
+        }
+    } else {
+        chunk = 32;
+        chunks = (max_rank + 31) / 32;
+        const dim3 grid(static_cast<unsigned>((max_rows + 15) / 16), static_cast<unsigned>(chunks), z);
+        switch (src_dtype) {
+            case RCH_DT_BF16: hipLaunchKernelGGL((project_kernel<RCH_DT_BF16, 1, 4>), grid, dim3(kThreads), 0, s, mats_dev, channels, chunk); break;
+            case RCH_DT_F16: hipLaunchKernelGGL((project_kernel<RCH_DT_F16, 1, 4>), grid, dim3(kThreads), 0, s, mats_dev, channels, chunk); break;
+            case RCH_DT_F32: hipLaunchKernelGGL((project_kernel<RCH_DT_F32, 1, 4>), grid, dim3(kThreads), 0, s, mats_dev, channels, chunk); break;
+            default: return fail(RCH_E_CONFIG, "rch_fit_project: source dtype must be bf16, f16 or f32");
+        }
+    }
     return check_launch("rch_fit_project");
 }
 
 int rch_fit_residual(const rch_fit_matrix* mats_dev, int n_mats, int channels, int64_t max_rows, int src_dtype,
                      void* stream) {
     if (int status = check_matrices(mats_dev, n_mats, channels, "rch_fit_residual")) return status;
-    if (max_rows <= 0 || (max_rows + 63) / 64 > 0x7fffffff) return fail(RCH_E_CONFIG, "rch_fit_residual: invalid max_rows");
-    const dim3 grid(static_cast<unsigned>((max_rows + 63) / 64), static_cast<unsigned>(n_mats));
+    if (max_rows <= 0 || (max_rows + 15) / 16 > 0x7fffffff) return fail(RCH_E_CONFIG, "rch_fit_residual: invalid max_rows");
     hipStream_t s = as_stream(stream);
-    RCH_DISPATCH_DTYPE(src_dtype, "rch_fit_residual", residual_kernel, grid, mats_dev, channels);
+    // 32-token workgroups while they fill the chip, else 16-token ones with the channels split.
+    const int tokens = (max_rows + 31) / 32 * n_mats >= kResidualPairGroups ? 32 : 16;
+    int splits = 1;
+    if (tokens == 16) {
+        const int64_t groups = (max_rows + 15) / 16 * n_mats, most = (channels + 255) / 256;
+        const int64_t wanted = (kResidualSplitGroups + groups - 1) / groups;
+        splits = static_cast<int>(wanted < most ? wanted : most);
+        splits = splits > RCH_RESIDUAL_SPLITS ? RCH_RESIDUAL_SPLITS : splits;
+    }
+    const dim3 grid(static_cast<unsigned>((max_rows + tokens - 1) / tokens), static_cast<unsigned>(n_mats),
+                    static_cast<unsigned>(splits));
+    switch (src_dtype) {
+        case RCH_DT_BF16:
+            if (tokens == 32) hipLaunchKernelGGL((residual_kernel<RCH_DT_BF16, 2>), grid, dim3(kThreads), 0, s, mats_dev, channels);
+            else hipLaunchKernelGGL((residual_kernel<RCH_DT_BF16, 1>), grid, dim3(kThreads), 0, s, mats_dev, channels);
+            break;
+        case RCH_DT_F16:
+            if (tokens == 32) hipLaunchKernelGGL((residual_kernel<RCH_DT_F16, 2>), grid, dim3(kThreads), 0, s, mats_dev, channels);
+            else hipLaunchKernelGGL((residual_kernel<RCH_DT_F16, 1>), grid, dim3(kThreads), 0, s, mats_dev, channels);
+            break;
+        case RCH_DT_F32:
+            if (tokens == 32) hipLaunchKernelGGL((residual_kernel<RCH_DT_F32, 2>), grid, dim3(kThreads), 0, s, mats_dev, channels);
+            else hipLaunchKernelGGL((residual_kernel<RCH_DT_F32, 1>), grid, dim3(kThreads), 0, s, mats_dev, channels);
+            break;
+        default: return fail(RCH_E_CONFIG, "rch_fit_residual: source dtype must be bf16, f16 or f32");
+    }
     if (int status = check_launch("rch_fit_residual")) return status;
-    hipLaunchKernelGGL(energy_total_kernel, dim3(n_mats), dim3(64), 0, s, mats_dev);
+    hipLaunchKernelGGL(energy_total_kernel, dim3(n_mats), dim3(64), 0, s, mats_dev, tokens, splits);
     return check_launch("rch_fit_residual (totals)");
 }
 

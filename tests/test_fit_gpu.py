@@ -308,3 +308,60 @@ def test_cholesky_inverse_flags_indefinite_members(device):
     assert (inverse[1] == np.eye(k)).all() and (inverse[2] == np.eye(k)).all()
     with pytest.raises(Exception):
         fk.cholesky_inverse(torch.zeros((1, 129, 129), dtype=torch.float64, device=device))
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16", "float32"])
+@pytest.mark.parametrize("count,rows,channels,ranks", [
+    (1, 17, 72, [1]),                   # one 16-token tile and a row of the next; channels below one step of each wave
+    (1, 4680, 264, [96]),               # channel-split projection and residual, several channel parts
+    (3, 31, 136, [16, 33, 130]),        # ragged ranks over several rank chunks
+    (70, 2000, 64, [49]),               # token-blocked shapes (32-token workgroups), 64-channel rows
+    (160, 1664, 40, [32]),              # 128-token projection workgroups
+])
+def test_fit_launch_shapes_match_fp64(device, dtype, count, rows, channels, ranks):
+    """absmax, projection and residual energies on both sides of their launch-shape rules: maxima
+    exact, P within an ulp of the rounded FP64 product (equal on 99.99 %), energies within 1e-12, the
+    first, last and middle matrices of a batch against numpy."""
+    rng = np.random.default_rng(83)
+    x, _ = _source(rng, rows, channels, dtype, device)
+    sources = [x * (1 + i % 3) if i % 2 else -x for i in range(count)]
+    ranks = [min(ranks[i % len(ranks)], rows, channels) for i in range(count)]
+    bases = [_basis(rng, rank, channels, device) for rank in ranks[:3]]
+    chosen = [bases[i % len(bases)] for i in range(count)]
+    ranks = [int(q.shape[0]) for q, _ in chosen]
+    keys = fk.absmax(sources)
+    coefficients, extrema = fk.project(sources, [q for q, _ in chosen], ranks, extrema=True)
+    totals = fk.energies(sources, keys, bases=[q for q, _ in chosen], ranks=ranks, coefficients=coefficients).cpu().numpy()
+    alone = fk.energies(sources, keys).cpu().numpy()
+    for i in sorted({0, count // 2, count - 1}):
+        host = sources[i].double().cpu().numpy()
+        q = np.asarray(chosen[i][1], dtype=np.float16).astype(np.float64)[:ranks[i]]
+        bits = np.abs(host).max().astype(np.float32).view(np.int32)
+        assert int(keys[i]) == int(bits)
+        p, want = coefficients[i].cpu().numpy(), (host @ q.T).astype(np.float32)
+        assert (p != want).mean() <= 1e-4
+        assert np.abs(p.view(np.int32).astype(np.int64) - want.view(np.int32).astype(np.int64)).max() <= 1
+        low, high = fk.split_keys(extrema[i].cpu().numpy(), ranks[i])
+        np.testing.assert_array_equal(low, p.min(0))
+        np.testing.assert_array_equal(high, p.max(0))
+        scale = np.abs(host).max()
+        source = np.square(host / scale).sum()
+        error = np.square((host - p.astype(np.float64) @ q) / scale).sum()
+        assert totals[i, 0] == pytest.approx(source, rel=1e-12) and alone[i, 0] == pytest.approx(source, rel=1e-12)
+        assert totals[i, 1] == pytest.approx(error, rel=1e-12)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16", "float32"])
+def test_absmax_flags_nonfinite_values(device, dtype):
+    """An infinity or a NaN anywhere (first and last element, either sign) puts the key at or above
+    the infinity's bits; the other matrices of the batch keep their exact maxima."""
+    values = torch.zeros((37, 48), dtype=DTYPES[dtype], device=device)
+    values[5, 7] = -3.5
+    bad = []
+    for value, at in ((float("inf"), (0, 0)), (float("-inf"), (36, 47)), (float("nan"), (36, 40)), (-float("nan"), (0, 7))):
+        member = values.clone()
+        member[at] = value
+        bad.append(member)
+    keys = fk.absmax([values] + bad + [torch.zeros_like(values)]).cpu().numpy()
+    assert keys[0] == np.float32(3.5).view(np.int32) and keys[-1] == 0
+    assert (keys[1:-1] >= fk.NONFINITE_BITS).all()
