@@ -16,7 +16,7 @@ import numpy as np
 from .errors import ConfigurationError, UnsupportedError
 
 LIBRARY = Path(__file__).resolve().with_name("libreelcache_hip.so")
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 # Status codes (RCH_E_*).
 OK, E_CONFIG, E_UNSUPPORTED, E_LAUNCH = 0, 1, 2, 3
@@ -89,6 +89,7 @@ _SIGNATURES = {
     "rch_quantize": ([_p, _i64, _i, _i64, _p, _p, _p, _i64, _p], _i),
     "rch_quantize_batched": ([_p, _i, _i64, _p], _i),
     "rch_cholesky_inverse": ([_p, _p, _p, _i, _i, _p], _i),
+    "rch_fit_span": ([_p, _i, _i, _i64, _i, _i, _p], _i),
     "rch_fit_gaussian": ([_p, _i, _i64, _p], _i),
 }
 # Further entry points registered by other modules are bound when present.

@@ -398,8 +398,9 @@ __global__ void __launch_bounds__(kGramThreads) gram_kernel(const rch_fit_matrix
 //     workgroup = 128 tokens x 64 ranks.
 //   * TB = 1, SPLIT = 4: for batches that would leave CUs idle, the four waves of a workgroup share 16
 //     tokens and split the channel steps; the partial sums are added through LDS in wave order.
+// GRAM: the sources are the basis rows themselves and the FP64 sums are stored as they are, G = Q Q^T.
 // One bf16 matrix [4680, 1536] at rank 96: 105 us with 64-token workgroups of one wave per 16 tokens and
-// loads in the step, 32 us now; 60 matrices at rank 96: 1563 -> 1396 us (59 of the 68 TFLOP/s that a
+// loads in the step, 36 us now; 60 matrices at rank 96: 1563 -> 1396 us (59 of the 68 TFLOP/s that a
 // large library FP64 product reaches on this card).
 // ---------------------------------------------------------------------------------------------
 
@@ -421,18 +422,25 @@ __device__ __forceinline__ double eight_at(const Eight<DT>& e, int i) {
     else return static_cast<double>(half_bits<DT>((e.w[0][i >> 1] >> (16 * (i & 1))) & 0xffffu));
 }
 
-template <int DT, int TB, int SPLIT, int NB>
+// Order of the padded FP64 k x k matrices of the span kernels.
+__device__ __forceinline__ int padded_order(int rank) { return (rank + 15) & ~15; }
+
+template <int DT, int TB, int SPLIT, int NB, bool GRAM = false>
 __device__ __forceinline__ void project_ranks(const rch_fit_matrix* M, int channels, int r0, int64_t wt, int wave, int lane,
                                               double* partial) {
     constexpr int E = esize<DT>();
-    const int64_t rows = M->rows;
+    static_assert(!GRAM || (DT == RCH_DT_F16 && SPLIT > 1), "the basis Gram runs on fp16 rows, channels split");
     const int rank = static_cast<int>(M->rank);
+    const int64_t rows = GRAM ? rank : M->rows;
     const int g = lane >> 4, i16 = lane & 15;
-    const __amdgpu_buffer_rsrc_t xs = source_rows<DT>(M, channels, wt);
     const __amdgpu_buffer_rsrc_t qs = make_rsrc(M->basis_ptr, ((rank - 1) * M->basis_stride + channels) * 2);
+    const __amdgpu_buffer_rsrc_t xs = GRAM ? qs : source_rows<DT>(M, channels, wt);
     uint32_t x_row[TB], q_row[NB];
 #pragma unroll
-    for (int t = 0; t < TB; ++t) x_row[t] = static_cast<uint32_t>((16 * t + i16) * M->src_stride * E);
+    for (int t = 0; t < TB; ++t) {
+        if constexpr (GRAM) x_row[t] = wt + i16 < rank ? static_cast<uint32_t>((wt + i16) * M->basis_stride * 2) : kOutOfRange;
+        else x_row[t] = static_cast<uint32_t>((16 * t + i16) * M->src_stride * E);
+    }
 #pragma unroll
     for (int b = 0; b < NB; ++b)  // rows past the rank read zeros
         q_row[b] = r0 + 16 * b + i16 < rank ? static_cast<uint32_t>((r0 + 16 * b + i16) * M->basis_stride * 2) : kOutOfRange;
@@ -488,6 +496,12 @@ __device__ __forceinline__ void project_ranks(const rch_fit_matrix* M, int chann
 #pragma unroll
             for (int v = 0; v < 4; ++v) sum[v] += partial[((wave * SPLIT + w) * 4 + v) * 64 + lane];
         acc[0][0] = sum;
+        if constexpr (GRAM) {  // rows and columns past the rank are zeros
+            const int kp = padded_order(rank), k = r0 + 16 * wave + i16;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) gout<double>(M->gram_ptr)[(wt + g + 4 * v) * kp + k] = sum[v];
+            return;
+        }
     }
     RCH_GLOBAL float* out = gout<float>(M->coef_ptr);
     unsigned int* ext = reinterpret_cast<unsigned int*>(M->extrema_ptr);
@@ -562,7 +576,7 @@ __global__ void __launch_bounds__(kThreads, 2) project_kernel(const rch_fit_matr
 // Bound by the FP64 matrix rate (rank 0, the source energy alone: by HBM): the next step's operands
 // and the next group's source elements are loaded before a step's products.  TB = 2 lets each
 // converted basis operand feed two products; small batches take TB = 1 and split the channels over
-// workgroups (grid z) until they fill the chip.  One bf16 matrix [4680, 1536] at rank 96: 137 -> 41 us;
+// workgroups (grid z) until they fill the chip.  One bf16 matrix [4680, 1536] at rank 96: 137 -> 40 us;
 // 60 matrices: 1808 -> 1527 us (54 TFLOP/s); source energy of one: 29 -> 18 us.
 // ---------------------------------------------------------------------------------------------
 
@@ -743,8 +757,11 @@ __global__ void __launch_bounds__(64) energy_total_kernel(const rch_fit_matrix* 
 }
 
 // ---------------------------------------------------------------------------------------------
-// Column extrema and the FP64 quantizer of an fp32 [rows, cols] matrix: workgroup = 64 rows,
-// threads stride over the columns (consecutive threads, consecutive columns).
+// Column extrema (workgroup = 64 rows, a thread per column) and the FP64 quantizer of fp32 [rows, cols]
+// matrices.  Both are latency-bound at archive sizes.  The quantizer spreads a tile's rows and columns
+// over all threads: one [4680, 96] matrix takes 5 us (15 us with a thread per column and 64 rows in
+// turn), 60 of mixed ranks 42 us (76).  The extrema, spread the same way over 4 or 16 waves, took 10
+// and 12 us against 10: they wait for their atomics.
 // ---------------------------------------------------------------------------------------------
 
 __global__ void __launch_bounds__(kThreads) extrema_kernel(const float* __restrict__ values, int64_t rows, int cols,
@@ -763,41 +780,67 @@ __global__ void __launch_bounds__(kThreads) extrema_kernel(const float* __restri
     }
 }
 
-__global__ void __launch_bounds__(kThreads) quantize_kernel(const float* __restrict__ values, int64_t rows, int cols,
-                                                            int64_t stride, const double* __restrict__ scale,
-                                                            const double* __restrict__ offset,
-                                                            uint8_t* __restrict__ codes, int64_t code_stride) {
-    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * 64;
-    const int64_t r1 = rows - r0 < 64 ? rows : r0 + 64;
-    for (int c = threadIdx.x; c < cols; c += kThreads) {
-        const double sc = scale[c], of = offset[c];
-        for (int64_t r = r0; r < r1; ++r) {
+constexpr int kQuantizeRows = 16;  // rows per workgroup
+
+// Codes of rows [r0, r0 + kQuantizeRows): a thread takes four consecutive columns of a row.
+__device__ __forceinline__ void quantize_rows(const RCH_GLOBAL float* values, int64_t r0, int64_t rows, int cols, int64_t stride,
+                                              const RCH_GLOBAL double* scale, const RCH_GLOBAL double* offset,
+                                              RCH_GLOBAL uint8_t* codes, int64_t code_stride) {
+    const int groups = (cols + 3) >> 2;
+    const int left = static_cast<int>(rows - r0 < kQuantizeRows ? rows - r0 : kQuantizeRows);
+    const bool vec = ((reinterpret_cast<int64_t>(values) | (stride * 4)) & 15) == 0;
+    const bool words = ((reinterpret_cast<int64_t>(codes) | code_stride) & 3) == 0;
+    for (int i = threadIdx.x; i < left * groups; i += kThreads) {
+        const int row = i / groups, c = 4 * (i - row * groups);
+        const RCH_GLOBAL float* v = values + (r0 + row) * stride + c;
+        const bool whole = c + 4 <= cols;
+        float x[4];
+        if (vec && whole) {
+            const f4 w = *reinterpret_cast<const RCH_GLOBAL f4*>(v);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) x[j] = w[j];
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) x[j] = c + j < cols ? v[j] : 0.0f;
+        }
+        uint32_t word = 0u;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (c + j >= cols) continue;
+            const double sc = scale[c + j], of = offset[c + j];
             double q = 0.0;
-            if (sc > 0.0) q = rint((static_cast<double>(values[r * stride + c]) - of) / sc);
+            if (sc > 0.0) q = rint((static_cast<double>(x[j]) - of) / sc);
             q = q < 0.0 ? 0.0 : (q > 255.0 ? 255.0 : q);
-            codes[r * code_stride + c] = static_cast<uint8_t>(q);
+            word |= static_cast<uint32_t>(static_cast<uint8_t>(q)) << (8 * j);
+        }
+        RCH_GLOBAL uint8_t* out = codes + (r0 + row) * code_stride + c;
+        if (words && whole) {
+            *reinterpret_cast<RCH_GLOBAL uint32_t*>(out) = word;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (c + j < cols) out[j] = static_cast<uint8_t>(word >> (8 * j));
         }
     }
 }
 
+__global__ void __launch_bounds__(kThreads) quantize_kernel(const float* __restrict__ values, int64_t rows, int cols,
+                                                            int64_t stride, const double* __restrict__ scale,
+                                                            const double* __restrict__ offset,
+                                                            uint8_t* __restrict__ codes, int64_t code_stride) {
+    quantize_rows(gin<float>(reinterpret_cast<int64_t>(values)), static_cast<int64_t>(blockIdx.x) * kQuantizeRows, rows, cols,
+                  stride, gin<double>(reinterpret_cast<int64_t>(scale)), gin<double>(reinterpret_cast<int64_t>(offset)),
+                  gout<uint8_t>(reinterpret_cast<int64_t>(codes)), code_stride);
+}
+
 __global__ void __launch_bounds__(kThreads) quantize_batched_kernel(const rch_quantize_job* __restrict__ jobs) {
     const rch_quantize_job* J = jobs + blockIdx.y;
-    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * 64;
+    const int64_t r0 = static_cast<int64_t>(blockIdx.x) * kQuantizeRows;
     if (r0 >= J->rows) return;
-    const int64_t r1 = J->rows - r0 < 64 ? J->rows : r0 + 64;
     const int cols = static_cast<int>(J->cols);
-    const RCH_GLOBAL float* values = gin<float>(J->values_ptr);
     const RCH_GLOBAL double* affine = gin<double>(J->affine_ptr);
-    RCH_GLOBAL uint8_t* codes = gout<uint8_t>(J->codes_ptr);
-    for (int c = threadIdx.x; c < cols; c += kThreads) {
-        const double sc = affine[c], of = affine[cols + c];
-        for (int64_t r = r0; r < r1; ++r) {
-            double q = 0.0;
-            if (sc > 0.0) q = rint((static_cast<double>(values[r * J->stride + c]) - of) / sc);
-            q = q < 0.0 ? 0.0 : (q > 255.0 ? 255.0 : q);
-            codes[r * J->code_stride + c] = static_cast<uint8_t>(q);
-        }
-    }
+    quantize_rows(gin<float>(J->values_ptr), r0, J->rows, cols, J->stride, affine, affine + cols, gout<uint8_t>(J->codes_ptr),
+                  J->code_stride);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -834,25 +877,27 @@ __device__ __forceinline__ double broadcast_lane(double v, int lane) {
                                           static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(w[1]), lane))}));
 }
 
-__global__ void __launch_bounds__(kCholThreads) cholesky_inverse_kernel(const double* __restrict__ a,
-                                                                         double* __restrict__ x,
-                                                                         int32_t* __restrict__ info, int k) {
+struct CholeskyShared {
+    double m[RCH_CHOLESKY_MAX_K * kCholPitch];   // A, then R; below the diagonal blocks X transposed by blocks
+    double inverse_diagonal[kCholBlocks][16 * 16];  // X_JJ
+    double pivot_inverse[RCH_CHOLESKY_MAX_K];    // 1 / R[j][j]
+    int failed_at;
+};
+
+// Factors the padded matrix in shared.m (upper triangle; visible to the workgroup) and inverts the
+// factor; store(row, column, value) takes the upper-triangular X in blocks.  Returns 0, or the order of
+// the first leading minor that is not positive definite (no X then).  Uniform over the workgroup.
+template <class Store>
+__device__ __forceinline__ int cholesky_invert(CholeskyShared& shared, int k, Store store) {
     constexpr int P = kCholPitch;
-    __shared__ double m[RCH_CHOLESKY_MAX_K * P];  // A, then R; below the diagonal blocks X transposed by blocks
-    __shared__ double inverse_diagonal[kCholBlocks][16 * 16];  // X_JJ
-    __shared__ double pivot_inverse[RCH_CHOLESKY_MAX_K];  // 1 / R[j][j]
-    __shared__ int failed_at;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    double* const m = shared.m;
+    double* const pivot_inverse = shared.pivot_inverse;
+    auto& inverse_diagonal = shared.inverse_diagonal;
+    int& failed_at = shared.failed_at;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i16 = lane & 15, g = lane >> 4;
     const int blocks = (k + 15) >> 4, kp = 16 * blocks;
-    const int64_t base = static_cast<int64_t>(blockIdx.x) * k * k;
-    const RCH_GLOBAL double* A = gin<double>(reinterpret_cast<int64_t>(a)) + base;
-    RCH_GLOBAL double* X = gout<double>(reinterpret_cast<int64_t>(x)) + base;
-    if (tid == 0) failed_at = 0;
-    for (int i = wave; i < kp; i += kCholWaves)
-        for (int c = i + lane; c < kp; c += 64) m[i * P + c] = (i < k && c < k) ? A[i * k + c] : (i == c ? 1.0 : 0.0);
-    __syncthreads();
     for (int J = 0; J < blocks; ++J) {
         const int j0 = 16 * J;
         const int right = kp - j0 - 16;  // columns beside the diagonal block
@@ -913,12 +958,7 @@ __global__ void __launch_bounds__(kCholThreads) cholesky_inverse_kernel(const do
         }
         __syncthreads();
     }
-    if (failed_at) {
-        for (int i = wave; i < k; i += kCholWaves)
-            for (int c = lane; c < k; c += 64) X[i * k + c] = i == c ? 1.0 : 0.0;
-        if (tid == 0) info[blockIdx.x] = failed_at;
-        return;
-    }
+    if (failed_at) return failed_at;
     if (wave < blocks) {
         const int J = wave;
         for (int I = J; I >= 0; --I) {
@@ -964,12 +1004,256 @@ __global__ void __launch_bounds__(kCholThreads) cholesky_inverse_kernel(const do
             const int col = 16 * J + i16;
 #pragma unroll
             for (int r = 0; r < 16; ++r)
-                if ((r & 3) == g && 16 * I + r < k && col < k) X[(16 * I + r) * k + col] = y[r];
+                if ((r & 3) == g) store(16 * I + r, col, y[r]);
         }
-        for (int row = 16 * (J + 1) + g; row < k; row += 4)
-            if (16 * J + i16 < k) X[row * k + 16 * J + i16] = 0.0;
     }
-    if (tid == 0) info[blockIdx.x] = 0;
+    return 0;
+}
+
+// Upper triangle of A (order k) into shared.m, padded to whole blocks with the identity.
+__device__ __forceinline__ void cholesky_load(CholeskyShared& shared, const RCH_GLOBAL double* A, int k, int pitch) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kp = padded_order(k);
+    if (threadIdx.x == 0) shared.failed_at = 0;
+    for (int i = wave; i < kp; i += kCholWaves)
+        for (int c = i + lane; c < kp; c += 64)
+            shared.m[i * kCholPitch + c] = (i < k && c < k) ? A[i * pitch + c] : (i == c ? 1.0 : 0.0);
+    __syncthreads();
+}
+
+__global__ void __launch_bounds__(kCholThreads) cholesky_inverse_kernel(const double* __restrict__ a,
+                                                                         double* __restrict__ x,
+                                                                         int32_t* __restrict__ info, int k) {
+    __shared__ CholeskyShared shared;
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * k * k;
+    RCH_GLOBAL double* X = gout<double>(reinterpret_cast<int64_t>(x)) + base;
+    cholesky_load(shared, gin<double>(reinterpret_cast<int64_t>(a)) + base, k, k);
+    const int failed = cholesky_invert(shared, k, [&](int row, int col, double value) {
+        if (row < k && col < k) X[row * k + col] = value;
+    });
+    if (threadIdx.x == 0) info[blockIdx.x] = failed;
+    // The identity for a failed member, else zeros below the diagonal blocks.
+    for (int e = threadIdx.x; e < k * k; e += kCholThreads) {
+        const int row = e / k, col = e - row * k;
+        if (failed) X[e] = row == col ? 1.0 : 0.0;
+        else if ((row >> 4) > (col >> 4)) X[e] = 0.0;
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Terms of a stored basis view Q (order k <= RCH_CHOLESKY_MAX_K) and its coefficients P: the span trace
+// trace(G^-1 C) with G = Q Q^T and C = P^T P, the Cholesky status of G, ||G - I||_inf, max |G_ii|,
+// ||G||_inf and ||G^-1||_inf, in FP64.  Four launches for a batch of any ranks in place of some twenty
+// library launches per rank group; each is latency- or FP64-rate-bound at a few tens of us:
+//   * basis_gram_kernel: G (the projection's channel-split body on the basis rows);
+//   * basis_terms_kernel: factor, X = R^-1, W = X X^T = G^-1 and the norms, one workgroup per matrix;
+//   * span_trace_kernel: sum over tiles of W o C.  A workgroup keeps its token range's share of C in
+//     accumulators and multiplies it by W at the end, so C is never written;
+//   * span_total_kernel: the workgroups' sums in order.
+// ---------------------------------------------------------------------------------------------
+
+__global__ void __launch_bounds__(kThreads) basis_gram_kernel(const rch_fit_matrix* __restrict__ mats, int channels) {
+    __shared__ double partial[4 * 4 * 4 * 64];
+    const rch_fit_matrix* M = mats + blockIdx.z;
+    const int kp = padded_order(static_cast<int>(M->rank));
+    const int t0 = 16 * blockIdx.x, r0 = 32 * blockIdx.y;
+    if (t0 >= kp || r0 >= kp) return;  // whole workgroup
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (r0 + 16 < kp) project_ranks<RCH_DT_F16, 1, 4, 2, true>(M, channels, r0, t0, wave, lane, partial);
+    else project_ranks<RCH_DT_F16, 1, 4, 1, true>(M, channels, r0, t0, wave, lane, partial);
+}
+
+__global__ void __launch_bounds__(kCholThreads) basis_terms_kernel(const rch_fit_matrix* __restrict__ mats) {
+    __shared__ CholeskyShared shared;
+    constexpr int P = kCholPitch;
+    const rch_fit_matrix* M = mats + blockIdx.x;
+    const int k = static_cast<int>(M->rank), kp = padded_order(k), blocks = kp >> 4;
+    const RCH_GLOBAL double* G = gin<double>(M->gram_ptr);
+    RCH_GLOBAL double* W = gout<double>(M->gram_ptr) + kp * kp;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i16 = lane & 15, g = lane >> 4;
+    cholesky_load(shared, G, k, kp);
+    // Row norms of G: four threads per row (k <= 128 rows), then the largest of the workgroup.
+    const int row = tid >> 2, part = tid & 3;
+    double eta = 0.0, largest = 0.0, norm = 0.0;
+    if (row < k) {
+        for (int c = part; c < k; c += 4) {
+            const double v = G[row * kp + c];
+            norm += fabs(v);
+            eta += fabs(c == row ? v - 1.0 : v);
+            if (c == row) largest = fabs(v);
+        }
+    }
+    const int failed = cholesky_invert(shared, k, [](int, int, double) {});
+    __syncthreads();
+    // W_IJ = sum_{Q >= J} X_IQ X_JQ^T for I <= J, into the blocks R no longer needs.
+    double* const m = shared.m;
+    if (!failed) {
+        auto x_at = [&](int I, int Q) -> const double* {
+            return I == Q ? shared.inverse_diagonal[I] : m + 16 * Q * P + 16 * I;
+        };
+        for (int t = wave; t < blocks * (blocks + 1) / 2; t += kCholWaves) {
+            int J = 0, I = t;
+            while (I > J) {
+                I -= J + 1;
+                ++J;
+            }
+            d4 acc = d4{};
+            for (int Q = J; Q < blocks; ++Q) {
+                const double* left = x_at(I, Q);
+                const double* right = x_at(J, Q);
+                const int lp = I == Q ? 16 : P, rp = J == Q ? 16 : P;
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(left[i16 * lp + 4 * s + g], right[i16 * rp + 4 * s + g], acc, 0, 0, 0);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                m[(16 * I + g + 4 * v) * P + 16 * J + i16] = acc[v];
+                W[(16 * I + g + 4 * v) * kp + 16 * J + i16] = acc[v];
+            }
+        }
+    }
+    __syncthreads();
+    double inverse_norm = 0.0;
+    if (row < k) {
+        // Upper blocks hold W; entries below the diagonal blocks come from the transposed place.
+        for (int c = part; c < k; c += 4)
+            inverse_norm += fabs((c >> 4) >= (row >> 4) ? m[row * P + c] : m[c * P + row]);
+    }
+#pragma unroll
+    for (int d = 1; d <= 2; d <<= 1) {
+        norm += __shfl_xor(norm, d);
+        eta += __shfl_xor(eta, d);
+        largest = fmax(largest, __shfl_xor(largest, d));
+        inverse_norm += __shfl_xor(inverse_norm, d);
+    }
+    // A NaN must survive the maximum: row sums that are not finite become infinity.
+    norm = norm < INFINITY ? norm : INFINITY;
+    eta = eta < INFINITY ? eta : INFINITY;
+    inverse_norm = inverse_norm < INFINITY ? inverse_norm : INFINITY;
+#pragma unroll
+    for (int d = 4; d <= 32; d <<= 1) {
+        norm = fmax(norm, __shfl_xor(norm, d));
+        eta = fmax(eta, __shfl_xor(eta, d));
+        largest = fmax(largest, __shfl_xor(largest, d));
+        inverse_norm = fmax(inverse_norm, __shfl_xor(inverse_norm, d));
+    }
+    __syncthreads();
+    double* const best = shared.pivot_inverse;
+    if (lane == 0) {
+        best[4 * wave] = eta;
+        best[4 * wave + 1] = largest;
+        best[4 * wave + 2] = norm;
+        best[4 * wave + 3] = inverse_norm;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        RCH_GLOBAL double* out = gout<double>(M->energy_ptr);
+        out[0] = 0.0;
+        out[1] = static_cast<double>(failed);
+        for (int q = 0; q < 4; ++q) {
+            double v = best[q];
+            for (int w = 1; w < kCholWaves; ++w) v = fmax(v, best[4 * w + q]);
+            out[2 + q] = v;
+        }
+        if (failed) out[5] = INFINITY;
+    }
+}
+
+constexpr int kSpanThreads = 512;
+constexpr int kSpanWaves = kSpanThreads / 64;
+constexpr int kSpanTokens = 32;  // tokens staged at a time
+constexpr int kSpanTiles = (kCholBlocks * (kCholBlocks + 1) / 2 + kSpanWaves - 1) / kSpanWaves;  // per wave
+
+// Workgroup (token range, matrix): the 16 x 16 tiles (ti <= tj) of C are dealt to the waves; 32 tokens
+// of P at a time are staged in LDS as doubles, the next 32 loaded meanwhile.
+__global__ void __launch_bounds__(kSpanThreads) span_trace_kernel(const rch_fit_matrix* __restrict__ mats) {
+    constexpr int kPitch = RCH_CHOLESKY_MAX_K + 16;
+    __shared__ double staged[kSpanTokens * kPitch];
+    __shared__ double sums[kSpanWaves];
+    const rch_fit_matrix* M = mats + blockIdx.y;
+    const int k = static_cast<int>(M->rank), kp = padded_order(k), blocks = kp >> 4;
+    const int tiles = blocks * (blocks + 1) / 2;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i16 = lane & 15, g = lane >> 4;
+    const int64_t share = (M->rows + gridDim.x - 1) / gridDim.x;
+    const int64_t per = (share + kSpanTokens - 1) / kSpanTokens * kSpanTokens;
+    const int64_t begin = blockIdx.x * per, end = begin + per < M->rows ? begin + per : M->rows;
+    int ti[kSpanTiles], tj[kSpanTiles];
+    d4 acc[kSpanTiles];
+#pragma unroll
+    for (int q = 0; q < kSpanTiles; ++q) {
+        int J = 0, I = wave + kSpanWaves * q;
+        while (I > J) {
+            I -= J + 1;
+            ++J;
+        }
+        ti[q] = 16 * I;
+        tj[q] = 16 * J;
+        acc[q] = d4{};
+    }
+    // Thread -> (token, columns 8 part .. 8 part + 7) of a 32-token stage.
+    const int token = tid >> 4, part = tid & 15;
+    const bool mine = 8 * part < kp;
+    float next[8];
+    auto load = [&](int64_t t0) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) next[j] = 0.0f;
+        if (mine && t0 + token < end) {
+            const RCH_GLOBAL float* p = gin<float>(M->coef_ptr) + (t0 + token) * M->coef_stride + 8 * part;
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (8 * part + j < k) next[j] = p[j];
+        }
+    };
+    load(begin);
+    for (int64_t t0 = begin; t0 < end; t0 += kSpanTokens) {
+        if (mine) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) staged[token * kPitch + 8 * part + j] = static_cast<double>(next[j]);
+        }
+        __syncthreads();
+        load(t0 + kSpanTokens);
+#pragma unroll
+        for (int q = 0; q < kSpanTiles; ++q) {
+            if (wave + kSpanWaves * q >= tiles) continue;  // uniform
+#pragma unroll
+            for (int s = 0; s < kSpanTokens / 4; ++s) {
+                const double* r = staged + (4 * s + g) * kPitch + i16;
+                acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(r[ti[q]], r[tj[q]], acc[q], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+    }
+    const RCH_GLOBAL double* W = gin<double>(M->gram_ptr) + kp * kp;
+    double sum = 0.0;
+#pragma unroll
+    for (int q = 0; q < kSpanTiles; ++q) {
+        if (wave + kSpanWaves * q >= tiles) continue;
+        double tile = 0.0;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) tile = fma(W[(ti[q] + g + 4 * v) * kp + tj[q] + i16], acc[q][v], tile);
+        sum += ti[q] == tj[q] ? tile : 2.0 * tile;
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d);
+    if (lane == 0) sums[wave] = sum;
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < kSpanWaves; ++w) sum += sums[w];
+        gout<double>(M->partial_ptr)[blockIdx.x] = sum;
+    }
+}
+
+// The span trace of each matrix from its workgroups' sums, in order (0 when G is not positive definite).
+__global__ void __launch_bounds__(64) span_total_kernel(const rch_fit_matrix* __restrict__ mats, int n, int splits) {
+    const int mat = blockIdx.x * 64 + threadIdx.x;
+    if (mat >= n) return;
+    const rch_fit_matrix* M = mats + mat;
+    RCH_GLOBAL double* out = gout<double>(M->energy_ptr);
+    double sum = 0.0;
+    for (int s = 0; s < splits; ++s) sum += gin<double>(M->partial_ptr)[s];
+    out[0] = out[1] == 0.0 ? sum : 0.0;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1166,9 +1450,9 @@ int rch_column_extrema(const float* values_dev, int64_t rows, int cols, int64_t 
 int rch_quantize(const float* values_dev, int64_t rows, int cols, int64_t stride, const double* scale_dev,
                  const double* offset_dev, uint8_t* codes_dev, int64_t code_stride, void* stream) {
     if (!values_dev || !scale_dev || !offset_dev || !codes_dev || rows <= 0 || cols <= 0 || stride < cols ||
-        code_stride < cols || (rows + 63) / 64 > 0x7fffffff)
+        code_stride < cols || (rows + kQuantizeRows - 1) / kQuantizeRows > 0x7fffffff)
         return fail(RCH_E_CONFIG, "rch_quantize: invalid arguments");
-    hipLaunchKernelGGL(quantize_kernel, dim3(static_cast<unsigned>((rows + 63) / 64)), dim3(kThreads), 0,
+    hipLaunchKernelGGL(quantize_kernel, dim3(static_cast<unsigned>((rows + kQuantizeRows - 1) / kQuantizeRows)), dim3(kThreads), 0,
                        as_stream(stream), values_dev, rows, cols, stride, scale_dev, offset_dev, codes_dev, code_stride);
     return check_launch("rch_quantize");
 }
@@ -1181,6 +1465,28 @@ int rch_cholesky_inverse(const double* a_dev, double* x_dev, int32_t* info_dev, 
     return check_launch("rch_cholesky_inverse");
 }
 
+int rch_fit_span(const rch_fit_matrix* mats_dev, int n_mats, int channels, int64_t max_rows, int max_rank,
+                 int with_coefficients, void* stream) {
+    if (int status = check_matrices(mats_dev, n_mats, channels, "rch_fit_span")) return status;
+    if (max_rank <= 0 || max_rank > RCH_CHOLESKY_MAX_K || (with_coefficients && max_rows <= 0))
+        return fail(RCH_E_CONFIG, "rch_fit_span: 1 <= max_rank <= %d and positive max_rows required", RCH_CHOLESKY_MAX_K);
+    hipStream_t s = as_stream(stream);
+    const unsigned n = static_cast<unsigned>(n_mats);
+    hipLaunchKernelGGL(basis_gram_kernel, dim3((max_rank + 15) / 16, (max_rank + 31) / 32, n), dim3(kThreads), 0, s, mats_dev,
+                       channels);
+    hipLaunchKernelGGL(basis_terms_kernel, dim3(n), dim3(kCholThreads), 0, s, mats_dev);
+    if (with_coefficients) {
+        // Two workgroups per CU over the batch, at least one 32-token stage each.
+        const int64_t stages = (max_rows + kSpanTokens - 1) / kSpanTokens;
+        int64_t splits = (512 + n_mats - 1) / n_mats;
+        splits = splits < stages ? splits : stages;
+        splits = splits < RCH_SPAN_SPLITS ? splits : RCH_SPAN_SPLITS;
+        hipLaunchKernelGGL(span_trace_kernel, dim3(static_cast<unsigned>(splits), n), dim3(kSpanThreads), 0, s, mats_dev);
+        hipLaunchKernelGGL(span_total_kernel, dim3((n + 63) / 64), dim3(64), 0, s, mats_dev, n_mats, static_cast<int>(splits));
+    }
+    return check_launch("rch_fit_span");
+}
+
 int rch_fit_gaussian(const rch_gauss_job* jobs_dev, int n_jobs, int64_t max_elements, void* stream) {
     if (!jobs_dev || n_jobs <= 0 || n_jobs > 65535 || max_elements <= 0 || (max_elements + 1023) / 1024 > 0x7fffffff)
         return fail(RCH_E_CONFIG, "rch_fit_gaussian: invalid arguments");
@@ -1190,9 +1496,10 @@ int rch_fit_gaussian(const rch_gauss_job* jobs_dev, int n_jobs, int64_t max_elem
 }
 
 int rch_quantize_batched(const rch_quantize_job* jobs_dev, int n_jobs, int64_t max_rows, void* stream) {
-    if (!jobs_dev || n_jobs <= 0 || n_jobs > 65535 || max_rows <= 0 || (max_rows + 63) / 64 > 0x7fffffff)
+    if (!jobs_dev || n_jobs <= 0 || n_jobs > 65535 || max_rows <= 0 ||
+        (max_rows + kQuantizeRows - 1) / kQuantizeRows > 0x7fffffff)
         return fail(RCH_E_CONFIG, "rch_quantize_batched: invalid arguments");
-    const dim3 grid(static_cast<unsigned>((max_rows + 63) / 64), static_cast<unsigned>(n_jobs));
+    const dim3 grid(static_cast<unsigned>((max_rows + kQuantizeRows - 1) / kQuantizeRows), static_cast<unsigned>(n_jobs));
     hipLaunchKernelGGL(quantize_batched_kernel, grid, dim3(kThreads), 0, as_stream(stream), jobs_dev);
     return check_launch("rch_quantize_batched");
 }

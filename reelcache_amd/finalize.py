@@ -16,11 +16,12 @@ What a finalized tile records, per matrix ``X`` and its FP16 rank-view rows ``Q`
 MI355X design: a batch of tiles (a whole chunk: 60 CausVid matrices) is one launch each of the
 absmax, projection (with per-column extrema) and residual-energy kernels, per channel count.
 The span energy uses the identity ``||L^-1 P^T||_F^2 = trace(G^-1 C)`` with ``G = Q Q^T`` and
-``C = P^T P`` (FP64): per group of tiles of one rank, one batched product ``C``, one batched
-Cholesky factorization of ``G`` and one batched solve, instead of an ``N x r`` triangular solve
-per tile.  The fast condition bound's Gram is one batched fp32
-product.  Every scalar the host needs (scales, extrema, energies, traces, factorization status,
-condition terms) crosses in one transfer; the quantizer is one launch for the batch.
+``C = P^T P`` (FP64) instead of an ``N x r`` triangular solve per tile: four hand-written launches
+for the batch, whatever its ranks up to 128 (``fit_kernels.span_terms``, with the fast condition
+bound's terms from the same FP64 Gram); larger ranks take, per group of one rank, one batched
+product ``C``, one batched Cholesky factorization and one batched solve.  Every scalar the host
+needs (scales, extrema, energies, traces, factorization status, condition terms) crosses in one
+transfer; the quantizer is one launch for the batch.
 """
 
 from __future__ import annotations
@@ -168,7 +169,7 @@ def _check_item(item: FinalizeItem) -> int:
 
 
 def _rank_terms(coefficients, rows):
-    """Per tile of one rank: FP64 span trace ``trace(G^-1 C)`` (``G = Q Q^T``, ``C = P^T P``), the
+    """Per tile of one rank above the native kernels' order (``fit_kernels.span_terms``): FP64 span trace ``trace(G^-1 C)`` (``G = Q Q^T``, ``C = P^T P``), the
     Cholesky status of ``G``, and the fast condition terms (``eta = ||Q Q^T - I||_inf`` of the fp32
     Gram -- fp16 products are exact in fp32 -- and its largest diagonal entry): a handful of
     batched launches for the whole group."""
@@ -181,13 +182,8 @@ def _rank_terms(coefficients, rows):
         products = torch.stack([c.double().T @ c.double() for c in coefficients])
     q64 = q.double()
     gram = torch.bmm(q64, q64.mT)
-    if gram.shape[1] <= fit_kernels.CHOLESKY_MAX_K and gram.device.type == "cuda":
-        # G = R^T R, X = R^-1 (one launch for the group): trace(G^-1 C) = trace(X^T C X) = sum X * (C X).
-        inverse, info = fit_kernels.cholesky_inverse(gram)
-        traces = (inverse * torch.bmm(products, inverse)).sum((1, 2))
-    else:
-        factor, info = torch.linalg.cholesky_ex(gram)
-        traces = torch.cholesky_solve(products, factor).diagonal(dim1=1, dim2=2).sum(-1)
+    factor, info = torch.linalg.cholesky_ex(gram)
+    traces = torch.cholesky_solve(products, factor).diagonal(dim1=1, dim2=2).sum(-1)
     q32 = q.float()
     gram32 = torch.bmm(q32, q32.mT)
     largest = gram32.diagonal(dim1=1, dim2=2).abs().amax(-1)
@@ -205,10 +201,19 @@ def _launch_group(items, ranks):
     coefficients, extrema = fit_kernels.project(sources, rows, ranks, extrema=True)
     totals = fit_kernels.energies(sources, keys, bases=rows, ranks=ranks, coefficients=coefficients)
     n = len(items)
+    small = [index for index, rank in enumerate(ranks) if rank <= fit_kernels.CHOLESKY_MAX_K]
+    if len(small) == n:  # span trace, Cholesky status and condition terms of every tile in one call
+        terms = fit_kernels.span_terms(rows, ranks, coefficients)[:, :4].T
+        return coefficients, torch.cat((keys.double(), totals.reshape(-1), terms.reshape(-1), extrema.double().reshape(-1)))
     terms = torch.zeros((4, n), dtype=torch.float64, device=sources[0].device)
     by_rank: dict = {}
     for index, rank in enumerate(ranks):
-        by_rank.setdefault(rank, []).append(index)
+        if rank > fit_kernels.CHOLESKY_MAX_K:
+            by_rank.setdefault(rank, []).append(index)
+    if small:
+        values = fit_kernels.span_terms([rows[i] for i in small], [ranks[i] for i in small], [coefficients[i] for i in small])
+        index = torch.tensor(small, dtype=torch.long).pin_memory().to(terms.device, non_blocking=True)
+        terms[:, index] = values[:, :4].T
     for members in by_rank.values():
         values = _rank_terms([coefficients[i] for i in members], [rows[i] for i in members])
         # Consecutive members (one rank: the usual case) take a slice; others an index tensor

@@ -309,6 +309,50 @@ def cholesky_inverse(gram: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     return inverse, info
 
 
+_SPAN_SPLITS = 64  # RCH_SPAN_SPLITS
+
+
+def span_terms(bases, ranks, coefficients=None) -> torch.Tensor:
+    """float64 ``[n, 6]`` of FP16 basis views ``Q = basis[:rank]`` (rank <= :data:`CHOLESKY_MAX_K`), with
+    ``G = Q Q^T`` in FP64: ``trace(G^-1 P^T P)`` (0 without ``coefficients``), the Cholesky status of G
+    (0 or the failing order), ``||G - I||_inf``, ``max |G_ii|``, ``||G||_inf`` and ``||G^-1||_inf``."""
+    device = _device(bases)
+    ranks = [int(rank) for rank in ranks]
+    if len(ranks) != len(bases) or not all(1 <= r <= min(CHOLESKY_MAX_K, b.shape[0]) for r, b in zip(ranks, bases)):
+        raise ConfigurationError(f"span terms take one rank per basis, at most {CHOLESKY_MAX_K} and its rows")
+    channels = {int(b.shape[1]) for b in bases}
+    if len(channels) != 1:
+        raise ConfigurationError("one fit batch must share the channel count")
+    c8, n = padded(channels.pop()), len(bases)
+    keep, table = [], _table(n)
+    rows = [_basis_rows(basis, rank, c8, keep) for basis, rank in zip(bases, ranks)]
+    table["basis_ptr"], table["basis_stride"] = [a for a, _ in rows], [stride for _, stride in rows]
+    table["rank"] = ranks
+    orders = [-(-rank // 16) * 16 for rank in ranks]
+    firsts = np.concatenate(([0], np.cumsum([2 * k * k for k in orders])))
+    total = int(firsts[-1])
+    # Scratch (G and G^-1 of every matrix, the trace's partial sums) and the terms in one allocation.
+    work = torch.empty(total + n * (_SPAN_SPLITS + 6), dtype=torch.float64, device=device)
+    table["gram_ptr"] = work.data_ptr() + 8 * firsts[:-1]
+    table["partial_ptr"] = work.data_ptr() + 8 * (total + _SPAN_SPLITS * np.arange(n))
+    terms = work[total + n * _SPAN_SPLITS:].view(n, 6)
+    table["energy_ptr"] = terms.data_ptr() + 48 * np.arange(n)
+    max_rows = 0
+    if coefficients is not None:
+        if len(coefficients) != n or any(p.dtype != torch.float32 or p.ndim != 2 or p.shape[1] != rank or p.stride(1) != 1
+                                         for p, rank in zip(coefficients, ranks)):
+            raise ConfigurationError("span terms take fp32 [rows, rank] coefficients with unit column stride")
+        table["rows"] = [p.shape[0] for p in coefficients]
+        table["coef_ptr"] = [p.data_ptr() for p in coefficients]
+        table["coef_stride"] = [p.stride(0) for p in coefficients]
+        max_rows = max(int(p.shape[0]) for p in coefficients)
+    descriptors = _upload(table, device)
+    _lib.call("rch_fit_span", descriptors.data_ptr(), n, c8, max_rows, max(ranks), int(coefficients is not None),
+              _stream(device))
+    del keep
+    return terms
+
+
 def gaussian(blocks) -> None:
     """Fill each ``(view, seed)`` of ``blocks`` with seeded standard normals in one launch: ``view``
     an fp32 ``[rows, cols]`` device tensor with unit column stride (e.g. the trailing columns of a

@@ -365,3 +365,99 @@ def test_absmax_flags_nonfinite_values(device, dtype):
     keys = fk.absmax([values] + bad + [torch.zeros_like(values)]).cpu().numpy()
     assert keys[0] == np.float32(3.5).view(np.int32) and keys[-1] == 0
     assert (keys[1:-1] >= fk.NONFINITE_BITS).all()
+
+
+@pytest.mark.parametrize("channels,rows,ranks", [(136, 500, [1, 15, 16, 17, 33, 64, 65, 127, 128]), (40, 1, [3]),
+                                                 (1536, 33, [32, 96]), (264, 4680, [128])])
+def test_span_terms_match_fp64(device, channels, rows, ranks):
+    """Span trace, Cholesky status and norms of a ragged batch of basis views against numpy in FP64
+    (relative 1e-11: the condition of these rows is below 4), and without coefficients."""
+    rng = np.random.default_rng(97)
+    bases, coefficients = [], []
+    for rank in ranks:
+        q, _ = np.linalg.qr(rng.standard_normal((channels, rank)))
+        bases.append(torch.from_numpy((q * rng.uniform(0.7, 1.3, rank)).T.copy()).to(torch.float16).to(device))
+        padded = torch.zeros((rows, -(-rank // 4) * 4), device=device)
+        padded[:, :rank] = torch.from_numpy(rng.standard_normal((rows, rank)).astype(np.float32)).to(device)
+        coefficients.append(padded[:, :rank])
+    terms = fk.span_terms(bases, ranks, coefficients).cpu().numpy()
+    plain = fk.span_terms(bases, ranks).cpu().numpy()
+    assert (plain[:, 0] == 0).all() and np.array_equal(plain[:, 1:], terms[:, 1:])
+    for basis, p, row in zip(bases, coefficients, terms):
+        q, c = basis.double().cpu().numpy(), p.double().cpu().numpy()
+        gram = q @ q.T
+        inverse = np.linalg.inv(gram)
+        want = [np.trace(inverse @ (c.T @ c)), 0.0, np.abs(gram - np.eye(len(q))).sum(1).max(), np.abs(np.diag(gram)).max(),
+                np.abs(gram).sum(1).max(), np.abs(inverse).sum(1).max()]
+        np.testing.assert_allclose(row, want, rtol=1e-11)
+
+
+def test_span_terms_flag_singular_views(device):
+    """A repeated row is not positive definite at its order (the exact FP64 factor's pivot is zero or
+    negative); a NaN at the first; the other views of the batch are unaffected."""
+    rng = np.random.default_rng(98)
+    q, _ = np.linalg.qr(rng.standard_normal((64, 20)))
+    good = torch.from_numpy(q.T.copy()).to(torch.float16).to(device)
+    zero = good.clone()
+    zero[17] = 0.0
+    nan = good.clone()
+    nan[0, 5] = float("nan")
+    terms = fk.span_terms([zero, good, nan], [20, 20, 20]).cpu().numpy()
+    assert terms[:, 1].tolist() == [18.0, 0.0, 1.0]
+    assert np.isinf(terms[0, 5]) and np.isinf(terms[2, 5]) and np.isfinite(terms[1]).all()
+
+
+def test_projection_reports_its_first_fault(device):
+    """project_onto_basis checks the basis before the matrix: a basis that is not finite (also past
+    the rank, also with a bad argument), a singular one, an ill-conditioned one, then the matrix."""
+    from reelcache_amd import factorization as fa
+    from reelcache_amd.errors import ConfigurationError
+
+    rng = np.random.default_rng(99)
+    x, _ = _source(rng, 100, 64, "bfloat16", device)
+    q, _ = np.linalg.qr(rng.standard_normal((64, 12)))
+    basis = torch.from_numpy(q.T.copy()).to(torch.float16).to(device)
+    projection = fa.project_onto_basis(x, basis, rank=10)
+    gram = basis[:10].double().cpu().numpy() @ basis[:10].double().cpu().numpy().T
+    want = np.abs(gram).sum(1).max() * np.abs(np.linalg.inv(gram)).sum(1).max()
+    assert projection.condition_bound == pytest.approx(want, rel=1e-12)
+    assert fa.basis_condition_bound(basis[:10]) == projection.condition_bound
+    bad = basis.clone()
+    bad[11, 3] = float("inf")
+    for arguments in ({"rank": 10}, {"rank": 99}):
+        with pytest.raises(ConfigurationError, match="stored basis must be finite"):
+            fa.project_onto_basis(x, bad, **arguments)
+    with pytest.raises(ConfigurationError, match="rank"):
+        fa.project_onto_basis(x, basis, rank=13)
+    singular = basis.clone()
+    singular[4] = 0.0
+    with pytest.raises(ConfigurationError, match="singular or ill-conditioned"):
+        fa.project_onto_basis(x, singular)
+    with pytest.raises(ConfigurationError, match="singular or ill-conditioned"):
+        fa.project_onto_basis(x, basis, max_condition=1.0)
+    infinite = x.clone()
+    infinite[99, 63] = float("inf")
+    with pytest.raises(ConfigurationError, match="nonempty finite"):
+        fa.project_onto_basis(infinite, basis)
+    with pytest.raises(ConfigurationError, match="singular or ill-conditioned"):
+        fa.project_onto_basis(infinite, singular)
+
+
+@pytest.mark.parametrize("rows,cols,stride", [(1, 1, 1), (17, 3, 5), (64, 96, 96), (65, 130, 132), (130, 63, 64)])
+def test_extrema_and_codes_at_tile_edges(device, rows, cols, stride):
+    """Column extrema and codes of strided matrices around the kernels' row tiles, column lanes and
+    four-column groups: exact extrema, codes equal to the oracle's, also through the batched launch."""
+    rng = np.random.default_rng(101)
+    storage = torch.from_numpy(rng.standard_normal((rows, stride)).astype(np.float32)).to(device)
+    values = storage[:, :cols]
+    host = values.cpu().numpy()
+    low, high = fk.split_keys(fk.column_extrema(values).cpu().numpy(), cols)
+    np.testing.assert_array_equal(low, host.min(0))
+    np.testing.assert_array_equal(high, host.max(0))
+    affine = np.asarray(oq.covering_affine(low, high), dtype=np.float64)
+    affine[0, 0] = 0.0  # a zero scale gives code 0
+    want = oq.quantize_with_affine(host, affine[0], affine[1])
+    scale, offset = (torch.from_numpy(v.copy()).to(device) for v in affine)
+    np.testing.assert_array_equal(fk.quantize(values, scale, offset).cpu().numpy(), want)
+    for codes in fk.quantize_batched([values, values], [affine, affine]):
+        np.testing.assert_array_equal(codes.cpu().numpy(), want)
