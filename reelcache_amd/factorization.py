@@ -21,6 +21,7 @@ import time
 from dataclasses import dataclass, field
 from typing import Any
 
+import numpy as np
 import torch
 
 from . import fit_kernels
@@ -115,13 +116,18 @@ def validate_rank(rank: int, shape: tuple[int, int]) -> int:
     return rank
 
 
-def validate_stored_basis(basis: torch.Tensor, channels: int) -> torch.Tensor:
+def _check_stored_basis(basis, channels: int) -> None:
+    """The checks of :func:`validate_stored_basis` that read no value."""
     if not isinstance(basis, torch.Tensor) or basis.layout != torch.strided:
         raise ConfigurationError("reuse basis must be a dense torch.Tensor")
     if basis.device.type == "meta" or basis.dtype != torch.float16:
         raise ConfigurationError("reuse basis must be the actual stored FP16 basis")
     if basis.ndim != 2 or basis.shape[1] != channels or not 1 <= basis.shape[0] <= channels:
         raise ConfigurationError("stored basis must have shape [canonical_rank, channels]")
+
+
+def validate_stored_basis(basis: torch.Tensor, channels: int) -> torch.Tensor:
+    _check_stored_basis(basis, channels)
     if not bool(torch.isfinite(basis).all()):
         raise ConfigurationError("stored basis must be finite")
     return basis.detach()
@@ -137,7 +143,11 @@ def _canonical_signs(basis: torch.Tensor) -> torch.Tensor:
 @torch.no_grad()
 def basis_condition_bound(basis: torch.Tensor) -> float:
     """Infinity-norm condition bound ||G|| ||G^-1|| of G = B B^T in FP64 via Cholesky
-    (inf for a singular basis)."""
+    (inf for a singular basis).  FP16 rows on a GPU, up to the native kernels' order, take one native
+    call and one read; others the library's factorization."""
+    if (basis.device.type == "cuda" and basis.dtype == torch.float16 and basis.ndim == 2
+            and 1 <= basis.shape[0] <= fit_kernels.CHOLESKY_MAX_K and basis.shape[1] >= 1):
+        return _terms_condition(fit_kernels.span_terms([basis], [int(basis.shape[0])])[0].tolist())
     rounded = basis.to(dtype=torch.float64)
     gram = rounded @ rounded.T
     factor, info = torch.linalg.cholesky_ex(gram, check_errors=False)
@@ -145,6 +155,12 @@ def basis_condition_bound(basis: torch.Tensor) -> float:
         return math.inf
     inverse = torch.cholesky_inverse(factor)
     condition = float((gram.abs().sum(1).max() * inverse.abs().sum(1).max()).item())
+    return condition if math.isfinite(condition) else math.inf
+
+
+def _terms_condition(terms) -> float:
+    """:func:`basis_condition_bound` from one host row of ``fit_kernels.span_terms``."""
+    condition = terms[4] * terms[5] if terms[1] == 0 else math.inf
     return condition if math.isfinite(condition) else math.inf
 
 
@@ -181,38 +197,64 @@ def _check_projection_input(tensor) -> None:
 def project_onto_basis(tensor: torch.Tensor, basis: torch.Tensor, *, rank: int | None = None, tile_rows: int = 1024,
                        max_condition: float = 1e6, _condition_bound: float | None = None,
                        _work: dict | None = None) -> Projection:
-    """Project once onto the stored FP16 basis and measure the direct residual in FP64."""
+    """Project once onto the stored FP16 basis and measure the direct residual in FP64.
+
+    Everything is enqueued before the one host read: the finite scans of the basis and of the matrix
+    (absmax keys), the condition terms, the projection with its column extrema and the energies.  The
+    checks then run on the host values in their order (basis, condition, matrix, overflow, energies)."""
     started = time.perf_counter()
     _check_projection_input(tensor)
-    stored = validate_stored_basis(basis, tensor.shape[1])
+    _check_stored_basis(basis, tensor.shape[1])
+    stored = basis.detach()
     rank = stored.shape[0] if rank is None else rank
-    validate_rank(rank, tuple(tensor.shape))
-    if rank > stored.shape[0]:
-        raise ConfigurationError("requested rank exceeds the immutable stored basis")
-    if type(tile_rows) is not int or tile_rows < 1:
-        raise ConfigurationError("tile_rows must be a positive integer")
-    if (isinstance(max_condition, bool) or not isinstance(max_condition, (int, float))
-            or not math.isfinite(max_condition) or max_condition < 1):
-        raise ConfigurationError("max_condition must be finite and at least one")
+    try:
+        validate_rank(rank, tuple(tensor.shape))
+        if rank > stored.shape[0]:
+            raise ConfigurationError("requested rank exceeds the immutable stored basis")
+        if type(tile_rows) is not int or tile_rows < 1:
+            raise ConfigurationError("tile_rows must be a positive integer")
+        if (isinstance(max_condition, bool) or not isinstance(max_condition, (int, float))
+                or not math.isfinite(max_condition) or max_condition < 1):
+            raise ConfigurationError("max_condition must be finite and at least one")
+    except ConfigurationError:
+        validate_stored_basis(basis, tensor.shape[1])  # a basis that is not finite is reported first
+        raise
     view = stored[:rank].to(device=tensor.device)
     condition_started = time.perf_counter()
-    condition = basis_condition_bound(view) if _condition_bound is None else _condition_bound
+    condition, terms, basis_keys = _condition_bound, None, None
+    if condition is None and rank <= fit_kernels.CHOLESKY_MAX_K and stored.device == tensor.device:
+        basis_keys = fit_kernels.absmax([stored])
+        terms = fit_kernels.span_terms([view], [rank])
+    else:
+        validate_stored_basis(basis, tensor.shape[1])
+        if condition is None:
+            condition = basis_condition_bound(view)
+        _check_condition(condition, max_condition)
     condition_seconds = time.perf_counter() - condition_started
-    if not math.isfinite(condition) or condition > max_condition:
-        raise ConfigurationError("stored basis is singular or ill-conditioned")
     coefficient_started = time.perf_counter()
     keys = fit_kernels.absmax([tensor])
     (coefficients,), extrema = fit_kernels.project([tensor], [view], [rank], extrema=True)
     totals = fit_kernels.energies([tensor], keys, bases=[view], ranks=[rank], coefficients=[coefficients])
-    bits, low, high = _read_scalars(keys, extrema, rank)
+    parts = [keys.double(), extrema.double().view(-1), totals.view(-1)]
+    if terms is not None:
+        parts += [basis_keys.double(), terms.view(-1)]
+    host = torch.cat(parts).cpu().numpy()
+    bits = int(host[0])
+    low, high = fit_kernels.split_keys(host[1:1 + 2 * rank].astype(np.int64).astype(np.int32), rank)
+    low, high = float(low.min()), float(high.max())
+    source_squared, error_squared = (float(v) for v in host[1 + 2 * rank:3 + 2 * rank])
+    if terms is not None:
+        if int(host[3 + 2 * rank]) >= fit_kernels.NONFINITE_BITS:
+            raise ConfigurationError("stored basis must be finite")
+        condition = _terms_condition([float(v) for v in host[4 + 2 * rank:]])
+        _check_condition(condition, max_condition)
     coefficient_seconds = time.perf_counter() - coefficient_started
     if bits >= fit_kernels.NONFINITE_BITS:
         raise ConfigurationError("projection requires a nonempty finite FP32-compatible matrix")
     if not (math.isfinite(low) and math.isfinite(high)):
         raise ConfigurationError("projection overflowed FP32")
     guard_started = time.perf_counter()
-    source_squared, error_squared = (float(v) for v in totals[0].cpu())
-    scale = float(torch.tensor(bits, dtype=torch.int32).view(torch.float32))
+    scale = float(np.array([bits], dtype=np.int32).view(np.float32)[0])
     if not math.isfinite(source_squared) or not math.isfinite(error_squared):
         raise ConfigurationError("nonfinite direct residual energy")
     zero = scale == 0.0
@@ -228,11 +270,9 @@ def project_onto_basis(tensor: torch.Tensor, basis: torch.Tensor, *, rank: int |
     )
 
 
-def _read_scalars(keys: torch.Tensor, extrema: torch.Tensor, rank: int) -> tuple[int, float, float]:
-    """One device->host read: (absmax bits, min of P, max of P)."""
-    host = torch.cat((keys.view(-1), extrema.view(-1))).cpu().numpy()
-    low, high = fit_kernels.split_keys(host[1:], rank)
-    return int(host[0]), float(low.min()), float(high.max())
+def _check_condition(condition: float, max_condition: float) -> None:
+    if not math.isfinite(condition) or condition > max_condition:
+        raise ConfigurationError("stored basis is singular or ill-conditioned")
 
 
 @torch.no_grad()

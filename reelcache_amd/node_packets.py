@@ -161,9 +161,9 @@ def _codes(coefficients: torch.Tensor, low: np.ndarray, high: np.ndarray, spec):
     layout = normalization_layout(rank, spec.normalization, spec.protected_fraction)
     affine = affine_from_extrema(low, high, layout)
     scale, offset = expanded_affine(affine, layout, rank)
-    device = coefficients.device
-    scale64 = torch.from_numpy(np.ascontiguousarray(scale, dtype=np.float64)).to(device)
-    offset64 = torch.from_numpy(np.ascontiguousarray(offset, dtype=np.float64)).to(device)
+    # One copy from pinned memory without a host wait (a pageable one drains the stream first).
+    both = torch.from_numpy(np.stack((np.asarray(scale, np.float64), np.asarray(offset, np.float64)))).pin_memory()
+    scale64, offset64 = both.to(coefficients.device, non_blocking=True)
     values = coefficients if coefficients.stride(1) == 1 else coefficients.contiguous()
     pixels = fit_kernels.quantize(values, scale64, offset64)
     return pixels, affine.astype("<f4", copy=False), layout
