@@ -20,7 +20,7 @@
 extern "C" {
 #endif
 
-#define RCH_ABI_VERSION 15
+#define RCH_ABI_VERSION 16
 
 /* Status codes (mapped to reelcache errors by the host). */
 #define RCH_OK 0
@@ -279,6 +279,41 @@ int rch_restore_noalloc(const rch_pack* packs_host, int n_packs, const rch_job* 
                         const int32_t* tiles_dev, int n_tiles, const int32_t* bounds_dev, int grid, int channels,
                         int head_dim, int source_kind, int out_dtype, int precision, int max_ksteps, int group_flags,
                         void* stream);
+
+/*
+ * A whole restore call from a prepared program: the call buffer's host image is filled (template, job and
+ * pack rows, affine blocks, picture offsets), copied to the device buffer on `stream` (hipMemcpyAsync;
+ * `image` must be pinned and stay untouched until the copy has run) and the program's launches follow in
+ * order on the same stream.  The program (host memory, read only) depends on the call's geometry alone;
+ * addresses and affine values come with each call.
+ *   jobs      int64 [n_jobs, RCH_CALL_JOB_WORDS]: dst, src, basis, RoPE cos, sin, pairs (0: none), host
+ *             address of the fp32 affine block (scale | offset) and its floats (0: none), coef_exp,
+ *             picture count.
+ *   pictures  int64: the picture addresses of the jobs that have any, in job order.
+ * Replaces one launch sequence's separate entries; no counterpart in the reference.
+ */
+#define RCH_CALL_JOB_WORDS 10
+#define RCH_CALL_LAUNCH_WORDS 12
+#define RCH_CALL_PACK 0    /* max_nblocks, max_ksteps */
+#define RCH_CALL_UNPACK 1  /* tiles offset, n_tiles, max_rank */
+#define RCH_CALL_DENSE 2   /* tiles offset, n_tiles, channels, head_dim, out_dtype */
+#define RCH_CALL_RESTORE 3 /* tiles offset, n_tiles, bounds offset, grid, channels, head_dim, source kind, out_dtype, ksteps, flags */
+#define RCH_CALL_PAIR 4    /* tiles offset, n_tiles0, n_tiles1, bounds offset, grid, channels, head_dim, source kind, out_dtype,
+                              ksteps0, ksteps1 */
+typedef struct rch_call {
+    int64_t template_ptr, image_bytes;   /* host image of the tables, and its size */
+    int64_t n_jobs, n_rows, desc_offset; /* job rows, then unpack rows, at desc_offset of the image */
+    int64_t rows_ptr, relative_ptr;      /* host int64 [n_rows, 40]: row values; 1 where the buffer base is added */
+    int64_t unpacked_ptr;                /* host int64 [n_rows - n_jobs]: job of each unpack row */
+    int64_t n_packs, packs_offset, packs_ptr, packs_relative_ptr, members_ptr; /* as rows; job of each pack */
+    int64_t scratch_offset;              /* exponent words, in the device buffer */
+    int64_t prescaled;                   /* nonzero: write coef_exp (fp16 modes) */
+    int64_t precision;
+    int64_t n_launches, launches_ptr;    /* host int64 [n_launches, RCH_CALL_LAUNCH_WORDS]: RCH_CALL_*, arguments */
+} rch_call;
+
+int rch_call_size(void);
+int rch_call_run(const rch_call* call, void* image, void* buffer, const int64_t* jobs, const int64_t* pictures, void* stream);
 
 /*
  * Dense rows -> RoPE -> cast -> native store (DenseSource jobs).

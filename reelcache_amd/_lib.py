@@ -16,7 +16,7 @@ import numpy as np
 from .errors import ConfigurationError, UnsupportedError
 
 LIBRARY = Path(__file__).resolve().with_name("libreelcache_hip.so")
-ABI_VERSION = 15
+ABI_VERSION = 16
 
 # Status codes (RCH_E_*).
 OK, E_CONFIG, E_UNSUPPORTED, E_LAUNCH = 0, 1, 2, 3
@@ -57,6 +57,12 @@ FIT_FIELDS = ("src_ptr", "src_dtype", "rows", "src_stride", "basis_ptr", "basis_
               "coef_stride", "gram_ptr", "gram_stride", "absmax_ptr", "extrema_ptr", "energy_ptr", "partial_ptr",
               "resid_ptr")
 FIT_DTYPE = np.dtype([(name, "<i8") for name in FIT_FIELDS])
+# rch_call field order; words per job and per launch record, launch kinds (RCH_CALL_*).
+CALL_FIELDS = ("template_ptr", "image_bytes", "n_jobs", "n_rows", "desc_offset", "rows_ptr", "relative_ptr",
+               "unpacked_ptr", "n_packs", "packs_offset", "packs_ptr", "packs_relative_ptr", "members_ptr",
+               "scratch_offset", "prescaled", "precision", "n_launches", "launches_ptr")
+CALL_LAUNCH_WORDS = 12
+CALL_PACK, CALL_UNPACK, CALL_DENSE, CALL_RESTORE, CALL_PAIR = 0, 1, 2, 3, 4
 QUANTIZE_FIELDS = ("values_ptr", "rows", "cols", "stride", "affine_ptr", "codes_ptr", "code_stride", "reserved")
 QUANTIZE_DTYPE = np.dtype([(name, "<i8") for name in QUANTIZE_FIELDS])
 GAUSS_FIELDS = ("dst_ptr", "rows", "cols", "stride", "seed", "reserved0", "reserved1", "reserved2")
@@ -76,6 +82,8 @@ _SIGNATURES = {
     "rch_restore_occupancy": ([_i, _i, _i, _i, _i, _i, ctypes.POINTER(_i)], _i),
     "rch_restore_pair": ([_p, _i, _p, _i, _i, _p, _i, _i, _i, _i, _i, _i, _i, _i, _p, _p], _i),
     "rch_restore_pair_occupancy": ([_i, _i, _i, _i, _i, _i, ctypes.POINTER(_i)], _i),
+    "rch_call_size": ([], _i),
+    "rch_call_run": ([_p, _p, _p, _p, _p, _p], _i),
     "rch_rope_store": ([_p, _i, _p, _i, _i, _i, _i, _p], _i),
     "rch_staged_unpack": ([_p, _i, _p, _i, _p, _p, _i64, _i, _i, _i, _i, _p, _p], _i),
     "rch_staged_store": ([_p, _i, _p, _i, _p, _p, _i64, _i, _i, _i, _i, _p, _p], _i),
@@ -120,7 +128,7 @@ def _load():
     if lib.rch_abi_version() != ABI_VERSION:
         raise UnsupportedError(f"{LIBRARY.name} has ABI {lib.rch_abi_version()}, expected {ABI_VERSION}; rebuild it")
     if (lib.rch_job_size() != JOB_DTYPE.itemsize or lib.rch_pack_size() != PACK_DTYPE.itemsize
-            or lib.rch_fit_matrix_size() != FIT_DTYPE.itemsize):
+            or lib.rch_fit_matrix_size() != FIT_DTYPE.itemsize or lib.rch_call_size() != 8 * len(CALL_FIELDS)):
         raise UnsupportedError(f"{LIBRARY.name} descriptor layout differs from this package; rebuild it")
     return lib
 

@@ -155,6 +155,18 @@ def _on(stream):
     return torch.cuda.stream(stream) if stream is not None else contextlib.nullcontext()
 
 
+_NULL = contextlib.nullcontext()
+
+
+def _entered(stream):
+    """A context in which ``stream`` is current: nothing to enter when it is already (the usual case;
+    entering and leaving a stream context costs as much as a launch)."""
+    device = stream.device
+    if torch.cuda.current_device() == device.index and torch.cuda.current_stream(device) == stream:
+        return _NULL
+    return torch.cuda.stream(stream)
+
+
 def _execution_stream(device, stream, wait_events):
     """The stream a call runs on (``None`` for host execution), after ``wait_events``."""
     if device.type != "cuda":
@@ -268,7 +280,7 @@ def reconstruct(jobs, *, backend="auto", precision="auto", stream=None, wait_eve
         native = [job for job in jobs if native_rope is not None and job.rope is not None]
         fused = [job for job in jobs if native_rope is None or job.rope is None]
         try:
-            with torch.cuda.stream(stream):
+            with _entered(stream):
                 if fused:
                     call.launch(fused)
                 if native:

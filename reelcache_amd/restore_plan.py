@@ -14,13 +14,16 @@ many layers of one model):
   the byte layout of the call buffer, memoized by the call's geometry (the jobs' static rows,
   alignment bits, and which jobs share a destination view, a basis or a RoPE table);
 * :func:`run_call` -- per call: read the addresses, copy the layout's template bytes into
-  pinned staging, write the pointer columns, affine tables and prescale exponents, upload, launch.
+  pinned staging, write the pointer columns, affine tables and prescale exponents, upload, launch:
+  in one native entry (``rch_call_run``), or here with one entry per launch where the host acts
+  between launches (stage events, staged and scratch-free calls, device coefficient bounds).
 """
 
 from __future__ import annotations
 
 import math
 import threading
+from array import array
 
 import numpy as np
 import torch
@@ -271,8 +274,8 @@ class _JobDesc:
     of a call's geometry key.  Addresses (destination, source, basis, tables) are read from the
     referenced tensors at every call."""
 
-    __slots__ = ("affine", "basis", "basis_key", "channels", "dst", "dst_shift", "dst_vec_rule", "dtype",
-                 "exponent", "grid", "head_dim", "host_bound", "key", "key_id", "kind", "out_dtype", "pictures",
+    __slots__ = ("affine", "affine_address", "affine_size", "basis", "basis_key", "channels", "dst", "dst_shift",
+                 "dst_vec_rule", "dtype", "exponent", "grid", "head_dim", "host_bound", "key", "key_id", "kind", "out_dtype", "pictures",
                  "rank", "rope_kind", "row", "section_pairs", "src", "src_vec_rule", "table", "tokens", "pic_vec_rule")
 
     def __init__(self, job):
@@ -297,6 +300,12 @@ class _JobDesc:
             row[_C_SRC_ROW], row[_C_SRC_COL] = self.src.stride()
         else:
             self._factorized(row, job, source)
+        if self.host_bound is not None:
+            with np.errstate(over="ignore"):  # a bound beyond fp32 concerns the fp16 modes only
+                self.exponent = _prescale_exponent(self.host_bound)
+        self.affine_address = self.affine_size = 0
+        if self.affine is not None:
+            self.affine_address, self.affine_size = self.affine.ctypes.data, self.affine.size
         self.row = row
         pictures = None if self.pictures is None else (len(source.pictures), len(source.pictures[0]))
         self.key = (row.tobytes(), self.kind, self.dtype, self.out_dtype, self.head_dim, self.channels, self.rope_kind,
@@ -369,13 +378,8 @@ class _JobDesc:
     def _affine(self, scale, offset):
         """The job's fp32 (scale | offset) block and the fp16 modes' prescale exponent of its
         coefficient bound max(|offset|, |255 * scale + offset|) (the affine arrays are read-only copies)."""
-        self.affine = np.concatenate((scale, offset)).astype(np.float32, copy=False)
+        self.affine = np.ascontiguousarray(np.concatenate((scale, offset)), dtype=np.float32)
         self.exponent = _prescale_exponent(_coefficient_bound(scale, offset))
-
-    def source_address(self):
-        if self.pictures is None:
-            return self.src.data_ptr()
-        return min(picture.data_ptr() for picture in self.pictures)
 
 
 # Distinct job geometries (descriptor keys) seen by this process, numbered for cheap call keys.
@@ -407,6 +411,8 @@ def _rank_steps_class(precision, rank):
 # ---------------------------------------------------------------------------
 # Call layouts
 # ---------------------------------------------------------------------------
+
+_NO_TABLE = (0, 0, 0)
 
 # Columns that hold an offset into the call buffer in a layout's rows; the base is added per call.
 _BASE_RELATIVE_PACK = ("dst_ptr", "exp_ptr", "scale_ptr", "offset_ptr")
@@ -484,7 +490,73 @@ class _Layout:
             # The restore reads the rows the unpack row writes.
             rows[index, _C_SRC_PTR] = rows[len(descs) + position, _C_DST_PTR] = self.codes_offset + at
         self.table_jobs = [i for i, d in enumerate(descs) if d.table is not None]
+        self.picture_jobs = [i for i, d in enumerate(descs) if d.pictures is not None]
+        self._call_program(len(descs))
         self.host_bound_jobs = [i for i, d in enumerate(descs) if self.fp16_mode and d.host_bound is not None]
+
+    def _call_program(self, count):
+        """The native call program (``rch_call_run``) of this geometry, or None for calls that need the
+        host between launches: staged and static-scratch calls, device coefficient bounds."""
+        self.program = None
+        if self.staged or self.static or self.bound_jobs:
+            return
+        launches = []
+        if len(self.pack_rows):
+            launches.append((_lib.CALL_PACK, int(self.pack_rows[:, _PACK_COLUMN["nblocks"]].max()),
+                             int(self.pack_rows[:, _PACK_COLUMN["ksteps"]].max())))
+        if self.unpacked:
+            launches.append((_lib.CALL_UNPACK, *self.unpack_tiles, self.unpack_rank))
+        for plan in self.plans:
+            if plan["variant"] == "dense":
+                kind, names = _lib.CALL_DENSE, ("tiles", "n_tiles", "channels", "head_dim", "out_dtype")
+            elif plan["variant"] == "pair":
+                kind, names = _lib.CALL_PAIR, ("tiles", "n_tiles0", "n_tiles1", "bounds", "grid", "channels", "head_dim",
+                                               "kind", "out_dtype", "ksteps0", "ksteps1")
+            else:
+                kind, names = _lib.CALL_RESTORE, ("tiles", "n_tiles", "bounds", "grid", "channels", "head_dim", "kind",
+                                                  "out_dtype", "max_ksteps", "flags")
+            launches.append((kind, *(plan[name] for name in names)))
+        table = np.zeros((len(launches), _lib.CALL_LAUNCH_WORDS), dtype=np.int64)
+        for row, launch in zip(table, launches):
+            row[:len(launch)] = launch
+        arrays = {"template": self.template, "rows": np.ascontiguousarray(self.rows),
+                  "relative": np.ascontiguousarray(self.rows_relative),
+                  "unpacked": np.array([index for index, _ in self.unpacked] or [0], dtype=np.int64),
+                  "packs": np.ascontiguousarray(self.pack_rows),
+                  "packs_relative": np.ascontiguousarray(self.pack_relative),
+                  "members": np.array(self.pack_sources or [0], dtype=np.int64), "launches": table}
+        fields = {name + "_ptr": value.ctypes.data for name, value in arrays.items()}
+        fields.update(image_bytes=self.template.size, n_jobs=count, n_rows=len(self.rows), desc_offset=self.desc_offset,
+                      n_packs=len(self.pack_rows), packs_offset=self.packs_offset or 0,
+                      scratch_offset=self.arena_bytes + self.pack_total, prescaled=int(self.fp16_mode),
+                      precision=self.code, n_launches=len(launches))
+        self.program_arrays = arrays  # referenced by the program's addresses
+        self.program = np.array([fields[name] for name in _lib.CALL_FIELDS], dtype=np.int64)
+        self.program_launches = len(launches)
+
+    def run_program(self, descs, dst, src, bases, pictures, device, stream, keepalive):
+        """Fill, upload and launch one call through the native program."""
+        buffer = torch.empty(self.buffer_bytes, dtype=torch.uint8, device=device)
+        host = _pinned_host(self.template.size)
+        tables: dict = {}
+        words = []
+        for index, desc in enumerate(descs):
+            entry = _NO_TABLE
+            table = desc.table
+            if table is not None:
+                entry = tables.get(id(table))
+                if entry is None:
+                    block = table._kernel_block(device, stream)
+                    entry = tables[id(table)] = (block.cos.data_ptr(), block.sin.data_ptr(), block.pairs.data_ptr())
+                    keepalive.append(block.block)
+            words += (dst[index], src[index], bases[index], *entry, desc.affine_address, desc.affine_size,
+                      desc.exponent, 0 if desc.pictures is None else len(desc.pictures))
+        words = array("q", words)
+        addresses = array("q", [address for index in self.picture_jobs for address in pictures[index]])
+        keepalive.extend((host, buffer))
+        _lib.call("rch_call_run", self.program.ctypes.data, host.data_ptr(), buffer.data_ptr(), words.buffer_info()[0],
+                  addresses.buffer_info()[0], stream.cuda_stream)
+        return self.program_launches
 
     def _unpack_layout(self, descs, kinds, rows, relative, arena):
         """Jobs whose codes are unpacked into aligned rows first (``rch_codes_unpack``): 16-bit modes'
@@ -832,7 +904,7 @@ class _Layout:
             if self.fp16_mode:
                 rows[self.affine_jobs, _C_COEF_EXP] = [descs[index].exponent for index in self.affine_jobs]
         for index in self.host_bound_jobs:
-            rows[index, _C_COEF_EXP] = _prescale_exponent(descs[index].host_bound)
+            rows[index, _C_COEF_EXP] = descs[index].exponent
         for index, at in self.picture_tables:
             pictures = descs[index].pictures
             offsets = np.fromiter((picture.data_ptr() for picture in pictures), dtype=np.int64, count=len(pictures))
@@ -1001,18 +1073,29 @@ def run_call(descs, device, stream, precision, config, keepalive, stage_events=N
     """Plan (or reuse the layout of) one HIP call and enqueue it on ``stream``; returns
     ``(launches, grids, variants)``.  ``staged``: the staged comparison path (unpack, library
     GEMM, store) for the factorized jobs instead of the fused kernels."""
-    dst = [desc.dst.data_ptr() + desc.dst_shift for desc in descs]
-    src = [desc.source_address() for desc in descs]
-    dynamic = [(_lib.JF_DST_VEC if desc.dst_vec_rule and not d & 15 else 0)
-               | (_lib.JF_SRC_VEC if desc.src_vec_rule and not s & 15 else 0)
-               | (_lib.JF_PIC_VEC4 if desc.pic_vec_rule and all(not p.data_ptr() & 3 for p in desc.pictures) else 0)
-               for desc, d, s in zip(descs, dst, src)]
-    bases, groups, first_of = [0] * len(descs), [None] * len(descs), {}
-    for index, desc in enumerate(descs):
+    dst, src, dynamic, bases, groups, first_of, pictures = [], [], [], [], [], {}, {}
+    for index, desc in enumerate(descs):  # every tensor's address read once
+        to = desc.dst.data_ptr() + desc.dst_shift
+        flags = _lib.JF_DST_VEC if desc.dst_vec_rule and not to & 15 else 0
+        if desc.pictures is None:
+            source = desc.src.data_ptr()
+            if desc.src_vec_rule and not source & 15:
+                flags |= _lib.JF_SRC_VEC
+        else:
+            addresses = pictures[index] = [picture.data_ptr() for picture in desc.pictures]
+            source = min(addresses)
+            if desc.pic_vec_rule and not any(address & 3 for address in addresses):
+                flags |= _lib.JF_PIC_VEC4
+        basis, group = 0, None
         if desc.basis is not None:
-            bases[index] = address = desc.basis.data_ptr()
-            groups[index] = first_of.setdefault((address, desc.basis_key), index)
-    key = (precision, _config_key(config), tuple(desc.key_id for desc in descs), tuple(dynamic), tuple(groups),
+            basis = desc.basis.data_ptr()
+            group = first_of.setdefault((basis, desc.basis_key), index)
+        dst.append(to)
+        src.append(source)
+        dynamic.append(flags)
+        bases.append(basis)
+        groups.append(group)
+    key = (precision, _config_key(config), tuple([desc.key_id for desc in descs]), tuple(dynamic), tuple(groups),
            staged)
     layout = _LAYOUTS.get(key)
     if layout is None:
@@ -1020,5 +1103,8 @@ def run_call(descs, device, stream, precision, config, keepalive, stage_events=N
         if len(_LAYOUTS) >= _LAYOUT_LIMIT:
             _LAYOUTS.clear()
         _LAYOUTS[key] = layout
-    launches = layout.enqueue(descs, dst, src, bases, device, stream, keepalive, stage_events)
+    if stage_events is None and layout.program is not None:
+        launches = layout.run_program(descs, dst, src, bases, pictures, device, stream, keepalive)
+    else:
+        launches = layout.enqueue(descs, dst, src, bases, device, stream, keepalive, stage_events)
     return launches, list(layout.grids), list(layout.variants)

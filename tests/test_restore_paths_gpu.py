@@ -288,3 +288,38 @@ def test_dense_rows_vector_and_element_paths_agree(device, heads, head_dim, layo
         np.testing.assert_array_equal(slots[0], slots[1])
         exact, bound = _rotation_bound(values.double().numpy(), heads, rope, out_dtype)
         assert float((np.abs(slots[0] - exact) - bound).max()) <= 0
+
+
+@pytest.mark.parametrize("precision", ["fp16x2", "bf16", "fp32"])
+def test_call_program_equals_separate_entries(device, precision):
+    """A call through the native call program (one entry) writes the same bits as the same call with
+    one entry per launch (stage events): rows, unaligned rows, pictures at low and high rank, float
+    sources (with a host bound in the fp16 modes) and dense rows, rotated and not, in one call; other
+    addresses on a second call of the same geometry."""
+    grid, heads, head_dim = (2, 6, 8), 4, 64
+    tokens = int(np.prod(grid))
+    shapes = [("uint8", 64, 64, "separable"), ("uint8", 33, 33, "none"), ("uint8", 201, 201, "none"),
+              ("pictures", 48, None, "separable"), ("pictures", 224, None, "none"), ("float", 40, None, "dense")]
+    for seed in (11, 12):
+        jobs = {}
+        for kind in ("program", "entries"):
+            rng = np.random.default_rng(seed)
+            cases = []
+            for source, rank, pitch, rope in shapes:
+                case = make_case(rng, grid=grid, heads=heads, head_dim=head_dim, rank=rank, source=source, rope=rope,
+                                 device=device, code_pitch=pitch, token_offset=2)
+                job = case.job
+                if source == "float":
+                    source_values = rk.CoefficientSource(job.source.values, bound=float(job.source.values.abs().max()))
+                    job = rk.ReconstructionJob(source_values, job.destination, job.grid, job.basis, job.rank, job.rope)
+                cases.append(job)
+            values = torch.from_numpy(rng.standard_normal((tokens, heads * head_dim)).astype(np.float32)).to(device)
+            cases.append(rk.ReconstructionJob(rk.DenseSource(values), rk.NativeView(
+                destination("BTHD", tokens, heads, head_dim, "bfloat16", device)), grid, rope=cases[0].rope))
+            jobs[kind] = cases
+        plain = rk.reconstruct(jobs["program"], precision=precision)
+        staged = rk.reconstruct(jobs["entries"], precision=precision, stage_events=[])
+        plain.release(), staged.release()
+        assert plain.stats["launches"] == staged.stats["launches"] and plain.stats["variants"] == staged.stats["variants"]
+        for a, b in zip(jobs["program"], jobs["entries"]):
+            assert torch.equal(a.destination.tensor, b.destination.tensor)
