@@ -20,7 +20,7 @@
 extern "C" {
 #endif
 
-#define RCH_ABI_VERSION 16
+#define RCH_ABI_VERSION 17
 
 /* Status codes (mapped to reelcache errors by the host). */
 #define RCH_OK 0
@@ -410,7 +410,7 @@ int rch_fit_gram(const rch_fit_matrix* mats_dev, int n_mats, int channels, int s
 int rch_fit_project(const rch_fit_matrix* mats_dev, int n_mats, int channels, int64_t max_rows, int max_rank,
                     int src_dtype, void* stream);
 
-#define RCH_RESIDUAL_SPLITS 4 /* most channel parts a 16-row partial is split into */
+#define RCH_RESIDUAL_SPLITS 8 /* most channel parts of a row tile, each with a partial of its own */
 /*
  * Direct residual and source energies of each matrix in FP64: sum (X / s)^2 and
  * sum ((X - P Q[:rank]) / s)^2 with s = max|X| read from *absmax_ptr (no scaling when s == 0),

@@ -1,8 +1,8 @@
 // One restore call from a prepared program: fills the call buffer's host image, uploads it and enqueues
 // the call's launches, so that a call whose geometry recurs costs one entry instead of a dozen array
 // operations and an entry per launch.  The host time of a call bounds restores below about 60 us of device
-// work: a K+V call of one 4680-token, 12-head chunk takes the host 40 us (67 with the rows filled by numpy
-// and every launch entered from Python), an eight-chunk history call 61 us (89).
+// work: a K+V call of one 390-token, 12-head chunk takes the host 40 us (67 with the rows filled by numpy
+// and every launch entered from Python), a seven-chunk history layer 61 us (89).
 #include <cstddef>
 #include <cstring>
 

@@ -15,6 +15,7 @@
 //     within ~1e-13 relative of a rounding boundary, i.e. independent of summation order.
 //   * Energies: FP64 sums of (x - r)^2 and x^2, divided by s^2 per partial (16 or 32 rows), fixed-order totals.
 //   * Quantizer: FP64 (v - offset) / scale, round half to even, clamp to [0, 255].
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -394,14 +395,17 @@ __global__ void __launch_bounds__(kGramThreads) gram_kernel(const rch_fit_matrix
 //
 // Bound by the FP64 matrix rate; the next step's loads are issued before a step's products and the
 // step body has no branch, so their latency is covered.  Two shapes (project_kernel's TB, SPLIT):
-//   * TB = 2, SPLIT = 1: a wave owns 32 tokens, so each converted basis operand feeds two products;
-//     workgroup = 128 tokens x 64 ranks.
+//   * TB = 2, SPLIT = 1: a wave owns 32 tokens; the four waves share a step's converted basis operands
+//     through LDS (two halves, one barrier a step), so a wave loads and converts a quarter of them and
+//     each feeds two of its products; workgroup = 128 tokens x 64 ranks.
 //   * TB = 1, SPLIT = 4: for batches that would leave CUs idle, the four waves of a workgroup share 16
 //     tokens and split the channel steps; the partial sums are added through LDS in wave order.
 // GRAM: the sources are the basis rows themselves and the FP64 sums are stored as they are, G = Q Q^T.
 // One bf16 matrix [4680, 1536] at rank 96: 105 us with 64-token workgroups of one wave per 16 tokens and
-// loads in the step, 36 us now; 60 matrices at rank 96: 1563 -> 1396 us (59 of the 68 TFLOP/s that a
-// large library FP64 product reaches on this card).
+// loads in the step, 36 us now; 60 matrices at rank 96: 1563 us, 1396 with every wave converting its own
+// basis operands, 1293-1329 now.  The vector instructions do not hide under FP64 products, and the rate
+// depends on the operands' bits: products of full 53-bit operands alone reach 46-49 TFLOP/s, a large
+// library product 68.
 // ---------------------------------------------------------------------------------------------
 
 // Eight consecutive source elements as loaded, and as doubles.
@@ -427,7 +431,7 @@ __device__ __forceinline__ int padded_order(int rank) { return (rank + 15) & ~15
 
 template <int DT, int TB, int SPLIT, int NB, bool GRAM = false>
 __device__ __forceinline__ void project_ranks(const rch_fit_matrix* M, int channels, int r0, int64_t wt, int wave, int lane,
-                                              double* partial) {
+                                              double* shared) {
     constexpr int E = esize<DT>();
     static_assert(!GRAM || (DT == RCH_DT_F16 && SPLIT > 1), "the basis Gram runs on fp16 rows, channels split");
     const int rank = static_cast<int>(M->rank);
@@ -445,56 +449,96 @@ __device__ __forceinline__ void project_ranks(const rch_fit_matrix* M, int chann
     for (int b = 0; b < NB; ++b)  // rows past the rank read zeros
         q_row[b] = r0 + 16 * b + i16 < rank ? static_cast<uint32_t>((r0 + 16 * b + i16) * M->basis_stride * 2) : kOutOfRange;
     Eight<DT> x_now[TB], x_next[TB];
-    Eight<RCH_DT_F16> q_now[NB], q_next[NB];
-    auto load = [&](int c0, Eight<DT> (&x)[TB], Eight<RCH_DT_F16> (&q)[NB]) __attribute__((always_inline)) {
+    auto load_x = [&](int c0) __attribute__((always_inline)) {
         const int c = c0 + 8 * g;  // channels % 8 == 0: a group is whole or past the end
         const uint32_t past = c < channels ? 0u : kOutOfRange;
 #pragma unroll
-        for (int t = 0; t < TB; ++t) x[t] = load_eight<DT>(xs, (x_row[t] + static_cast<uint32_t>(c * E)) | past);
-#pragma unroll
-        for (int b = 0; b < NB; ++b) q[b] = load_eight<RCH_DT_F16>(qs, (q_row[b] + static_cast<uint32_t>(c * 2)) | past);
+        for (int t = 0; t < TB; ++t) x_next[t] = load_eight<DT>(xs, (x_row[t] + static_cast<uint32_t>(c * E)) | past);
+    };
+    auto q_at = [&](int b, int c0, int first) __attribute__((always_inline)) {  // from channel `first` of a group
+        const int c = c0 + 8 * g;
+        return (q_row[b] + static_cast<uint32_t>((c + first) * 2)) | (c < channels ? 0u : kOutOfRange);
     };
     d4 acc[TB][NB];
 #pragma unroll
     for (int t = 0; t < TB; ++t)
 #pragma unroll
         for (int b = 0; b < NB; ++b) acc[t][b] = d4{};
-    const int first = SPLIT > 1 ? 32 * wave : 0;
-    load(first, x_now, q_now);
-    for (int c0 = first; c0 < channels; c0 += 32 * SPLIT) {
-        load(c0 + 32 * SPLIT, x_next, q_next);
+    auto products = [&](auto&& basis) __attribute__((always_inline)) {  // basis(b, s): channel s of rank block b
         double xv[TB][8];
 #pragma unroll
         for (int t = 0; t < TB; ++t)
 #pragma unroll
             for (int s = 0; s < 8; ++s) xv[t][s] = eight_at<DT>(x_now[t], s);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
             for (int s = 0; s < 8; ++s) {
-                const double qv = eight_at<RCH_DT_F16>(q_now[b], s);
+                const double qv = basis(b, s);
 #pragma unroll
                 for (int t = 0; t < TB; ++t)
                     acc[t][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv[t][s], qv, acc[t][b], 0, 0, 0);
             }
-        }
+    };
+    auto advance = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < TB; ++t) x_now[t] = x_next[t];
+    };
+    if constexpr (SPLIT == 1) {  // wave w converts channels 2w, 2w + 1 of every group for all four waves
+        static_assert(kThreads == 256, "four waves share a step's eight channels");
+        constexpr int kStep = 8 * NB * 64;
+        uint32_t pair[NB];
+        auto load_pair = [&](int c0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int b = 0; b < NB; ++b) q_now[b] = q_next[b];
+            for (int b = 0; b < NB; ++b) pair[b] = __builtin_amdgcn_raw_buffer_load_b32(qs, q_at(b, c0, 2 * wave), 0, 0);
+        };
+        auto stage = [&](int at) __attribute__((always_inline)) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                double* to = shared + at + (8 * b + 2 * wave) * 64 + lane;
+                to[0] = static_cast<double>(half_bits<RCH_DT_F16>(pair[b] & 0xffffu));
+                to[64] = static_cast<double>(half_bits<RCH_DT_F16>(pair[b] >> 16));
+            }
+        };
+        load_x(0), load_pair(0);
+        stage(0), advance();
+        __syncthreads();
+        for (int c0 = 0, at = 0; c0 < channels; c0 += 32, at = kStep - at) {
+            load_x(c0 + 32), load_pair(c0 + 32);
+            products([&](int b, int s) { return shared[at + (8 * b + s) * 64 + lane]; });
+            stage(kStep - at), advance();  // this half was last read before the previous barrier
+            __syncthreads();
+        }
+    } else {
+        Eight<RCH_DT_F16> q_now[NB], q_next[NB];
+        auto load_q = [&](int c0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) q_next[b] = load_eight<RCH_DT_F16>(qs, q_at(b, c0, 0));
+        };
+        auto advance_q = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) q_now[b] = q_next[b];
+        };
+        load_x(32 * wave), load_q(32 * wave);
+        advance(), advance_q();
+        for (int c0 = 32 * wave; c0 < channels; c0 += 32 * SPLIT) {
+            load_x(c0 + 32 * SPLIT), load_q(c0 + 32 * SPLIT);
+            products([&](int b, int s) { return eight_at<RCH_DT_F16>(q_now[b], s); });
+            advance(), advance_q();
+        }
     }
     if constexpr (SPLIT > 1) {  // block b of every wave is added, in wave order, by wave b
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) partial[((b * SPLIT + wave) * 4 + v) * 64 + lane] = acc[0][b][v];
+            for (int v = 0; v < 4; ++v) shared[((b * SPLIT + wave) * 4 + v) * 64 + lane] = acc[0][b][v];
         __syncthreads();
         if (wave >= NB) return;
         d4 sum = d4{};
 #pragma unroll
         for (int w = 0; w < SPLIT; ++w)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) sum[v] += partial[((wave * SPLIT + w) * 4 + v) * 64 + lane];
+            for (int v = 0; v < 4; ++v) sum[v] += shared[((wave * SPLIT + w) * 4 + v) * 64 + lane];
         acc[0][0] = sum;
         if constexpr (GRAM) {  // rows and columns past the rank are zeros
             const int kp = padded_order(rank), k = r0 + 16 * wave + i16;
@@ -546,7 +590,8 @@ template <int DT, int TB, int SPLIT>
 __global__ void __launch_bounds__(kThreads, 2) project_kernel(const rch_fit_matrix* __restrict__ mats, int channels,
                                                               int chunk) {
     static_assert(SPLIT == 1 || (SPLIT == kThreads / 64 && TB == 1), "all waves split the channels, or none");
-    __shared__ double partial[SPLIT > 1 ? 4 * SPLIT * 4 * 64 : 1];
+    // Partial sums of up to four rank blocks, or the basis operands of two steps.
+    __shared__ double shared[SPLIT > 1 ? 4 * SPLIT * 4 * 64 : 2 * 8 * 4 * 64];
     const rch_fit_matrix* M = mats + blockIdx.z;
     const int rank = static_cast<int>(M->rank);
     const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kProjectTokens<TB, SPLIT>;
@@ -555,29 +600,33 @@ __global__ void __launch_bounds__(kThreads, 2) project_kernel(const rch_fit_matr
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int64_t wt = SPLIT > 1 ? t0 : t0 + 16 * TB * wave;  // first token of this wave
     switch (min(chunk >> 4, (rank - r0 + 15) >> 4)) {  // 16-rank blocks of this chunk (uniform)
-        case 1: project_ranks<DT, TB, SPLIT, 1>(M, channels, r0, wt, wave, lane, partial); break;
-        case 2: project_ranks<DT, TB, SPLIT, 2>(M, channels, r0, wt, wave, lane, partial); break;
-        case 3: project_ranks<DT, TB, SPLIT, 3>(M, channels, r0, wt, wave, lane, partial); break;
-        default: project_ranks<DT, TB, SPLIT, 4>(M, channels, r0, wt, wave, lane, partial); break;
+        case 1: project_ranks<DT, TB, SPLIT, 1>(M, channels, r0, wt, wave, lane, shared); break;
+        case 2: project_ranks<DT, TB, SPLIT, 2>(M, channels, r0, wt, wave, lane, shared); break;
+        case 3: project_ranks<DT, TB, SPLIT, 3>(M, channels, r0, wt, wave, lane, shared); break;
+        default: project_ranks<DT, TB, SPLIT, 4>(M, channels, r0, wt, wave, lane, shared); break;
     }
 }
 
 // ---------------------------------------------------------------------------------------------
 // Residual energies on v_mfma_f64_16x16x4f64: D[m = token][n = channel] = sum_k P[token][k] Q[k][c].
-// Workgroup = 16 TB tokens of one matrix and every gridDim.z-th set of four 64-channel groups, one
-// group per wave.  A group
-// is four 16 x 16 blocks per 16 tokens whose columns interleave: column i of block b is channel
+// Workgroup = some tokens of one matrix and every gridDim.z-th set of 64-channel groups.  A group is four 16 x 16 blocks per 16 tokens whose columns interleave: column i of block b is channel
 // 4i + b of the group, so after the four blocks lane l (i = l % 16, g = l / 16) holds channels 4i ..
 // 4i + 3 of tokens g + 4v (v = 0..3, the f64 accumulator's row (l / 16) + 4v): X and the residual move
 // as 4-channel vectors, 16 lanes covering 64 contiguous channels of a row.  Per 16-rank step a lane
 // takes P[token i][4g .. 4g + 3] (the A operand; MFMA step j takes rank 4g + j) and, for each j,
 // Q[4g + j][4i .. 4i + 3] (one 8-byte load: the B operands of the four blocks).
 //
-// Bound by the FP64 matrix rate (rank 0, the source energy alone: by HBM): the next step's operands
-// and the next group's source elements are loaded before a step's products.  TB = 2 lets each
-// converted basis operand feed two products; small batches take TB = 1 and split the channels over
-// workgroups (grid z) until they fill the chip.  One bf16 matrix [4680, 1536] at rank 96: 137 -> 40 us;
-// 60 matrices: 1808 -> 1527 us (54 TFLOP/s); source energy of one: 29 -> 18 us.
+// Two shapes:
+//   * SHARED: a wave owns 32 of the workgroup's 128 tokens and all waves walk the same channel groups,
+//     sharing a step's converted basis operands through LDS (two halves, one barrier a step): a wave loads
+//     and converts a quarter of them and each feeds two of its products.
+//   * for batches that would leave CUs idle: 16 tokens, a channel group per wave.
+// Bound by the FP64 matrix rate (rank 0, the source energy alone: by HBM), with the vector instructions
+// beside it: they do not hide under FP64 products.  The next step's operands are loaded before a step's
+// products and a group's source elements before all of its products.
+// One bf16 matrix [4680, 1536] at rank 96: 137 -> 40 us; 60 matrices at rank 96: 1808 us with 16-token
+// workgroups, 1527 with 32-token ones of unshared operands, 1450 now (57 TFLOP/s); ranks 32 to 128 in one
+// batch: 1350 -> 1290 us; 8 matrices [4680, 4096] at ranks 256 and 512: 2394 -> 2184 us; source energy of one: 29 -> 18 us.
 // ---------------------------------------------------------------------------------------------
 
 // The 4 channels of tokens g + 4v (v = 0..3) of a lane's 64-channel group, as raw 16-bit pairs
@@ -588,21 +637,61 @@ struct SourceQuad {
     word w[4];
 };
 
-template <int DT, int TB>
+__device__ __forceinline__ void residual_total(const rch_fit_matrix* M, double src, double err,
+                                               double (*part)[kThreads / 64], int wave, int lane) {
+    // Fixed-order reduction: butterfly within the wave, then waves 0..3 in order.
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        src += __shfl_xor(src, d);
+        err += __shfl_xor(err, d);
+    }
+    if (lane == 0) {
+        part[0][wave] = src;
+        part[1][wave] = err;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double a = 0.0, b = 0.0;
+        for (int w = 0; w < kThreads / 64; ++w) {
+            a += part[0][w];
+            b += part[1][w];
+        }
+        const float smax = __uint_as_float(*gin<unsigned int>(M->absmax_ptr));
+        if (smax != 0.0f) {
+            const double s = static_cast<double>(smax);
+            a = a / s / s;
+            b = b / s / s;
+        }
+        RCH_GLOBAL double* out = gout<double>(M->partial_ptr) + 2 * (gridDim.z * blockIdx.x + blockIdx.z);
+        out[0] = a;
+        out[1] = b;
+    }
+}
+
+// Tokens of a residual_kernel workgroup, and channels that its waves cover at once.
+template <bool SHARED>
+constexpr int kResidualTokens = SHARED ? 32 * (kThreads / 64) : 16;
+template <bool SHARED>
+constexpr int kResidualChannels = SHARED ? 64 : 64 * (kThreads / 64);
+
+template <int DT, bool SHARED>
 __global__ void __launch_bounds__(kThreads, 2) residual_kernel(const rch_fit_matrix* __restrict__ mats, int channels) {
-    constexpr int E = esize<DT>();
-    constexpr int kTokens = 16 * TB, kWaves = kThreads / 64;
+    constexpr int E = esize<DT>(), TB = SHARED ? 2 : 1, kWaves = kThreads / 64;
+    constexpr int kStep = 16 * 64;  // basis operands of a 16-rank step, [j: rank 4g + j][block][lane]
+    static_assert(kWaves == 4, "wave j shares the rows of ranks 4g + j");
+    __shared__ double staged[SHARED ? 2 * kStep : 1];
+    __shared__ double part[2][kWaves];
     const rch_fit_matrix* M = mats + blockIdx.y;
     const int64_t rows = M->rows;
     const int rank = static_cast<int>(M->rank);
-    const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kTokens;
-    if (t0 >= rows) return;
+    const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kResidualTokens<SHARED>;
+    if (t0 >= rows) return;  // whole workgroup
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int g = lane >> 4, i16 = lane & 15;
-    const int64_t left = rows - t0;
-    const __amdgpu_buffer_rsrc_t xs = source_rows<DT>(M, channels, t0);
-    const __amdgpu_buffer_rsrc_t ps = make_rsrc(M->coef_ptr + t0 * M->coef_stride * 4,
-                                                rank > 0 ? ((left - 1) * M->coef_stride + rank) * 4 : 0);
+    const int64_t wt = SHARED ? t0 + 32 * wave : t0, left = rows - wt;  // rows past the end read zeros
+    const __amdgpu_buffer_rsrc_t xs = source_rows<DT>(M, channels, wt);
+    const __amdgpu_buffer_rsrc_t ps = make_rsrc(M->coef_ptr + wt * M->coef_stride * 4,
+                                                rank > 0 && left > 0 ? ((left - 1) * M->coef_stride + rank) * 4 : 0);
     const __amdgpu_buffer_rsrc_t qs = make_rsrc(M->basis_ptr, rank > 0 ? ((rank - 1) * M->basis_stride + channels) * 2 : 0);
     const uint32_t q_stride = static_cast<uint32_t>(M->basis_stride * 2);
     RCH_GLOBAL float* resid = M->resid_ptr ? gout<float>(M->resid_ptr) : nullptr;
@@ -625,56 +714,47 @@ __global__ void __launch_bounds__(kThreads, 2) residual_kernel(const rch_fit_mat
                 else q[t].w[v] = __builtin_amdgcn_raw_buffer_load_b64(xs, offset, 0, 0);
             }
     };
-    struct Operands {
-        u2 q[4];   // Q[k + j][4 channels], j = 0..3
-        u4 p[TB];  // P[token][k .. k + 3]
-    };
-    auto load_operands = [&](int c64, int k0, Operands& o) __attribute__((always_inline)) {
+    // Q[k0 + 4g + j][4 channels] (SHARED: j = wave alone) and P[token][k0 + 4g ..].
+    u2 q_now[SHARED ? 1 : 4], q_next[SHARED ? 1 : 4];
+    u4 p_now[TB], p_next[TB];
+    auto load_operands = [&](int c64, int k0) __attribute__((always_inline)) {
         const int c = c64 + 4 * i16, k = k0 + 4 * g;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t offset = (k + j < rank && c < channels) ? static_cast<uint32_t>(k + j) * q_stride + 2u * c : kOutOfRange;
-            o.q[j] = __builtin_amdgcn_raw_buffer_load_b64(qs, offset, 0, 0);
+        for (int q = 0; q < (SHARED ? 1 : 4); ++q) {
+            const int kq = k + (SHARED ? wave : q);
+            const uint32_t offset = (kq < rank && c < channels) ? static_cast<uint32_t>(kq) * q_stride + 2u * c : kOutOfRange;
+            q_next[q] = __builtin_amdgcn_raw_buffer_load_b64(qs, offset, 0, 0);
         }
 #pragma unroll
         for (int t = 0; t < TB; ++t)
-            o.p[t] = __builtin_amdgcn_raw_buffer_load_b128(ps, k < rank ? p_row[t] + static_cast<uint32_t>(k * 4) : kOutOfRange, 0, 0);
+            p_next[t] = __builtin_amdgcn_raw_buffer_load_b128(ps, k < rank ? p_row[t] + static_cast<uint32_t>(k * 4) : kOutOfRange, 0, 0);
+    };
+    auto basis_at = [](const u2& q, int b) __attribute__((always_inline)) {
+        return static_cast<double>(half_bits<RCH_DT_F16>((q[b >> 1] >> (16 * (b & 1))) & 0xffffu));
+    };
+    auto advance = [&](int k0, int at) __attribute__((always_inline)) {  // the loaded operands are the next step's
+        if constexpr (SHARED) {
+#pragma unroll
+            for (int b = 0; b < 4; ++b) staged[at + (4 * wave + b) * 64 + lane] = basis_at(q_next[0], b);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) q_now[q] = q_next[q];
+        }
+        if (k0 + 16 > rank) {  // P rows may hold padding beyond the rank; its basis rows read as zero
+#pragma unroll
+            for (int t = 0; t < TB; ++t)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) p_next[t][j] = k0 + 4 * g + j < rank ? p_next[t][j] : 0u;
+        }
+#pragma unroll
+        for (int t = 0; t < TB; ++t) p_now[t] = p_next[t];
+        if constexpr (SHARED) __syncthreads();
     };
 
     double src = 0.0, err = 0.0;
-    SourceQuad<DT> x_now[TB], x_next[TB];
-    Operands now, next;
-    const int first = 64 * (wave + kWaves * static_cast<int>(blockIdx.z));
-    const int stride = 64 * kWaves * static_cast<int>(gridDim.z);
-    load_source(first, x_now);
-    if (rank > 0) load_operands(first, 0, now);
-    for (int c64 = first; c64 < channels; c64 += stride) {
-        load_source(c64 + stride, x_next);
-        d4 acc[TB][4];
-#pragma unroll
-        for (int t = 0; t < TB; ++t)
-#pragma unroll
-            for (int b = 0; b < 4; ++b) acc[t][b] = d4{};
-        for (int k0 = 0; k0 < rank; k0 += 16) {
-            const bool last = k0 + 16 >= rank;
-            load_operands(last ? c64 + stride : c64, last ? 0 : k0 + 16, next);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                // P rows may hold padding beyond the rank; its basis rows read as zero.
-                double pa[TB];
-#pragma unroll
-                for (int t = 0; t < TB; ++t)
-                    pa[t] = k0 + 4 * g + j < rank ? static_cast<double>(__uint_as_float(now.p[t][j])) : 0.0;
-#pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    const double qb = static_cast<double>(half_bits<RCH_DT_F16>((now.q[j][b >> 1] >> (16 * (b & 1))) & 0xffffu));
-#pragma unroll
-                    for (int t = 0; t < TB; ++t) acc[t][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(pa[t], qb, acc[t][b], 0, 0, 0);
-                }
-            }
-            now = next;
-        }
-        // e = x - r per element: FP64 sums of x^2 and e^2, optional fp32 store.
+    d4 acc[TB][4];
+    // e = x - r per element: FP64 sums of x^2 and e^2, optional fp32 store.
+    auto finish = [&](int c64, const SourceQuad<DT> (&x)[TB]) __attribute__((always_inline)) {
         const int c = c64 + 4 * i16;
 #pragma unroll
         for (int t = 0; t < TB; ++t)
@@ -684,11 +764,9 @@ __global__ void __launch_bounds__(kThreads, 2) residual_kernel(const rch_fit_mat
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
                     double a;
-                    if constexpr (DT == RCH_DT_F32) a = static_cast<double>(__uint_as_float(x_now[t].w[v][b]));
-                    else a = static_cast<double>(half_bits<DT>((x_now[t].w[v][b >> 1] >> (16 * (b & 1))) & 0xffffu));
+                    if constexpr (DT == RCH_DT_F32) a = static_cast<double>(__uint_as_float(x[t].w[v][b]));
+                    else a = static_cast<double>(half_bits<DT>((x[t].w[v][b >> 1] >> (16 * (b & 1))) & 0xffffu));
                     e[b] = a - acc[t][b][v];
-                    // The scale s is applied once per tile: sum (a / s)^2 = (sum a^2) / s^2 up to the
-                    // rounding of the FP64 sums (relative 1e-16), without two FP64 divisions per element.
                     src = fma(a, a, src);
                     err = fma(e[b], e[b], err);
                 }
@@ -696,40 +774,61 @@ __global__ void __launch_bounds__(kThreads, 2) residual_kernel(const rch_fit_mat
                 if (resid && c < channels && token < left) {
                     const f4 out = {static_cast<float>(e[0]), static_cast<float>(e[1]), static_cast<float>(e[2]),
                                     static_cast<float>(e[3])};
-                    *reinterpret_cast<RCH_GLOBAL f4*>(resid + (t0 + token) * channels + c) = out;
+                    *reinterpret_cast<RCH_GLOBAL f4*>(resid + (wt + token) * channels + c) = out;
                 }
             }
+    };
+    const int first = kResidualChannels<SHARED> * static_cast<int>(blockIdx.z) + (SHARED ? 0 : 64 * wave);
+    const int stride = kResidualChannels<SHARED> * static_cast<int>(gridDim.z);
+    SourceQuad<DT> x_now[TB];
+    if (rank > 0) {
+        load_operands(first, 0);
+        advance(0, 0);
+        int at = 0;
+        for (int c64 = first; c64 < channels; c64 += stride) {
+            load_source(c64, x_now);  // in flight under the group's products
 #pragma unroll
-        for (int t = 0; t < TB; ++t) x_now[t] = x_next[t];
-    }
-    // Fixed-order reduction: butterfly within the wave, then waves 0..3 in order.
+            for (int t = 0; t < TB; ++t)
 #pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-        src += __shfl_xor(src, d);
-        err += __shfl_xor(err, d);
-    }
-    __shared__ double part[2][kWaves];
-    if (lane == 0) {
-        part[0][wave] = src;
-        part[1][wave] = err;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double a = 0.0, b = 0.0;
-        for (int w = 0; w < kWaves; ++w) {
-            a += part[0][w];
-            b += part[1][w];
+                for (int b = 0; b < 4; ++b) acc[t][b] = d4{};
+            for (int k0 = 0; k0 < rank; k0 += 16) {
+                const bool last = k0 + 16 >= rank;
+                const int k_next = last ? 0 : k0 + 16;
+                load_operands(last ? c64 + stride : c64, k_next);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    double pa[TB];
+#pragma unroll
+                    for (int t = 0; t < TB; ++t) pa[t] = static_cast<double>(__uint_as_float(p_now[t][j]));
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) {
+                        double qb;
+                        if constexpr (SHARED) qb = staged[at + (4 * j + b) * 64 + lane];
+                        else qb = basis_at(q_now[j], b);
+#pragma unroll
+                        for (int t = 0; t < TB; ++t) acc[t][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(pa[t], qb, acc[t][b], 0, 0, 0);
+                    }
+                }
+                at = kStep - at;  // this half was last read before the previous barrier
+                advance(k_next, at);
+            }
+            finish(c64, x_now);
         }
-        const float smax = __uint_as_float(*gin<unsigned int>(M->absmax_ptr));
-        if (smax != 0.0f) {
-            const double s = static_cast<double>(smax);
-            a = a / s / s;
-            b = b / s / s;
+    } else {  // the source energy alone: one group ahead
+#pragma unroll
+        for (int t = 0; t < TB; ++t)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) acc[t][b] = d4{};
+        SourceQuad<DT> x_next[TB];
+        load_source(first, x_now);
+        for (int c64 = first; c64 < channels; c64 += stride) {
+            load_source(c64 + stride, x_next);
+            finish(c64, x_now);
+#pragma unroll
+            for (int t = 0; t < TB; ++t) x_now[t] = x_next[t];
         }
-        RCH_GLOBAL double* out = gout<double>(M->partial_ptr) + 2 * (gridDim.z * blockIdx.x + blockIdx.z);
-        out[0] = a;
-        out[1] = b;
     }
+    residual_total(M, src, err, part, wave, lane);
 }
 
 // Sum of the partials of each matrix (`splits` per `tokens` rows): one wave per matrix, lane l takes
@@ -1311,11 +1410,17 @@ __global__ void __launch_bounds__(256) gaussian_kernel(const rch_gauss_job* __re
 
 // Measured on [n x 4680, 1536] bf16 (MI355X, host-side upload included): the projection's 128-token
 // workgroups beat the channel-split ones at 2220 workgroups (60 matrices, rank 32: 514 / 533 us) and lose
-// at 592 (8 matrices, rank 96: 254 / 224 us); the residual's 32-token workgroups win at 1176 (8
-// matrices: 242 / 269 us) and lose at 588 (4 matrices, rank 96: 156 / 134 us).
+// at 592 (8 matrices, rank 96: 254 / 224 us); the residual's shared form against its 16-token one at rank
+// 96: 123 / 140 us at 588 groups (4 matrices), 78 / 80 at 294, 55 / 51 at 147 (one matrix).
 constexpr int64_t kProjectWholeGroups = 2000;
-constexpr int64_t kResidualPairGroups = 1000;
-constexpr int64_t kResidualSplitGroups = 2000;  // workgroups that the channel splits aim at
+constexpr int64_t kResidualSharedGroups = 500;  // of 32 tokens
+// Workgroups that the channel splits aim at, and the fewest parts of the 128-token ones, which are long and
+// at mixed ranks unequal (60 matrices at ranks 32 to 128: one part 1400 us, two 1304, three 1285, four 1270;
+// more parts cost a batch without bases, whose workgroups then end before their loads overlap: 24 matrices 72
+// us at three parts, 84 at seven).
+constexpr int64_t kResidualSplitAim = 2000, kResidualSharedSplits = 3;
+constexpr int64_t kResidualSplits = 4;  // of 16-token tiles: a wave's first loads then serve one or two groups
+static_assert(kResidualSplits <= RCH_RESIDUAL_SPLITS, "partials are allocated for RCH_RESIDUAL_SPLITS parts");
 
 int check_matrices(const rch_fit_matrix* mats, int n, int channels, const char* what) {
     if (!mats || n <= 0 || n > 65535) return fail(RCH_E_CONFIG, "%s: 1 <= n_mats <= 65535 required", what);
@@ -1407,29 +1512,30 @@ int rch_fit_residual(const rch_fit_matrix* mats_dev, int n_mats, int channels, i
     if (int status = check_matrices(mats_dev, n_mats, channels, "rch_fit_residual")) return status;
     if (max_rows <= 0 || (max_rows + 15) / 16 > 0x7fffffff) return fail(RCH_E_CONFIG, "rch_fit_residual: invalid max_rows");
     hipStream_t s = as_stream(stream);
-    // 32-token workgroups while they fill the chip, else 16-token ones with the channels split.
-    const int tokens = (max_rows + 31) / 32 * n_mats >= kResidualPairGroups ? 32 : 16;
-    int splits = 1;
-    if (tokens == 16) {
-        const int64_t groups = (max_rows + 15) / 16 * n_mats, most = (channels + 255) / 256;
-        const int64_t wanted = (kResidualSplitGroups + groups - 1) / groups;
-        splits = static_cast<int>(wanted < most ? wanted : most);
-        splits = splits > RCH_RESIDUAL_SPLITS ? RCH_RESIDUAL_SPLITS : splits;
-    }
+    // 128-token workgroups, the channels split where those are few, while their waves fill the chip, else
+    // 16-token ones, the channels split as well.
+    const bool shared = (max_rows + 31) / 32 * n_mats >= kResidualSharedGroups;
+    const int tokens = shared ? kResidualTokens<true> : kResidualTokens<false>;
+    const int channel_part = shared ? kResidualChannels<true> : kResidualChannels<false>;
+    const int64_t groups = (max_rows + tokens - 1) / tokens * n_mats;
+    const int64_t wanted = std::max<int64_t>((kResidualSplitAim + groups - 1) / groups, shared ? kResidualSharedSplits : 1);
+    const int64_t most = std::min<int64_t>((channels + channel_part - 1) / channel_part,
+                                           shared ? RCH_RESIDUAL_SPLITS : kResidualSplits);
+    const int splits = static_cast<int>(std::min(wanted, most));
     const dim3 grid(static_cast<unsigned>((max_rows + tokens - 1) / tokens), static_cast<unsigned>(n_mats),
                     static_cast<unsigned>(splits));
     switch (src_dtype) {
         case RCH_DT_BF16:
-            if (tokens == 32) hipLaunchKernelGGL((residual_kernel<RCH_DT_BF16, 2>), grid, dim3(kThreads), 0, s, mats_dev, channels);
-            else hipLaunchKernelGGL((residual_kernel<RCH_DT_BF16, 1>), grid, dim3(kThreads), 0, s, mats_dev, channels);
+            if (shared) hipLaunchKernelGGL((residual_kernel<RCH_DT_BF16, true>), grid, dim3(kThreads), 0, s, mats_dev, channels);
+            else hipLaunchKernelGGL((residual_kernel<RCH_DT_BF16, false>), grid, dim3(kThreads), 0, s, mats_dev, channels);
             break;
         case RCH_DT_F16:
-            if (tokens == 32) hipLaunchKernelGGL((residual_kernel<RCH_DT_F16, 2>), grid, dim3(kThreads), 0, s, mats_dev, channels);
-            else hipLaunchKernelGGL((residual_kernel<RCH_DT_F16, 1>), grid, dim3(kThreads), 0, s, mats_dev, channels);
+            if (shared) hipLaunchKernelGGL((residual_kernel<RCH_DT_F16, true>), grid, dim3(kThreads), 0, s, mats_dev, channels);
+            else hipLaunchKernelGGL((residual_kernel<RCH_DT_F16, false>), grid, dim3(kThreads), 0, s, mats_dev, channels);
             break;
         case RCH_DT_F32:
-            if (tokens == 32) hipLaunchKernelGGL((residual_kernel<RCH_DT_F32, 2>), grid, dim3(kThreads), 0, s, mats_dev, channels);
-            else hipLaunchKernelGGL((residual_kernel<RCH_DT_F32, 1>), grid, dim3(kThreads), 0, s, mats_dev, channels);
+            if (shared) hipLaunchKernelGGL((residual_kernel<RCH_DT_F32, true>), grid, dim3(kThreads), 0, s, mats_dev, channels);
+            else hipLaunchKernelGGL((residual_kernel<RCH_DT_F32, false>), grid, dim3(kThreads), 0, s, mats_dev, channels);
             break;
         default: return fail(RCH_E_CONFIG, "rch_fit_residual: source dtype must be bf16, f16 or f32");
     }

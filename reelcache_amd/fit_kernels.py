@@ -20,7 +20,7 @@ from .errors import ConfigurationError, UnsupportedError
 _DTYPE_CODES = {torch.bfloat16: _lib.DT_BF16, torch.float16: _lib.DT_F16, torch.float32: _lib.DT_F32}
 #: fp32 bits of +inf: an absmax key at or above it marks a non-finite source element.
 NONFINITE_BITS = 0x7F800000
-_ROW_TILE, _ROW_SPLITS = 16, 4  # fewest rows per partial energy, most channel parts of one (RCH_RESIDUAL_SPLITS)
+_ROW_TILE, _ROW_SPLITS = 16, 8  # fewest rows per partial energy, most channel parts of one (RCH_RESIDUAL_SPLITS)
 
 
 def _device(tensors) -> torch.device:

@@ -317,6 +317,9 @@ def test_cholesky_inverse_flags_indefinite_members(device):
     (3, 31, 136, [16, 33, 130]),        # ragged ranks over several rank chunks
     (70, 2000, 64, [49]),               # token-blocked shapes (32-token workgroups), 64-channel rows
     (160, 1664, 40, [32]),              # 128-token projection workgroups
+    (350, 700, 72, [1, 33, 64]),        # shared basis operands: a last wave of 28 rows, one to four rank blocks
+    (18, 1000, 200, [16, 130, 75]),     # shared residual operands, four channel parts, ranks past a step
+    (500, 33, 72, [20, 5, 48]),         # waves of 32 rows, one row and none
 ])
 def test_fit_launch_shapes_match_fp64(device, dtype, count, rows, channels, ranks):
     """absmax, projection and residual energies on both sides of their launch-shape rules: maxima
