@@ -169,10 +169,10 @@ def _check_item(item: FinalizeItem) -> int:
 
 
 def _rank_terms(coefficients, rows):
-    """Per tile of one rank above the native kernels' order (``fit_kernels.span_terms``): FP64 span trace ``trace(G^-1 C)`` (``G = Q Q^T``, ``C = P^T P``), the
-    Cholesky status of ``G``, and the fast condition terms (``eta = ||Q Q^T - I||_inf`` of the fp32
-    Gram -- fp16 products are exact in fp32 -- and its largest diagonal entry): a handful of
-    batched launches for the whole group."""
+    """Per tile of one rank above the native kernels' order (``fit_kernels.span_terms`` takes the
+    others): FP64 span trace ``trace(G^-1 C)`` (``G = Q Q^T``, ``C = P^T P``), the Cholesky status of
+    ``G``, and the fast condition terms (``eta = ||Q Q^T - I||_inf`` of the fp32 Gram -- fp16 products
+    are exact in fp32 -- and its largest diagonal entry): a handful of batched launches for the group."""
     q = torch.stack(rows)
     # Tiles of one token count: one stack and one widening for the group.
     p = torch.stack(coefficients).double() if len({c.shape[0] for c in coefficients}) == 1 else None
