@@ -20,7 +20,7 @@
 extern "C" {
 #endif
 
-#define RCH_ABI_VERSION 17
+#define RCH_ABI_VERSION 18
 
 /* Status codes (mapped to reelcache errors by the host). */
 #define RCH_OK 0
@@ -375,7 +375,7 @@ typedef struct rch_fit_matrix {
     int64_t absmax_ptr;   /* uint32: fp32 bits of max|X| (zero-filled, then rch_fit_absmax) */
     int64_t extrema_ptr;  /* uint32 [2, rank]: ~key(min) then key(max) of each column of P, or 0 */
     int64_t energy_ptr;   /* float64 [2]: sum (X/s)^2 and sum ((X - P Q)/s)^2, s = max|X| */
-    int64_t partial_ptr;  /* float64 [RCH_RESIDUAL_SPLITS * ceil(rows / 16), 2]: partial energies */
+    int64_t partial_ptr;  /* float64 [RCH_RESIDUAL_PARTS * ceil(rows / 16), 2]: partial energies */
     int64_t resid_ptr;    /* fp32 [rows, channels] (row stride = channels): X - P Q[:rank], or 0 */
 } rch_fit_matrix;         /* 16 x int64 = 128 bytes */
 
@@ -402,7 +402,8 @@ int rch_fit_gram(const rch_fit_matrix* mats_dev, int n_mats, int channels, int s
 
 /*
  * Coefficients P = X Q[:rank]^T of each matrix: exact products accumulated in FP64 on
- * v_mfma_f64_16x16x4f64, rounded once to fp32.  When extrema_ptr is set, also the per-column
+ * v_mfma_f64_16x16x4f64 in an order that depends on the channels alone (a matrix's P has the same bits
+ * in every batch), rounded once to fp32.  When extrema_ptr is set, also the per-column
  * min / max of P as order-preserving keys (unsigned atomic max, zero-filled by the caller).
  * Replaces `tensor.float() @ b32.T` of project_onto_basis (reelcache/factorization.py:384-392)
  * and the extrema of quantize_device (reelcache/node_packets.py:164).
@@ -410,13 +411,14 @@ int rch_fit_gram(const rch_fit_matrix* mats_dev, int n_mats, int channels, int s
 int rch_fit_project(const rch_fit_matrix* mats_dev, int n_mats, int channels, int64_t max_rows, int max_rank,
                     int src_dtype, void* stream);
 
-#define RCH_RESIDUAL_SPLITS 8 /* most channel parts of a row tile, each with a partial of its own */
+#define RCH_RESIDUAL_PARTS 16 /* most channel parts of a 16-row tile, each with a partial of its own */
 /*
  * Direct residual and source energies of each matrix in FP64: sum (X / s)^2 and
  * sum ((X - P Q[:rank]) / s)^2 with s = max|X| read from *absmax_ptr (no scaling when s == 0),
- * the reconstruction accumulated in FP64 on v_mfma_f64_16x16x4f64.  Partials (of 16 or 32 rows and all
- * or a part of the channels) go to partial_ptr and are summed in a fixed order into energy_ptr (deterministic).  rank == 0
- * measures the source energy alone.  With resid_ptr set, also writes the residual matrix
+ * the reconstruction accumulated in FP64 on v_mfma_f64_16x16x4f64.  Partials (of 16 rows and a part of the
+ * channels) go to partial_ptr and are summed into energy_ptr; the order of every sum depends on the matrix's
+ * rows, channels and rank alone, so its energies have the same bits in every batch.  rank == 0 measures the
+ * source energy alone.  With resid_ptr set, also writes the residual matrix
  * fp32(X - P Q[:rank]) (the residual an inherited basis leaves for augmentation,
  * reelcache/rank_method.py:1347-1358).
  * Replaces the tiled residual guard of project_onto_basis (reelcache/factorization.py:398-419)

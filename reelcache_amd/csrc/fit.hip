@@ -13,7 +13,10 @@
 //     exactly to FP64, products and sums on v_mfma_f64_16x16x4f64, P rounded once to fp32.
 //     The FP64 sum makes P the correctly rounded fp32 value of the exact dot product except
 //     within ~1e-13 relative of a rounding boundary, i.e. independent of summation order.
-//   * Energies: FP64 sums of (x - r)^2 and x^2, divided by s^2 per partial (16 or 32 rows), fixed-order totals.
+//   * Energies: FP64 sums of (x - r)^2 and x^2 over partials of 16 rows and a part of the channels, totalled in
+//     one order and divided by s^2.
+//   * P, energies and span traces of a matrix have the same bits in every batch: the launch shape depends on
+//     the batch, the order of the sums only on the matrix.
 //   * Quantizer: FP64 (v - offset) / scale, round half to even, clamp to [0, 255].
 #include <algorithm>
 #include <type_traits>
@@ -389,23 +392,27 @@ __global__ void __launch_bounds__(kGramThreads) gram_kernel(const rch_fit_matrix
 // ---------------------------------------------------------------------------------------------
 // Projection P = X Q^T on v_mfma_f64_16x16x4f64: D[m = token][n = rank] = sum_c X[token][c] Q[rank][c].
 // Per 32-channel step a lane (i = l % 16, group g = l / 16) holds channels 8g .. 8g + 7 of its token
-// rows and of its basis rows (16-byte loads, no LDS), and MFMA step s takes channel 8g + s from every
-// group.  The f64 accumulator holds element v of lane l at row (l / 16) + 4v, column l % 16: token
-// g + 4v, rank i of the block.
+// rows and of its basis rows (16-byte loads), and MFMA step s takes channel 8g + s from every group.  The
+// f64 accumulator holds element v of lane l at row (l / 16) + 4v, column l % 16: token g + 4v, rank i of
+// the block.
 //
-// Bound by the FP64 matrix rate; the next step's loads are issued before a step's products and the
-// step body has no branch, so their latency is covered.  Two shapes (project_kernel's TB, SPLIT):
-//   * TB = 2, SPLIT = 1: a wave owns 32 tokens; the four waves share a step's converted basis operands
-//     through LDS (two halves, one barrier a step), so a wave loads and converts a quarter of them and
-//     each feeds two of its products; workgroup = 128 tokens x 64 ranks.
-//   * TB = 1, SPLIT = 4: for batches that would leave CUs idle, the four waves of a workgroup share 16
-//     tokens and split the channel steps; the partial sums are added through LDS in wave order.
-// GRAM: the sources are the basis rows themselves and the FP64 sums are stored as they are, G = Q Q^T.
-// One bf16 matrix [4680, 1536] at rank 96: 105 us with 64-token workgroups of one wave per 16 tokens and
-// loads in the step, 36 us now; 60 matrices at rank 96: 1563 us, 1396 with every wave converting its own
-// basis operands, 1293-1329 now.  The vector instructions do not hide under FP64 products, and the rate
-// depends on the operands' bits: products of full 53-bit operands alone reach 46-49 TFLOP/s, a large
+// Every element is the sum of two chains, over the first and the second half of the channel steps, each run
+// by a wave of its own, whatever the shape of the launch: the bits of P do not depend on the batch, which
+// chooses the shape.
+//   * kShared: a wave owns 32 tokens and half of the channels; the four waves of a half share a step's
+//     converted basis operands through LDS (two parts, one barrier a step), so a wave loads and converts a
+//     quarter of them and each feeds two of its products; workgroup = 128 tokens x 64 ranks, eight waves.
+//   * kDeep: for batches whose last round of those would leave CUs idle: a wave owns 16 tokens, 16 or 32 ranks
+//     and half of the channels, and keeps kProjectDeep steps of loads in flight; workgroup = 32 tokens.
+//   * kGram: the sources are the basis rows themselves, the channel steps dealt to four waves, and the FP64
+//     sums are stored as they are, G = Q Q^T.
+// Bound by the FP64 matrix rate; the next step's loads are issued before a step's products and the step body
+// has no branch, so their latency is covered.  The vector instructions do not hide under FP64 products, and the
+// rate depends on the operands' bits: products of full 53-bit operands alone reach 46-49 TFLOP/s, a large
 // library product 68.
+// bf16 [4680, 1536] at rank 96 (MI355X): one matrix 105 us with 64-token workgroups of one wave per 16 tokens
+// and loads in the step, 38 now (34 with four chains per element, whose partial sums a wave of kShared has no
+// registers for); 60 matrices 1563 us, 1396 with every wave converting its own basis operands, 1306 now.
 // ---------------------------------------------------------------------------------------------
 
 // Eight consecutive source elements as loaded, and as doubles.
@@ -426,14 +433,29 @@ __device__ __forceinline__ double eight_at(const Eight<DT>& e, int i) {
     else return static_cast<double>(half_bits<DT>((e.w[0][i >> 1] >> (16 * (i & 1))) & 0xffffu));
 }
 
+constexpr int kProjectDeep = 3;  // 4 and 6 measure the same
+
+enum class Project { kShared, kDeep, kGram };
+
+// Waves of a workgroup, tokens of a wave, and first channel of the second half.
+template <Project SHAPE>
+constexpr int kProjectWaves = SHAPE == Project::kShared ? 8 : 4;
+template <Project SHAPE>
+constexpr int kProjectTiles = SHAPE == Project::kShared ? 2 : 1;  // of 16 tokens
+__device__ __forceinline__ int project_middle(int channels) { return min(channels, 32 * (((channels + 31) / 32 + 1) / 2)); }
+
 // Order of the padded FP64 k x k matrices of the span kernels.
 __device__ __forceinline__ int padded_order(int rank) { return (rank + 15) & ~15; }
 
-template <int DT, int TB, int SPLIT, int NB, bool GRAM = false>
+template <int DT, Project SHAPE, int NB>
 __device__ __forceinline__ void project_ranks(const rch_fit_matrix* M, int channels, int r0, int64_t wt, int wave, int lane,
                                               double* shared) {
     constexpr int E = esize<DT>();
-    static_assert(!GRAM || (DT == RCH_DT_F16 && SPLIT > 1), "the basis Gram runs on fp16 rows, channels split");
+    constexpr bool GRAM = SHAPE == Project::kGram;
+    static_assert(!GRAM || DT == RCH_DT_F16, "the basis Gram runs on fp16 rows");
+    constexpr int TB = kProjectTiles<SHAPE>, kWaves = kProjectWaves<SHAPE>;
+    const int half = GRAM ? 0 : wave / (kWaves / 2), middle = project_middle(channels);
+    const int begin = half ? middle : 0, end = GRAM || half ? channels : middle;  // of this wave's channels
     const int rank = static_cast<int>(M->rank);
     const int64_t rows = GRAM ? rank : M->rows;
     const int g = lane >> 4, i16 = lane & 15;
@@ -451,25 +473,25 @@ __device__ __forceinline__ void project_ranks(const rch_fit_matrix* M, int chann
     Eight<DT> x_now[TB], x_next[TB];
     auto load_x = [&](int c0) __attribute__((always_inline)) {
         const int c = c0 + 8 * g;  // channels % 8 == 0: a group is whole or past the end
-        const uint32_t past = c < channels ? 0u : kOutOfRange;
+        const uint32_t past = c < end ? 0u : kOutOfRange;
 #pragma unroll
         for (int t = 0; t < TB; ++t) x_next[t] = load_eight<DT>(xs, (x_row[t] + static_cast<uint32_t>(c * E)) | past);
     };
     auto q_at = [&](int b, int c0, int first) __attribute__((always_inline)) {  // from channel `first` of a group
         const int c = c0 + 8 * g;
-        return (q_row[b] + static_cast<uint32_t>((c + first) * 2)) | (c < channels ? 0u : kOutOfRange);
+        return (q_row[b] + static_cast<uint32_t>((c + first) * 2)) | (c < end ? 0u : kOutOfRange);
     };
     d4 acc[TB][NB];
 #pragma unroll
     for (int t = 0; t < TB; ++t)
 #pragma unroll
         for (int b = 0; b < NB; ++b) acc[t][b] = d4{};
-    auto products = [&](auto&& basis) __attribute__((always_inline)) {  // basis(b, s): channel s of rank block b
+    auto products = [&](const Eight<DT> (&x)[TB], auto&& basis) __attribute__((always_inline)) {  // basis(b, s): channel s of rank block b
         double xv[TB][8];
 #pragma unroll
         for (int t = 0; t < TB; ++t)
 #pragma unroll
-            for (int s = 0; s < 8; ++s) xv[t][s] = eight_at<DT>(x_now[t], s);
+            for (int s = 0; s < 8; ++s) xv[t][s] = eight_at<DT>(x[t], s);
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
@@ -484,31 +506,78 @@ __device__ __forceinline__ void project_ranks(const rch_fit_matrix* M, int chann
 #pragma unroll
         for (int t = 0; t < TB; ++t) x_now[t] = x_next[t];
     };
-    if constexpr (SPLIT == 1) {  // wave w converts channels 2w, 2w + 1 of every group for all four waves
-        static_assert(kThreads == 256, "four waves share a step's eight channels");
+    d4 sum[NB];  // of the 16 tokens that this wave stores
+    if constexpr (SHAPE == Project::kShared) {  // wave w of a half converts channels 2w, 2w + 1 of every group for its four
+        static_assert(kWaves == 8, "four waves share a step's eight channels");
         constexpr int kStep = 8 * NB * 64;
+        const int pair_at = 2 * (wave & 3);
+        double* const staged = shared + 2 * half * kStep;
         uint32_t pair[NB];
         auto load_pair = [&](int c0) __attribute__((always_inline)) {
 #pragma unroll
-            for (int b = 0; b < NB; ++b) pair[b] = __builtin_amdgcn_raw_buffer_load_b32(qs, q_at(b, c0, 2 * wave), 0, 0);
+            for (int b = 0; b < NB; ++b) pair[b] = __builtin_amdgcn_raw_buffer_load_b32(qs, q_at(b, c0, pair_at), 0, 0);
         };
         auto stage = [&](int at) __attribute__((always_inline)) {
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
-                double* to = shared + at + (8 * b + 2 * wave) * 64 + lane;
+                double* to = staged + at + (8 * b + pair_at) * 64 + lane;
                 to[0] = static_cast<double>(half_bits<RCH_DT_F16>(pair[b] & 0xffffu));
                 to[64] = static_cast<double>(half_bits<RCH_DT_F16>(pair[b] >> 16));
             }
         };
-        load_x(0), load_pair(0);
+        load_x(begin), load_pair(begin);
         stage(0), advance();
         __syncthreads();
-        for (int c0 = 0, at = 0; c0 < channels; c0 += 32, at = kStep - at) {
-            load_x(c0 + 32), load_pair(c0 + 32);
-            products([&](int b, int s) { return shared[at + (8 * b + s) * 64 + lane]; });
-            stage(kStep - at), advance();  // this half was last read before the previous barrier
+        // Both halves take the first half's count of steps (a step past the end multiplies zeros).
+        for (int c = 0, at = 0; c < middle; c += 32, at = kStep - at) {
+            load_x(begin + c + 32), load_pair(begin + c + 32);
+            products(x_now, [&](int b, int s) { return staged[at + (8 * b + s) * 64 + lane]; });
+            stage(kStep - at), advance();  // this part was last read before the previous barrier
             __syncthreads();
         }
+        // Each half stores one of the two tiles: the other's sums go to the wave that shares the tokens.
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) shared[((wave * NB + b) * 4 + v) * 64 + lane] = half ? acc[0][b][v] : acc[1][b][v];
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                sum[b][v] = (half ? acc[1][b][v] : acc[0][b][v]) + shared[(((wave ^ 4) * NB + b) * 4 + v) * 64 + lane];
+        wt += 16 * half;
+    } else if constexpr (SHAPE == Project::kDeep) {
+        Eight<DT> x[kProjectDeep][TB];
+        Eight<RCH_DT_F16> q[kProjectDeep][NB];
+        auto load = [&](int c0, Eight<DT> (&x_to)[TB], Eight<RCH_DT_F16> (&q_to)[NB]) __attribute__((always_inline)) {
+            load_x(c0);
+#pragma unroll
+            for (int t = 0; t < TB; ++t) x_to[t] = x_next[t];
+#pragma unroll
+            for (int b = 0; b < NB; ++b) q_to[b] = load_eight<RCH_DT_F16>(qs, q_at(b, c0, 0));
+        };
+#pragma unroll
+        for (int d = 0; d < kProjectDeep; ++d) load(begin + 32 * d, x[d], q[d]);
+        for (int c0 = begin; c0 < end; c0 += 32 * kProjectDeep) {
+#pragma unroll
+            for (int d = 0; d < kProjectDeep; ++d) {  // a step past the end multiplies zeros
+                products(x[d], [&](int b, int s) { return eight_at<RCH_DT_F16>(q[d][b], s); });
+                load(c0 + 32 * (d + kProjectDeep), x[d], q[d]);
+            }
+        }
+        if (half) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) shared[(((wave & 1) * NB + b) * 4 + v) * 64 + lane] = acc[0][b][v];
+        }
+        __syncthreads();
+        if (half) return;
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) sum[b][v] = acc[0][b][v] + shared[((wave * NB + b) * 4 + v) * 64 + lane];
     } else {
         Eight<RCH_DT_F16> q_now[NB], q_next[NB];
         auto load_q = [&](int c0) __attribute__((always_inline)) {
@@ -521,50 +590,43 @@ __device__ __forceinline__ void project_ranks(const rch_fit_matrix* M, int chann
         };
         load_x(32 * wave), load_q(32 * wave);
         advance(), advance_q();
-        for (int c0 = 32 * wave; c0 < channels; c0 += 32 * SPLIT) {
-            load_x(c0 + 32 * SPLIT), load_q(c0 + 32 * SPLIT);
-            products([&](int b, int s) { return eight_at<RCH_DT_F16>(q_now[b], s); });
+        for (int c0 = 32 * wave; c0 < channels; c0 += 32 * kWaves) {
+            load_x(c0 + 32 * kWaves), load_q(c0 + 32 * kWaves);
+            products(x_now, [&](int b, int s) { return eight_at<RCH_DT_F16>(q_now[b], s); });
             advance(), advance_q();
         }
-    }
-    if constexpr (SPLIT > 1) {  // block b of every wave is added, in wave order, by wave b
+        // Block b of every wave is added, in wave order, by wave b.
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) shared[((b * SPLIT + wave) * 4 + v) * 64 + lane] = acc[0][b][v];
+            for (int v = 0; v < 4; ++v) shared[((b * kWaves + wave) * 4 + v) * 64 + lane] = acc[0][b][v];
         __syncthreads();
         if (wave >= NB) return;
-        d4 sum = d4{};
+        d4 entry = d4{};
 #pragma unroll
-        for (int w = 0; w < SPLIT; ++w)
+        for (int w = 0; w < kWaves; ++w)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) sum[v] += shared[((wave * SPLIT + w) * 4 + v) * 64 + lane];
-        acc[0][0] = sum;
-        if constexpr (GRAM) {  // rows and columns past the rank are zeros
-            const int kp = padded_order(rank), k = r0 + 16 * wave + i16;
+            for (int v = 0; v < 4; ++v) entry[v] += shared[((wave * kWaves + w) * 4 + v) * 64 + lane];
+        const int kp = padded_order(rank), k = r0 + 16 * wave + i16;  // rows and columns past the rank are zeros
 #pragma unroll
-            for (int v = 0; v < 4; ++v) gout<double>(M->gram_ptr)[(wt + g + 4 * v) * kp + k] = sum[v];
-            return;
-        }
+        for (int v = 0; v < 4; ++v) gout<double>(M->gram_ptr)[(wt + g + 4 * v) * kp + k] = entry[v];
+        return;
     }
     RCH_GLOBAL float* out = gout<float>(M->coef_ptr);
     unsigned int* ext = reinterpret_cast<unsigned int*>(M->extrema_ptr);
 #pragma unroll
-    for (int b = 0; b < (SPLIT > 1 ? 1 : NB); ++b) {
-        const int k = r0 + 16 * (SPLIT > 1 ? wave : b) + i16;  // this lane's rank
+    for (int b = 0; b < NB; ++b) {
+        const int k = r0 + 16 * b + i16;  // this lane's rank
         uint32_t lo = 0u, hi = 0u;
 #pragma unroll
-        for (int t = 0; t < TB; ++t) {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int64_t token = wt + 16 * t + g + 4 * v;
-                const float value = static_cast<float>(acc[t][b][v]);
-                if (token < rows) {
-                    if (k < rank) out[token * M->coef_stride + k] = value;  // 16 lanes: 64 contiguous bytes of a row
-                    const uint32_t key = order_key(value);
-                    lo = ~key > lo ? ~key : lo;
-                    hi = key > hi ? key : hi;
-                }
+        for (int v = 0; v < 4; ++v) {
+            const int64_t token = wt + g + 4 * v;
+            const float value = static_cast<float>(sum[b][v]);
+            if (token < rows) {
+                if (k < rank) out[token * M->coef_stride + k] = value;  // 16 lanes: 64 contiguous bytes of a row
+                const uint32_t key = order_key(value);
+                lo = ~key > lo ? ~key : lo;
+                hi = key > hi ? key : hi;
             }
         }
         if (ext) {
@@ -582,35 +644,36 @@ __device__ __forceinline__ void project_ranks(const rch_fit_matrix* M, int chann
     }
 }
 
-// Tokens of a project_kernel workgroup.
-template <int TB, int SPLIT>
-constexpr int kProjectTokens = 16 * TB * (SPLIT > 1 ? 1 : kThreads / 64);
+// Tokens of a project_kernel workgroup: its halves' waves share them.
+template <Project SHAPE>
+constexpr int kProjectTokens = 16 * kProjectTiles<SHAPE> * kProjectWaves<SHAPE> / 2;
 
-template <int DT, int TB, int SPLIT>
-__global__ void __launch_bounds__(kThreads, 2) project_kernel(const rch_fit_matrix* __restrict__ mats, int channels,
-                                                              int chunk) {
-    static_assert(SPLIT == 1 || (SPLIT == kThreads / 64 && TB == 1), "all waves split the channels, or none");
-    // Partial sums of up to four rank blocks, or the basis operands of two steps.
-    __shared__ double shared[SPLIT > 1 ? 4 * SPLIT * 4 * 64 : 2 * 8 * 4 * 64];
+template <int DT, Project SHAPE>
+__global__ void __launch_bounds__(64 * kProjectWaves<SHAPE>, 4) project_kernel(const rch_fit_matrix* __restrict__ mats,
+                                                                              int channels, int chunk) {
+    constexpr bool kShared = SHAPE == Project::kShared;
+    // The basis operands of two steps of four rank blocks per half, then the exchanged sums: the same size.
+    __shared__ double shared[kShared ? 2 * 2 * 8 * 4 * 64 : 2 * 2 * 4 * 64];
     const rch_fit_matrix* M = mats + blockIdx.z;
     const int rank = static_cast<int>(M->rank);
-    const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kProjectTokens<TB, SPLIT>;
-    const int r0 = blockIdx.y * chunk;  // chunk: 16, 32, 48 or 64 ranks
+    const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kProjectTokens<SHAPE>;
+    const int r0 = blockIdx.y * chunk;  // chunk: 16 or 32 ranks, kShared also 48 or 64
     if (t0 >= M->rows || r0 >= rank) return;  // whole workgroup
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int64_t wt = SPLIT > 1 ? t0 : t0 + 16 * TB * wave;  // first token of this wave
-    switch (min(chunk >> 4, (rank - r0 + 15) >> 4)) {  // 16-rank blocks of this chunk (uniform)
-        case 1: project_ranks<DT, TB, SPLIT, 1>(M, channels, r0, wt, wave, lane, shared); break;
-        case 2: project_ranks<DT, TB, SPLIT, 2>(M, channels, r0, wt, wave, lane, shared); break;
-        case 3: project_ranks<DT, TB, SPLIT, 3>(M, channels, r0, wt, wave, lane, shared); break;
-        default: project_ranks<DT, TB, SPLIT, 4>(M, channels, r0, wt, wave, lane, shared); break;
+    const int64_t wt = t0 + 16 * kProjectTiles<SHAPE> * (wave % (kProjectWaves<SHAPE> / 2));  // first token of this wave
+    const int blocks = min(chunk >> 4, (rank - r0 + 15) >> 4);  // 16-rank blocks of this chunk (uniform)
+    if (blocks == 1) project_ranks<DT, SHAPE, 1>(M, channels, r0, wt, wave, lane, shared);
+    else if (!kShared || blocks == 2) project_ranks<DT, SHAPE, 2>(M, channels, r0, wt, wave, lane, shared);
+    if constexpr (kShared) {
+        if (blocks == 3) project_ranks<DT, SHAPE, 3>(M, channels, r0, wt, wave, lane, shared);
+        else if (blocks >= 4) project_ranks<DT, SHAPE, 4>(M, channels, r0, wt, wave, lane, shared);
     }
 }
 
 // ---------------------------------------------------------------------------------------------
 // Residual energies on v_mfma_f64_16x16x4f64: D[m = token][n = channel] = sum_k P[token][k] Q[k][c].
-// Workgroup = some tokens of one matrix and every gridDim.z-th set of 64-channel groups.  A group is four 16 x 16 blocks per 16 tokens whose columns interleave: column i of block b is channel
-// 4i + b of the group, so after the four blocks lane l (i = l % 16, g = l / 16) holds channels 4i ..
+// Workgroup = some tokens of one matrix and every gridDim.z-th part of its 64-channel groups.  A group is
+// four 16 x 16 blocks per 16 tokens whose columns interleave: column i of block b is channel 4i + b of the group, so after the four blocks lane l (i = l % 16, g = l / 16) holds channels 4i ..
 // 4i + 3 of tokens g + 4v (v = 0..3, the f64 accumulator's row (l / 16) + 4v): X and the residual move
 // as 4-channel vectors, 16 lanes covering 64 contiguous channels of a row.  Per 16-rank step a lane
 // takes P[token i][4g .. 4g + 3] (the A operand; MFMA step j takes rank 4g + j) and, for each j,
@@ -624,9 +687,9 @@ __global__ void __launch_bounds__(kThreads, 2) project_kernel(const rch_fit_matr
 // Bound by the FP64 matrix rate (rank 0, the source energy alone: by HBM), with the vector instructions
 // beside it: they do not hide under FP64 products.  The next step's operands are loaded before a step's
 // products and a group's source elements before all of its products.
-// One bf16 matrix [4680, 1536] at rank 96: 137 -> 40 us; 60 matrices at rank 96: 1808 us with 16-token
-// workgroups, 1527 with 32-token ones of unshared operands, 1450 now (57 TFLOP/s); ranks 32 to 128 in one
-// batch: 1350 -> 1290 us; 8 matrices [4680, 4096] at ranks 256 and 512: 2394 -> 2184 us; source energy of one: 29 -> 18 us.
+// bf16 [4680, 1536] (MI355X, with the totals): one matrix at rank 96 137 -> 42 us; 60 at rank 96 1808 us with
+// 16-token workgroups, 1527 with 32-token ones of unshared operands, 1450 now (57 TFLOP/s); 60 at ranks 32 to
+// 128 1350 -> 1285 us; source energy alone of one 8 us, of 60 169.
 // ---------------------------------------------------------------------------------------------
 
 // The 4 channels of tokens g + 4v (v = 0..3) of a lane's 64-channel group, as raw 16-bit pairs
@@ -637,42 +700,51 @@ struct SourceQuad {
     word w[4];
 };
 
-__device__ __forceinline__ void residual_total(const rch_fit_matrix* M, double src, double err,
-                                               double (*part)[kThreads / 64], int wave, int lane) {
-    // Fixed-order reduction: butterfly within the wave, then waves 0..3 in order.
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-        src += __shfl_xor(src, d);
-        err += __shfl_xor(err, d);
-    }
-    if (lane == 0) {
-        part[0][wave] = src;
-        part[1][wave] = err;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double a = 0.0, b = 0.0;
-        for (int w = 0; w < kThreads / 64; ++w) {
-            a += part[0][w];
-            b += part[1][w];
-        }
-        const float smax = __uint_as_float(*gin<unsigned int>(M->absmax_ptr));
-        if (smax != 0.0f) {
-            const double s = static_cast<double>(smax);
-            a = a / s / s;
-            b = b / s / s;
-        }
-        RCH_GLOBAL double* out = gout<double>(M->partial_ptr) + 2 * (gridDim.z * blockIdx.x + blockIdx.z);
-        out[0] = a;
-        out[1] = b;
-    }
+// A partial energy sums 16 tokens and one part of the channels, a run of 64-channel groups, whatever the
+// shape of the launch: a lane adds its elements in order, then the wave its lanes.  So the bits of a matrix's
+// energies do not depend on the batch that it is measured in, which chooses the shape.
+__host__ __device__ __forceinline__ int residual_groups(int channels) { return (channels + 63) >> 6; }
+__host__ __device__ __forceinline__ int residual_part_groups(int channels) {
+    return (residual_groups(channels) + RCH_RESIDUAL_PARTS - 1) / RCH_RESIDUAL_PARTS;
+}
+__host__ __device__ __forceinline__ int residual_parts(int channels) {
+    const int each = residual_part_groups(channels);
+    return (residual_groups(channels) + each - 1) / each;
 }
 
-// Tokens of a residual_kernel workgroup, and channels that its waves cover at once.
+// v plus the value `Turn` lanes on within the row of 16 lanes.
+template <int Turn>
+__device__ __forceinline__ double add_turned(double v) {
+    const u2 w = __builtin_bit_cast(u2, v);
+    const u2 o = {static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(w[0]), 0x120 + Turn, 0xf, 0xf, true)),
+                  static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(w[1]), 0x120 + Turn, 0xf, 0xf, true))};
+    return v + __builtin_bit_cast(double, o);
+}
+
+// Sums over the wave of the TB tiles' two energies: lanes 0-15 and 16-31 return src[0] and src[TB - 1], lanes
+// 32-47 and 48-63 err[0] and err[TB - 1].  Per value a tree over lane distances 32, 16, 8, 4, 2, 1.
+template <int TB>
+__device__ __forceinline__ double residual_sums(const double (&src)[TB], const double (&err)[TB], int lane) {
+    double half[TB];
+#pragma unroll
+    for (int t = 0; t < TB; ++t) {  // the lower half keeps src, the upper half err
+        const double give = lane < 32 ? err[t] : src[t];
+        half[t] = (lane < 32 ? src[t] : err[t]) + __shfl_xor(give, 32);
+    }
+    const bool odd = lane & 16;
+    const double give = odd ? half[0] : half[TB - 1];
+    double sum = (odd ? half[TB - 1] : half[0]) + __shfl_xor(give, 16);
+    sum = add_turned<8>(sum);
+    sum = add_turned<4>(sum);
+    sum = add_turned<2>(sum);
+    return add_turned<1>(sum);
+}
+
+// Tokens of a residual_kernel workgroup, and channel parts that its waves work on at once.
 template <bool SHARED>
 constexpr int kResidualTokens = SHARED ? 32 * (kThreads / 64) : 16;
 template <bool SHARED>
-constexpr int kResidualChannels = SHARED ? 64 : 64 * (kThreads / 64);
+constexpr int kResidualAtOnce = SHARED ? 1 : kThreads / 64;
 
 template <int DT, bool SHARED>
 __global__ void __launch_bounds__(kThreads, 2) residual_kernel(const rch_fit_matrix* __restrict__ mats, int channels) {
@@ -680,7 +752,6 @@ __global__ void __launch_bounds__(kThreads, 2) residual_kernel(const rch_fit_mat
     constexpr int kStep = 16 * 64;  // basis operands of a 16-rank step, [j: rank 4g + j][block][lane]
     static_assert(kWaves == 4, "wave j shares the rows of ranks 4g + j");
     __shared__ double staged[SHARED ? 2 * kStep : 1];
-    __shared__ double part[2][kWaves];
     const rch_fit_matrix* M = mats + blockIdx.y;
     const int64_t rows = M->rows;
     const int rank = static_cast<int>(M->rank);
@@ -751,10 +822,10 @@ __global__ void __launch_bounds__(kThreads, 2) residual_kernel(const rch_fit_mat
         if constexpr (SHARED) __syncthreads();
     };
 
-    double src = 0.0, err = 0.0;
+    double src[TB], err[TB];
     d4 acc[TB][4];
     // e = x - r per element: FP64 sums of x^2 and e^2, optional fp32 store.
-    auto finish = [&](int c64, const SourceQuad<DT> (&x)[TB]) __attribute__((always_inline)) {
+    auto finish = [&](auto source_only, int c64, const SourceQuad<DT> (&x)[TB]) __attribute__((always_inline)) {
         const int c = c64 + 4 * i16;
 #pragma unroll
         for (int t = 0; t < TB; ++t)
@@ -766,9 +837,13 @@ __global__ void __launch_bounds__(kThreads, 2) residual_kernel(const rch_fit_mat
                     double a;
                     if constexpr (DT == RCH_DT_F32) a = static_cast<double>(__uint_as_float(x[t].w[v][b]));
                     else a = static_cast<double>(half_bits<DT>((x[t].w[v][b >> 1] >> (16 * (b & 1))) & 0xffffu));
-                    e[b] = a - acc[t][b][v];
-                    src = fma(a, a, src);
-                    err = fma(e[b], e[b], err);
+                    src[t] = fma(a, a, src[t]);
+                    if constexpr (source_only.value) {
+                        e[b] = a;
+                    } else {
+                        e[b] = a - acc[t][b][v];
+                        err[t] = fma(e[b], e[b], err[t]);
+                    }
                 }
                 const int token = 16 * t + g + 4 * v;
                 if (resid && c < channels && token < left) {
@@ -778,14 +853,42 @@ __global__ void __launch_bounds__(kThreads, 2) residual_kernel(const rch_fit_mat
                 }
             }
     };
-    const int first = kResidualChannels<SHARED> * static_cast<int>(blockIdx.z) + (SHARED ? 0 : 64 * wave);
-    const int stride = kResidualChannels<SHARED> * static_cast<int>(gridDim.z);
+    const int parts = residual_parts(channels), each = residual_part_groups(channels);
+    const int stride = kResidualAtOnce<SHARED> * static_cast<int>(gridDim.z);
+    auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < TB; ++t) src[t] = err[t] = 0.0;
+    };
+    // The wave's parts are stored together at the end, lane i16 the i16-th: a store in the loop would hold up the
+    // loads behind it, which complete in order.
+    double kept = 0.0;
+    int done = 0;
+    auto end_part = [&]() __attribute__((always_inline)) {
+        const double sum = residual_sums<TB>(src, err, lane);
+        kept = i16 == done ? sum : kept;
+        ++done;
+        clear();
+    };
+    // The 64-channel groups of this wave's parts in turn; past the channels at the end.
+    auto part_end = [&](int part) __attribute__((always_inline)) { return min(64 * each * (part + 1), channels); };
+    auto next_group = [&](int& part, int& c64) __attribute__((always_inline)) {
+        c64 += 64;
+        if (c64 < part_end(part)) return;
+        part += stride;
+        c64 = part < parts ? 64 * each * part : channels;
+    };
+    const int first_part = kResidualAtOnce<SHARED> * static_cast<int>(blockIdx.z) + (SHARED ? 0 : wave);
+    const int first = first_part < parts ? 64 * each * first_part : channels;
+    int part = first_part;
+    int part_next = part, next = first;  // of the group after the current one
+    next_group(part_next, next);
     SourceQuad<DT> x_now[TB];
+    clear();
     if (rank > 0) {
         load_operands(first, 0);
         advance(0, 0);
         int at = 0;
-        for (int c64 = first; c64 < channels; c64 += stride) {
+        for (int c64 = first; c64 < channels;) {
             load_source(c64, x_now);  // in flight under the group's products
 #pragma unroll
             for (int t = 0; t < TB; ++t)
@@ -794,7 +897,7 @@ __global__ void __launch_bounds__(kThreads, 2) residual_kernel(const rch_fit_mat
             for (int k0 = 0; k0 < rank; k0 += 16) {
                 const bool last = k0 + 16 >= rank;
                 const int k_next = last ? 0 : k0 + 16;
-                load_operands(last ? c64 + stride : c64, k_next);
+                load_operands(last ? next : c64, k_next);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     double pa[TB];
@@ -812,43 +915,77 @@ __global__ void __launch_bounds__(kThreads, 2) residual_kernel(const rch_fit_mat
                 at = kStep - at;  // this half was last read before the previous barrier
                 advance(k_next, at);
             }
-            finish(c64, x_now);
+            finish(std::false_type{}, c64, x_now);
+            if (c64 + 64 >= part_end(part)) end_part();  // uniform
+            part = part_next, c64 = next;
+            next_group(part_next, next);
         }
-    } else {  // the source energy alone: one group ahead
-#pragma unroll
-        for (int t = 0; t < TB; ++t)
-#pragma unroll
-            for (int b = 0; b < 4; ++b) acc[t][b] = d4{};
+    } else {  // the source energy alone (the residual is the source): one group ahead
         SourceQuad<DT> x_next[TB];
         load_source(first, x_now);
-        for (int c64 = first; c64 < channels; c64 += stride) {
-            load_source(c64 + stride, x_next);
-            finish(c64, x_now);
+        for (int c64 = first; c64 < channels;) {
+            load_source(next, x_next);
+            finish(std::true_type{}, c64, x_now);
+            if (c64 + 64 >= part_end(part)) {
+#pragma unroll
+                for (int t = 0; t < TB; ++t) err[t] = src[t];
+                end_part();
+            }
+            part = part_next, c64 = next;
+            next_group(part_next, next);
 #pragma unroll
             for (int t = 0; t < TB; ++t) x_now[t] = x_next[t];
         }
     }
-    residual_total(M, src, err, part, wave, lane);
+    const int64_t tile = (wt >> 4) + (TB > 1 ? g & 1 : 0);  // residual_sums: 16 lanes per tile and energy
+    if (i16 < done && (TB > 1 || !(g & 1)) && 16 * tile < rows)
+        gout<double>(M->partial_ptr)[2 * (tile * parts + first_part + stride * i16) + (g >> 1)] = kept;
 }
 
-// Sum of the partials of each matrix (`splits` per `tokens` rows): one wave per matrix, lane l takes
-// partials l, l + 64, ... in order, then a butterfly -- the same order whatever the launch.
-__global__ void __launch_bounds__(64) energy_total_kernel(const rch_fit_matrix* __restrict__ mats, int tokens,
-                                                          int splits) {
+// Sum of the partials of each matrix, one workgroup per matrix: thread t takes partials t, t + 1024, ... in
+// order, then its wave's lanes and the waves in order; divided by s^2 (s = max|X|).  The order depends on the
+// matrix's rows and channels alone.
+constexpr int kTotalThreads = 1024;
+typedef double d2 __attribute__((ext_vector_type(2)));
+
+__global__ void __launch_bounds__(kTotalThreads) energy_total_kernel(const rch_fit_matrix* __restrict__ mats, int channels) {
+    constexpr int kWaves = kTotalThreads / 64;
+    __shared__ double sums[2][kWaves];
     const rch_fit_matrix* M = mats + blockIdx.x;
-    const int64_t tiles = (M->rows + tokens - 1) / tokens * splits;
-    const RCH_GLOBAL double* p = gin<double>(M->partial_ptr);
+    const int64_t count = ((M->rows + 15) >> 4) * residual_parts(channels);
+    const RCH_GLOBAL d2* p = gin<d2>(M->partial_ptr);
     double a = 0.0, b = 0.0;
-    for (int64_t t = threadIdx.x; t < tiles; t += 64) {
-        a += p[2 * t];
-        b += p[2 * t + 1];
+    for (int64_t t0 = threadIdx.x; t0 < count; t0 += 4 * kTotalThreads) {
+        d2 v[4];  // four loads in flight
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = t0 + i * kTotalThreads < count ? p[t0 + i * kTotalThreads] : d2{};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            a += v[i][0];
+            b += v[i][1];
+        }
     }
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) {
         a += __shfl_xor(a, d);
         b += __shfl_xor(b, d);
     }
+    if ((threadIdx.x & 63) == 0) {
+        sums[0][threadIdx.x >> 6] = a;
+        sums[1][threadIdx.x >> 6] = b;
+    }
+    __syncthreads();
     if (threadIdx.x == 0) {
+        for (int w = 1; w < kWaves; ++w) {
+            a += sums[0][w];
+            b += sums[1][w];
+        }
+        const float smax = __uint_as_float(*gin<unsigned int>(M->absmax_ptr));
+        if (smax != 0.0f) {
+            const double s = static_cast<double>(smax);
+            a = a / s / s;
+            b = b / s / s;
+        }
         RCH_GLOBAL double* out = gout<double>(M->energy_ptr);
         out[0] = a;
         out[1] = b;
@@ -1151,14 +1288,14 @@ __global__ void __launch_bounds__(kCholThreads) cholesky_inverse_kernel(const do
 // ---------------------------------------------------------------------------------------------
 
 __global__ void __launch_bounds__(kThreads) basis_gram_kernel(const rch_fit_matrix* __restrict__ mats, int channels) {
-    __shared__ double partial[4 * 4 * 4 * 64];
+    __shared__ double partial[2 * 4 * 4 * 64];  // the four waves' sums of two 16-column blocks
     const rch_fit_matrix* M = mats + blockIdx.z;
     const int kp = padded_order(static_cast<int>(M->rank));
     const int t0 = 16 * blockIdx.x, r0 = 32 * blockIdx.y;
     if (t0 >= kp || r0 >= kp) return;  // whole workgroup
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (r0 + 16 < kp) project_ranks<RCH_DT_F16, 1, 4, 2, true>(M, channels, r0, t0, wave, lane, partial);
-    else project_ranks<RCH_DT_F16, 1, 4, 1, true>(M, channels, r0, t0, wave, lane, partial);
+    if (r0 + 16 < kp) project_ranks<RCH_DT_F16, Project::kGram, 2>(M, channels, r0, t0, wave, lane, partial);
+    else project_ranks<RCH_DT_F16, Project::kGram, 1>(M, channels, r0, t0, wave, lane, partial);
 }
 
 __global__ void __launch_bounds__(kCholThreads) basis_terms_kernel(const rch_fit_matrix* __restrict__ mats) {
@@ -1262,7 +1399,17 @@ __global__ void __launch_bounds__(kCholThreads) basis_terms_kernel(const rch_fit
 constexpr int kSpanThreads = 512;
 constexpr int kSpanWaves = kSpanThreads / 64;
 constexpr int kSpanTokens = 32;  // tokens staged at a time
+constexpr int kSpanRange = 96;   // fewest tokens of a range
 constexpr int kSpanTiles = (kCholBlocks * (kCholBlocks + 1) / 2 + kSpanWaves - 1) / kSpanWaves;  // per wave
+
+// Tokens of a range (one workgroup, one partial sum), by the matrix's rows alone: its trace then has the same
+// bits in every batch.  96 tokens or, beyond RCH_SPAN_SPLITS of those, an equal share: one matrix at rank 96
+// takes 118 us (all four launches; 64 tokens 117, 256 125), 60 at ranks 32 to 128 283 (300, 291).
+__device__ __forceinline__ int64_t span_range(int64_t rows) {
+    const int64_t share = (rows + RCH_SPAN_SPLITS - 1) / RCH_SPAN_SPLITS;
+    const int64_t whole = (share + kSpanTokens - 1) / kSpanTokens * kSpanTokens;
+    return whole > kSpanRange ? whole : kSpanRange;
+}
 
 // Workgroup (token range, matrix): the 16 x 16 tiles (ti <= tj) of C are dealt to the waves; 32 tokens
 // of P at a time are staged in LDS as doubles, the next 32 loaded meanwhile.
@@ -1275,9 +1422,9 @@ __global__ void __launch_bounds__(kSpanThreads) span_trace_kernel(const rch_fit_
     const int tiles = blocks * (blocks + 1) / 2;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int i16 = lane & 15, g = lane >> 4;
-    const int64_t share = (M->rows + gridDim.x - 1) / gridDim.x;
-    const int64_t per = (share + kSpanTokens - 1) / kSpanTokens * kSpanTokens;
+    const int64_t per = span_range(M->rows);
     const int64_t begin = blockIdx.x * per, end = begin + per < M->rows ? begin + per : M->rows;
+    if (begin >= M->rows) return;  // whole workgroup
     int ti[kSpanTiles], tj[kSpanTiles];
     d4 acc[kSpanTiles];
 #pragma unroll
@@ -1345,13 +1492,15 @@ __global__ void __launch_bounds__(kSpanThreads) span_trace_kernel(const rch_fit_
 }
 
 // The span trace of each matrix from its workgroups' sums, in order (0 when G is not positive definite).
-__global__ void __launch_bounds__(64) span_total_kernel(const rch_fit_matrix* __restrict__ mats, int n, int splits) {
+__global__ void __launch_bounds__(64) span_total_kernel(const rch_fit_matrix* __restrict__ mats, int n) {
     const int mat = blockIdx.x * 64 + threadIdx.x;
     if (mat >= n) return;
     const rch_fit_matrix* M = mats + mat;
     RCH_GLOBAL double* out = gout<double>(M->energy_ptr);
+    const int64_t per = span_range(M->rows);
+    const int ranges = static_cast<int>((M->rows + per - 1) / per);
     double sum = 0.0;
-    for (int s = 0; s < splits; ++s) sum += gin<double>(M->partial_ptr)[s];
+    for (int s = 0; s < ranges; ++s) sum += gin<double>(M->partial_ptr)[s];
     out[0] = out[1] == 0.0 ? sum : 0.0;
 }
 
@@ -1408,19 +1557,27 @@ __global__ void __launch_bounds__(256) gaussian_kernel(const rch_gauss_job* __re
     }
 }
 
-// Measured on [n x 4680, 1536] bf16 (MI355X, host-side upload included): the projection's 128-token
-// workgroups beat the channel-split ones at 2220 workgroups (60 matrices, rank 32: 514 / 533 us) and lose
-// at 592 (8 matrices, rank 96: 254 / 224 us); the residual's shared form against its 16-token one at rank
-// 96: 123 / 140 us at 588 groups (4 matrices), 78 / 80 at 294, 55 / 51 at 147 (one matrix).
-constexpr int64_t kProjectWholeGroups = 2000;
+// The projection's 128-token workgroups run in rounds of one per CU.  They win while the last round is nearly
+// full, else the finer shape, n matrices [4680, 1536] of bf16 (MI355X, us, kShared / kDeep; groups of kShared in
+// brackets):
+//   rank 96: 3 [222] 85 / 90, 4 [296] 153 / 107, 6 [444] 154 / 161, 8 [592] 227 / 206, 10 [740] 226 / 259,
+//            12 [888] 297 / 302, 24 [1776] 514 / 596, 60 [4440] 1306 / 1465;
+//   rank 32: 12 [444] 112 / 108, 20 [740] 165 / 178, 24 [888] 216 / 207, 30 [1110] 266 / 262, 60 [2220] 470 / 501;
+//   fp32, rank 96: 8 225 / 205, 10 233 / 259, 12 299 / 310.
+// In the finer shape 16-rank chunks balance few waves better, and 32-rank ones convert less: 38 / 38 us at one
+// matrix of rank 96 (1758 tiles of 16 x 16), 62 / 65 at 3516, 113 / 107 at 7032; [390, 1536]: 12 / 19.
+constexpr int64_t kChipCus = 256, kProjectNarrowTiles = 6000;
+// The residual's 128-token form against the 16-token one, in 32-token groups: rank 96 49 / 41 us at 147 (one
+// matrix), 66 / 64 at 294, 91 / 94 at 441, 104 / 117 at 588, 207 / 243 at 1176; rank 32 31 / 29 at 294, 47 / 49 at
+// 588, 87 / 96 at 1176; fp32 the same within 2 us.  The source energy alone would stay with the 16-token form (60
+// matrices 169 / 161), but one rule serves both.
+static_assert(RCH_RESIDUAL_PARTS <= 16, "a wave keeps its parts' sums in 16 lanes");
 constexpr int64_t kResidualSharedGroups = 500;  // of 32 tokens
-// Workgroups that the channel splits aim at, and the fewest parts of the 128-token ones, which are long and
-// at mixed ranks unequal (60 matrices at ranks 32 to 128: one part 1400 us, two 1304, three 1285, four 1270;
-// more parts cost a batch without bases, whose workgroups then end before their loads overlap: 24 matrices 72
-// us at three parts, 84 at seven).
-constexpr int64_t kResidualSplitAim = 2000, kResidualSharedSplits = 3;
+// Workgroups that the channel splits aim at, and the fewest and most splits of the 128-token ones, which are
+// long and at mixed ranks unequal (60 matrices at ranks 32 to 128: one 1415 us, three 1288, six 1276; a batch
+// without bases, whose workgroups then end before their loads overlap, takes 169 at three and 191 at six).
+constexpr int64_t kResidualSplitAim = 2000, kResidualSharedSplits = 3, kResidualSharedMost = 8;
 constexpr int64_t kResidualSplits = 4;  // of 16-token tiles: a wave's first loads then serve one or two groups
-static_assert(kResidualSplits <= RCH_RESIDUAL_SPLITS, "partials are allocated for RCH_RESIDUAL_SPLITS parts");
 
 int check_matrices(const rch_fit_matrix* mats, int n, int channels, const char* what) {
     if (!mats || n <= 0 || n > 65535) return fail(RCH_E_CONFIG, "%s: 1 <= n_mats <= 65535 required", what);
@@ -1482,25 +1639,23 @@ int rch_fit_project(const rch_fit_matrix* mats_dev, int n_mats, int channels, in
     // The fewest rank chunks of at most 64 ranks, as equal as 16-rank blocks allow.
     const int blocks = (max_rank + 15) / 16;
     int chunks = (blocks + 3) / 4, chunk = 16 * ((blocks + chunks - 1) / chunks);
-    // 128-token workgroups while they fill the chip several times over; fewer leave CUs idle for most
-    // of the launch (one matrix [4680, 1536] at rank 96 is 74 of them), so the channel-split shape
-    // runs, in chunks of 32 ranks.
-    if ((max_rows + 127) / 128 * chunks * n_mats >= kProjectWholeGroups) {
+    const int64_t groups = (max_rows + 127) / 128 * chunks * n_mats, rounds = (groups + kChipCus - 1) / kChipCus;
+    if (7 * groups >= 6 * kChipCus * rounds) {
         const dim3 grid(static_cast<unsigned>((max_rows + 127) / 128), static_cast<unsigned>(chunks), z);
         switch (src_dtype) {
-            case RCH_DT_BF16: hipLaunchKernelGGL((project_kernel<RCH_DT_BF16, 2, 1>), grid, dim3(kThreads), 0, s, mats_dev, channels, chunk); break;
-            case RCH_DT_F16: hipLaunchKernelGGL((project_kernel<RCH_DT_F16, 2, 1>), grid, dim3(kThreads), 0, s, mats_dev, channels, chunk); break;
-            case RCH_DT_F32: hipLaunchKernelGGL((project_kernel<RCH_DT_F32, 2, 1>), grid, dim3(kThreads), 0, s, mats_dev, channels, chunk); break;
+            case RCH_DT_BF16: hipLaunchKernelGGL((project_kernel<RCH_DT_BF16, Project::kShared>), grid, dim3(64 * kProjectWaves<Project::kShared>), 0, s, mats_dev, channels, chunk); break;
+            case RCH_DT_F16: hipLaunchKernelGGL((project_kernel<RCH_DT_F16, Project::kShared>), grid, dim3(64 * kProjectWaves<Project::kShared>), 0, s, mats_dev, channels, chunk); break;
+            case RCH_DT_F32: hipLaunchKernelGGL((project_kernel<RCH_DT_F32, Project::kShared>), grid, dim3(64 * kProjectWaves<Project::kShared>), 0, s, mats_dev, channels, chunk); break;
             default: return fail(RCH_E_CONFIG, "rch_fit_project: source dtype must be bf16, f16 or f32");
         }
     } else {
-        chunk = 32;
-        chunks = (max_rank + 31) / 32;
-        const dim3 grid(static_cast<unsigned>((max_rows + 15) / 16), static_cast<unsigned>(chunks), z);
+        chunk = (max_rows + 15) / 16 * blocks * n_mats < kProjectNarrowTiles ? 16 : 32;
+        chunks = (max_rank + chunk - 1) / chunk;
+        const dim3 grid(static_cast<unsigned>((max_rows + 31) / 32), static_cast<unsigned>(chunks), z);
         switch (src_dtype) {
-            case RCH_DT_BF16: hipLaunchKernelGGL((project_kernel<RCH_DT_BF16, 1, 4>), grid, dim3(kThreads), 0, s, mats_dev, channels, chunk); break;
-            case RCH_DT_F16: hipLaunchKernelGGL((project_kernel<RCH_DT_F16, 1, 4>), grid, dim3(kThreads), 0, s, mats_dev, channels, chunk); break;
-            case RCH_DT_F32: hipLaunchKernelGGL((project_kernel<RCH_DT_F32, 1, 4>), grid, dim3(kThreads), 0, s, mats_dev, channels, chunk); break;
+            case RCH_DT_BF16: hipLaunchKernelGGL((project_kernel<RCH_DT_BF16, Project::kDeep>), grid, dim3(64 * kProjectWaves<Project::kDeep>), 0, s, mats_dev, channels, chunk); break;
+            case RCH_DT_F16: hipLaunchKernelGGL((project_kernel<RCH_DT_F16, Project::kDeep>), grid, dim3(64 * kProjectWaves<Project::kDeep>), 0, s, mats_dev, channels, chunk); break;
+            case RCH_DT_F32: hipLaunchKernelGGL((project_kernel<RCH_DT_F32, Project::kDeep>), grid, dim3(64 * kProjectWaves<Project::kDeep>), 0, s, mats_dev, channels, chunk); break;
             default: return fail(RCH_E_CONFIG, "rch_fit_project: source dtype must be bf16, f16 or f32");
         }
     }
@@ -1516,11 +1671,11 @@ int rch_fit_residual(const rch_fit_matrix* mats_dev, int n_mats, int channels, i
     // 16-token ones, the channels split as well.
     const bool shared = (max_rows + 31) / 32 * n_mats >= kResidualSharedGroups;
     const int tokens = shared ? kResidualTokens<true> : kResidualTokens<false>;
-    const int channel_part = shared ? kResidualChannels<true> : kResidualChannels<false>;
+    const int at_once = shared ? kResidualAtOnce<true> : kResidualAtOnce<false>;
     const int64_t groups = (max_rows + tokens - 1) / tokens * n_mats;
     const int64_t wanted = std::max<int64_t>((kResidualSplitAim + groups - 1) / groups, shared ? kResidualSharedSplits : 1);
-    const int64_t most = std::min<int64_t>((channels + channel_part - 1) / channel_part,
-                                           shared ? RCH_RESIDUAL_SPLITS : kResidualSplits);
+    const int64_t most = std::min<int64_t>((residual_parts(channels) + at_once - 1) / at_once,
+                                           shared ? kResidualSharedMost : kResidualSplits);
     const int splits = static_cast<int>(std::min(wanted, most));
     const dim3 grid(static_cast<unsigned>((max_rows + tokens - 1) / tokens), static_cast<unsigned>(n_mats),
                     static_cast<unsigned>(splits));
@@ -1540,7 +1695,7 @@ int rch_fit_residual(const rch_fit_matrix* mats_dev, int n_mats, int channels, i
         default: return fail(RCH_E_CONFIG, "rch_fit_residual: source dtype must be bf16, f16 or f32");
     }
     if (int status = check_launch("rch_fit_residual")) return status;
-    hipLaunchKernelGGL(energy_total_kernel, dim3(n_mats), dim3(64), 0, s, mats_dev, tokens, splits);
+    hipLaunchKernelGGL(energy_total_kernel, dim3(n_mats), dim3(kTotalThreads), 0, s, mats_dev, channels);
     return check_launch("rch_fit_residual (totals)");
 }
 
@@ -1582,13 +1737,9 @@ int rch_fit_span(const rch_fit_matrix* mats_dev, int n_mats, int channels, int64
                        channels);
     hipLaunchKernelGGL(basis_terms_kernel, dim3(n), dim3(kCholThreads), 0, s, mats_dev);
     if (with_coefficients) {
-        // Two workgroups per CU over the batch, at least one 32-token stage each.
-        const int64_t stages = (max_rows + kSpanTokens - 1) / kSpanTokens;
-        int64_t splits = (512 + n_mats - 1) / n_mats;
-        splits = splits < stages ? splits : stages;
-        splits = splits < RCH_SPAN_SPLITS ? splits : RCH_SPAN_SPLITS;
-        hipLaunchKernelGGL(span_trace_kernel, dim3(static_cast<unsigned>(splits), n), dim3(kSpanThreads), 0, s, mats_dev);
-        hipLaunchKernelGGL(span_total_kernel, dim3((n + 63) / 64), dim3(64), 0, s, mats_dev, n_mats, static_cast<int>(splits));
+        const int64_t ranges = std::min<int64_t>((max_rows + kSpanRange - 1) / kSpanRange, RCH_SPAN_SPLITS);
+        hipLaunchKernelGGL(span_trace_kernel, dim3(static_cast<unsigned>(ranges), n), dim3(kSpanThreads), 0, s, mats_dev);
+        hipLaunchKernelGGL(span_total_kernel, dim3((n + 63) / 64), dim3(64), 0, s, mats_dev, n_mats);
     }
     return check_launch("rch_fit_span");
 }

@@ -9,7 +9,7 @@ measure_source_energy :692-724).  A stored basis is FP16 and coefficients follow
 
 MI355X design: one launch each for max|X| (which is also the finite scan), the projection
 (exact products summed in FP64 on MFMA, rounded once to fp32, with the per-column extrema of P
-fused in) and the residual / source energies (FP64 MFMA reconstruction, per-16- or 32-row partials,
+fused in) and the residual / source energies (FP64 MFMA reconstruction, per-16-row partials,
 fixed-order totals); the host reads the scalars it needs in one transfer.  ``tile_rows`` is
 validated but does not change the result beyond FP64 summation order.
 """

@@ -20,7 +20,7 @@ from .errors import ConfigurationError, UnsupportedError
 _DTYPE_CODES = {torch.bfloat16: _lib.DT_BF16, torch.float16: _lib.DT_F16, torch.float32: _lib.DT_F32}
 #: fp32 bits of +inf: an absmax key at or above it marks a non-finite source element.
 NONFINITE_BITS = 0x7F800000
-_ROW_TILE, _ROW_SPLITS = 16, 8  # fewest rows per partial energy, most channel parts of one (RCH_RESIDUAL_SPLITS)
+_ROW_TILE, _ROW_PARTS = 16, 16  # rows of a partial energy, most channel parts of one (RCH_RESIDUAL_PARTS)
 
 
 def _device(tensors) -> torch.device:
@@ -249,7 +249,7 @@ def energies(sources, absmax_keys: torch.Tensor, *, bases=None, ranks=None, coef
         raise ConfigurationError("residual energies need one basis, rank and coefficient matrix per source")
     table = _table(n)
     _fill_sources(table, aligned)
-    tiles = [_ROW_SPLITS * -(-int(x.shape[0]) // _ROW_TILE) for x in aligned]
+    tiles = [_ROW_PARTS * -(-int(x.shape[0]) // _ROW_TILE) for x in aligned]
     partials = torch.empty(2 * sum(tiles), dtype=torch.float64, device=device)
     totals = torch.empty((n, 2), dtype=torch.float64, device=device)
     table["absmax_ptr"] = absmax_keys.data_ptr() + 4 * np.arange(n)

@@ -354,6 +354,43 @@ def test_fit_launch_shapes_match_fp64(device, dtype, count, rows, channels, rank
         assert totals[i, 1] == pytest.approx(error, rel=1e-12)
 
 
+@pytest.mark.parametrize("dtype,count,rows,channels,rank", [
+    ("bfloat16", 400, 700, 264, 49),    # 128-token projection workgroups, shared residual operands
+    ("float16", 60, 4680, 136, 96),     # several channel parts, span ranges of more than one stage
+    ("float32", 300, 129, 520, 128),    # a last tile of one row, channels beside four equal parts
+    ("bfloat16", 24, 333, 1536, 17),    # channel-split projection, shared residual operands
+    ("float32", 600, 33, 8, 5),         # one 64-channel group, most waves without rows
+])
+def test_measurements_do_not_depend_on_the_batch(device, dtype, count, rows, channels, rank):
+    """P, its extrema, both energies, the residual matrix and the span terms of a matrix are the same
+    bits alone and in a batch, whatever shapes the batch's launches take and whatever rows and ranks
+    its other members have: a planned rank is verified in small rounds and finalized in the chunk."""
+    rng = np.random.default_rng(131)
+    x, _ = _source(rng, rows, channels, dtype, device)
+    basis, _ = _basis(rng, rank, channels, device)
+    low, _ = _basis(rng, max(1, rank // 2), channels, device)
+    # Members of other row counts and ranks between copies of one scaled matrix.
+    sources = [x * (1 + i % 3) if i % 4 else x[: 1 + (7 * i) % rows] for i in range(count)]
+    bases = [basis if i % 3 else low for i in range(count)]
+    ranks = [int(q.shape[0]) for q in bases]
+
+    def measure(members):
+        xs, qs, rs = ([values[i] for i in members] for values in (sources, bases, ranks))
+        keys = fk.absmax(xs)
+        coefficients, extrema = fk.project(xs, qs, rs, extrema=True)
+        totals, residuals = fk.energies(xs, keys, bases=qs, ranks=rs, coefficients=coefficients, residuals=True)
+        return coefficients, extrema, totals, residuals, fk.energies(xs, keys), fk.span_terms(qs, rs, coefficients)
+
+    together = measure(range(count))
+    for i in sorted({0, 1, 4, count // 2, count - 2, count - 1}):
+        for members in ([i], [i, (i + 1) % count, (i + 5) % count]):
+            part = measure(members)
+            assert torch.equal(part[0][0], together[0][i])
+            assert torch.equal(part[1][0, :2 * ranks[i]], together[1][i, :2 * ranks[i]])
+            assert torch.equal(part[2][0], together[2][i]) and torch.equal(part[3][0], together[3][i])
+            assert torch.equal(part[4][0], together[4][i]) and torch.equal(part[5][0], together[5][i])
+
+
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16", "float32"])
 def test_absmax_flags_nonfinite_values(device, dtype):
     """An infinity or a NaN anywhere (first and last element, either sign) puts the key at or above
