@@ -20,7 +20,7 @@
 extern "C" {
 #endif
 
-#define RCH_ABI_VERSION 18
+#define RCH_ABI_VERSION 19
 
 /* Status codes (mapped to reelcache errors by the host). */
 #define RCH_OK 0
@@ -288,11 +288,11 @@ int rch_restore_noalloc(const rch_pack* packs_host, int n_packs, const rch_job* 
  * addresses and affine values come with each call.
  *   jobs      int64 [n_jobs, RCH_CALL_JOB_WORDS]: dst, src, basis, RoPE cos, sin, pairs (0: none), host
  *             address of the fp32 affine block (scale | offset) and its floats (0: none), coef_exp,
- *             picture count.
+ *             picture count, device address of the rows that its unpack row writes (0: none).
  *   pictures  int64: the picture addresses of the jobs that have any, in job order.
  * Replaces one launch sequence's separate entries; no counterpart in the reference.
  */
-#define RCH_CALL_JOB_WORDS 10
+#define RCH_CALL_JOB_WORDS 11
 #define RCH_CALL_LAUNCH_WORDS 12
 #define RCH_CALL_PACK 0    /* max_nblocks, max_ksteps */
 #define RCH_CALL_UNPACK 1  /* tiles offset, n_tiles, max_rank */

@@ -58,7 +58,9 @@ int rch_call_run(const rch_call* call, void* image, void* buffer, const int64_t*
         bool rows_first = false;  // the job reads the rows that its unpack row writes
         for (int64_t u = 0; u < extra; ++u) {
             if (unpacked[u] != i) continue;
-            rows[(call->n_jobs + u) * kJobColumns + RCH_COLUMN(rch_job, src_ptr)] = in[1];
+            int64_t* unpack = rows + (call->n_jobs + u) * kJobColumns;
+            unpack[RCH_COLUMN(rch_job, src_ptr)] = in[1];
+            unpack[RCH_COLUMN(rch_job, dst_ptr)] = row[RCH_COLUMN(rch_job, src_ptr)] = in[10];
             rows_first = true;
         }
         row[RCH_COLUMN(rch_job, dst_ptr)] = in[0];

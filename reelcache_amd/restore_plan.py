@@ -225,6 +225,7 @@ _FAST_MAX_KSTEPS = {"fp16x2": 12, "fp16": 16, "bf16": 16, "fp32": 0}
 _PAIRS_MAX_KSTEPS = 12
 _STREAM_MAX_KSTEPS = 16  # the stream kernel keeps W (both fp16 parts) of up to 256 ranks in registers
 STREAM_TOKENS = 32  # tokens per work unit of the stream kernel (csrc/restore_stream.h)
+_UNPACK_BYTES = 64 << 20  # code rows unpacked at a time (a larger job alone): about a LongCat layer's 16 chunks
 _SPLIT_MAX_KSTEPS = 32  # rank halves (RCH_GF_SPLIT_RANK): up to 512 ranks
 
 
@@ -466,8 +467,7 @@ class _Layout:
             self.template[offset:offset + array.nbytes] = array.reshape(-1).view(np.uint8)
         self.plans, self.jobs = plans, len(descs)
         self.scratch_words = self.exp_words + len(descs)
-        self.codes_offset = (self.arena_bytes + self.pack_total + 4 * self.scratch_words + 255) // 256 * 256
-        self.buffer_bytes = self.codes_offset + self.codes_total + 256
+        self.buffer_bytes = self.arena_bytes + self.pack_total + 4 * self.scratch_words + 256
         # Pack-table and pack-pointer offsets are relative to the buffer base.
         pack_rows = np.zeros((len(packs), len(_lib.PACK_FIELDS)), dtype=np.int64)
         pack_relative = np.zeros_like(pack_rows)
@@ -486,9 +486,6 @@ class _Layout:
             self.pack_sources.append(pack["member"])
         self.pack_rows, self.pack_relative = pack_rows, pack_relative
         self.rows, self.rows_relative = rows, relative
-        for position, (index, at) in enumerate(self.unpacked):
-            # The restore reads the rows the unpack row writes.
-            rows[index, _C_SRC_PTR] = rows[len(descs) + position, _C_DST_PTR] = self.codes_offset + at
         self.table_jobs = [i for i, d in enumerate(descs) if d.table is not None]
         self.picture_jobs = [i for i, d in enumerate(descs) if d.pictures is not None]
         self._call_program(len(descs))
@@ -504,9 +501,9 @@ class _Layout:
         if len(self.pack_rows):
             launches.append((_lib.CALL_PACK, int(self.pack_rows[:, _PACK_COLUMN["nblocks"]].max()),
                              int(self.pack_rows[:, _PACK_COLUMN["ksteps"]].max())))
-        if self.unpacked:
-            launches.append((_lib.CALL_UNPACK, *self.unpack_tiles, self.unpack_rank))
-        for plan in self.plans:
+        for plan, unpack in self._plans_with_unpacks():
+            if unpack is not None:
+                launches.append((_lib.CALL_UNPACK, *unpack))
             if plan["variant"] == "dense":
                 kind, names = _lib.CALL_DENSE, ("tiles", "n_tiles", "channels", "head_dim", "out_dtype")
             elif plan["variant"] == "pair":
@@ -521,7 +518,7 @@ class _Layout:
             row[:len(launch)] = launch
         arrays = {"template": self.template, "rows": np.ascontiguousarray(self.rows),
                   "relative": np.ascontiguousarray(self.rows_relative),
-                  "unpacked": np.array([index for index, _ in self.unpacked] or [0], dtype=np.int64),
+                  "unpacked": np.array(list(self.unpacked) or [0], dtype=np.int64),
                   "packs": np.ascontiguousarray(self.pack_rows),
                   "packs_relative": np.ascontiguousarray(self.pack_relative),
                   "members": np.array(self.pack_sources or [0], dtype=np.int64), "launches": table}
@@ -537,6 +534,7 @@ class _Layout:
     def run_program(self, descs, dst, src, bases, pictures, device, stream, keepalive):
         """Fill, upload and launch one call through the native program."""
         buffer = torch.empty(self.buffer_bytes, dtype=torch.uint8, device=device)
+        codes, code_rows = self._code_rows(len(descs), device)
         host = _pinned_host(self.template.size)
         tables: dict = {}
         words = []
@@ -550,29 +548,52 @@ class _Layout:
                     entry = tables[id(table)] = (block.cos.data_ptr(), block.sin.data_ptr(), block.pairs.data_ptr())
                     keepalive.append(block.block)
             words += (dst[index], src[index], bases[index], *entry, desc.affine_address, desc.affine_size,
-                      desc.exponent, 0 if desc.pictures is None else len(desc.pictures))
+                      desc.exponent, 0 if desc.pictures is None else len(desc.pictures), code_rows[index])
         words = array("q", words)
         addresses = array("q", [address for index in self.picture_jobs for address in pictures[index]])
         keepalive.extend((host, buffer))
         _lib.call("rch_call_run", self.program.ctypes.data, host.data_ptr(), buffer.data_ptr(), words.buffer_info()[0],
                   addresses.buffer_info()[0], stream.cuda_stream)
+        del codes
         return self.program_launches
+
+    def _code_rows(self, count, device):
+        """The call's area of unpacked code rows, and each job's address in it (0: none).  The area is
+        allocated on the launch stream (the current one) and dropped by the caller once the launches
+        are enqueued: the allocator hands it to later work of that stream only, which runs after them.
+        So the calls of a stream, or of a captured graph, share one area instead of holding one each."""
+        addresses = [0] * count
+        if not self.unpacked:
+            return None, addresses
+        codes = torch.empty(self.codes_bytes, dtype=torch.uint8, device=device)
+        base = codes.data_ptr()
+        for index, at in self.unpacked.items():
+            addresses[index] = base + at
+        return codes, addresses
+
+    def _plans_with_unpacks(self):
+        """The plans in launch order, each with the ``(tiles, n_tiles, max_rank)`` of the unpack launch
+        ahead of it or None."""
+        ahead = dict(enumerate(self.unpack_passes))
+        return [(plan, ahead.pop(plan.get("pass", 0), None)) for plan in self.plans]
 
     def _unpack_layout(self, descs, kinds, rows, relative, arena):
         """Jobs whose codes are unpacked into aligned rows first (``rch_codes_unpack``): 16-bit modes'
         ranks beyond one wave's registers, which the rank-halves kernel takes from uint8 rows only.
         Without it they run the chunked general kernel, which converts (and gathers) a tile's codes
         again for every 32-channel block: two chunks of K and V, 32 x 128 channels, ranks 256-512,
-        from pictures take 4.24 ms there and 0.19 ms here (MI355X).  Smaller ranks stay as they are: the straight-line kernels gather
-        pictures themselves.  Appends an unpack row per such job to the tables; its rows and
-        ``kinds`` entry become those of an aligned uint8 source."""
-        self.unpacked, self.codes_total, self.unpack_rank = [], 0, 0
+        from pictures take 4.24 ms there and 0.19 ms here (MI355X).  Smaller ranks stay as they are: the
+        straight-line kernels gather pictures themselves.  Appends an unpack row per such job to the
+        tables; its rows and ``kinds`` entry become those of an aligned uint8 source.  Rows beyond
+        ``_UNPACK_BYTES`` go in passes over one area, each unpacked once the pass before is restored."""
+        self.unpacked, self.codes_bytes, self.unpack_passes = {}, 0, []  # unpacked: job -> offset in the area
+        self.pass_of = {}
         config, precision = self.config, self.precision
         limit = _FAST_MAX_KSTEPS[precision] if precision in _FAST_MAX_KSTEPS else 0
         if (self.staged or self.static or not limit or not _config_value(config, "fast_variant")
                 or not _config_value(config, "split_rank")):
             return rows, relative
-        extra, extra_relative, members = [], [], []
+        extra, extra_relative, members, first = [], [], [[]], 0
         for index, desc in enumerate(descs):
             row = rows[index]
             if not (desc.kind == _lib.SRC_PICTURE or (desc.kind == _lib.SRC_U8 and not row[_C_FLAGS] & _lib.JF_SRC_VEC)):
@@ -584,27 +605,30 @@ class _Layout:
             if not _fast_eligibility(_lib.SRC_U8, desc.head_dim, desc.table is not None, aligned, precision):
                 continue
             pitch = (desc.rank + 15) // 16 * 16
-            unpack, shifts = row.copy(), relative[index].copy()
+            unpack = row.copy()
             unpack[_C_DST_TOKEN] = pitch
-            shifts[_C_DST_PTR] = 1
             extra.append(unpack)
-            extra_relative.append(shifts)
+            extra_relative.append(relative[index].copy())
             aligned[_C_SRC_ROW], aligned[_C_SRC_COL] = pitch, 1
             aligned[[_C_PIC_SLOTS, _C_PIC_TABLE]] = 0
             rows[index] = aligned
             relative[index, _C_PIC_TABLE] = 0
-            relative[index, _C_SRC_PTR] = 1
             kinds[index] = _lib.SRC_U8
-            members.append(index)
-            self.unpacked.append((index, self.codes_total))
-            self.unpack_rank = max(self.unpack_rank, desc.rank)
-            self.codes_total += (desc.tokens * pitch + 255) // 256 * 256
-        if not members:
+            size = (desc.tokens * pitch + 255) // 256 * 256
+            if members[-1] and first + size > _UNPACK_BYTES:
+                members.append([])
+                first = 0
+            members[-1].append(index)
+            self.unpacked[index], self.pass_of[index] = first, len(members) - 1
+            first += size
+            self.codes_bytes = max(self.codes_bytes, first)
+        if not extra:
             return rows, relative
-        tiles = _tiles(members, descs)
-        positions = {index: len(descs) + position for position, index in enumerate(members)}
-        tiles[:, 0] = [positions[index] for index in tiles[:, 0].tolist()]
-        self.unpack_tiles = (arena.add(tiles), len(tiles))
+        positions = {index: len(descs) + position for position, index in enumerate(self.unpacked)}
+        for indices in members:
+            tiles = _tiles(indices, descs)
+            tiles[:, 0] = [positions[index] for index in tiles[:, 0].tolist()]
+            self.unpack_passes.append((arena.add(tiles), len(tiles), max(descs[index].rank for index in indices)))
         return np.concatenate([rows, np.stack(extra)]), np.concatenate([relative, np.stack(extra_relative)])
 
     def _affine_layout(self, descs, rows, relative, arena):
@@ -639,19 +663,19 @@ class _Layout:
                      if allow_fast else 0)
             key = (kinds[index], desc.dtype, desc.out_dtype, desc.head_dim, desc.channels,
                    _rank_steps_class(precision, desc.rank), None if desc.table is None else desc.rope_kind == "dense",
-                   flags)
+                   self.pass_of.get(index, 0), flags)
             groups.setdefault(key, []).append(index)
         compute_units = _compute_units(device)
         passes = 2 if precision == "fp16x2" else (4 if precision == "fp32" else 1)
         store_cost = _config_value(config, "store_cost")
         store_cost = float(_STORE_COST[precision] if store_cost is None else store_cost)
         plans = []
-        for key, members in groups.items():
+        for key, members in sorted(groups.items(), key=lambda group: group[0][-2]):  # pass by pass
             kind, group_flags = key[0], key[-1]
             first = descs[members[0]]
             channels, head_dim = first.channels, first.head_dim
             plan = {"kind": kind, "members": members, "channels": channels, "head_dim": head_dim,
-                    "out_dtype": first.out_dtype}
+                    "out_dtype": first.out_dtype, "pass": key[-2]}
             plans.append(plan)
             if kind == _lib.SRC_DENSE:
                 tiles = _tiles(members, descs)
@@ -875,15 +899,12 @@ class _Layout:
         base = buffer.data_ptr()
         rows = self.rows + self.rows_relative * base
         count = len(descs)
-        if not self.unpacked:
-            rows[:, _C_DST_PTR] = dst
-            rows[:, _C_SRC_PTR] = src
-        else:  # unpacked jobs read the call buffer's rows, their unpack rows the source
-            codes = rows[:count, _C_SRC_PTR].copy()
-            rows[:count, _C_DST_PTR] = dst
-            rows[:count, _C_SRC_PTR] = src
-            for position, (index, _) in enumerate(self.unpacked):
-                rows[index, _C_SRC_PTR], rows[count + position, _C_SRC_PTR] = codes[index], src[index]
+        rows[:count, _C_DST_PTR] = dst
+        rows[:count, _C_SRC_PTR] = src
+        codes, code_rows = self._code_rows(count, device)
+        for position, index in enumerate(self.unpacked):  # the restore reads the rows that the unpack row writes
+            rows[count + position, _C_SRC_PTR] = src[index]
+            rows[count + position, _C_DST_PTR] = rows[index, _C_SRC_PTR] = code_rows[index]
         tables: dict = {}
         for index in self.table_jobs:
             table = descs[index].table
@@ -921,8 +942,9 @@ class _Layout:
             buffer[start:start + 4 * len(self.bound_jobs)].zero_()  # fill kernel, not a memset (graph-capture safe)
         buffer[:image.size].copy_(host, non_blocking=True)
         keepalive.extend((host, buffer))
-        return self._launch(base, scratch_base, packs, stream, stage_events, descs, keepalive)
-
+        launches = self._launch(base, scratch_base, packs, stream, stage_events, descs, keepalive)
+        del codes
+        return launches
 
     def _launch(self, base, scratch_base, packs, stream, stage_events, descs, keepalive):
         hip_stream = stream.cuda_stream
@@ -940,11 +962,10 @@ class _Layout:
             _lib.call("rch_coefficient_bound", table, jobs, base + self.bound_tile_offset, len(self.bound_tiles),
                       int(max(self.rows[i, _C_RANK] for i in self.bound_jobs)), scratch_base, hip_stream)
             launches += 1
-        if self.unpacked:
-            _lib.call("rch_codes_unpack", table, len(self.rows), base + self.unpack_tiles[0], self.unpack_tiles[1],
-                      self.unpack_rank, hip_stream)
-            launches += 1
-        for plan in self.plans:
+        for plan, unpack in self._plans_with_unpacks():
+            if unpack is not None:
+                _lib.call("rch_codes_unpack", table, len(self.rows), base + unpack[0], *unpack[1:], hip_stream)
+                launches += 1
             variant = plan["variant"]
             if variant == "staged":
                 launches += self._launch_staged(plan, base, scratch_base, stream, stage_events, descs, keepalive)

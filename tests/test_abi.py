@@ -75,7 +75,7 @@ def test_call_program_layout_matches_the_header():
     names = [name.strip().split()[-1] for line in body.split(";") if line.strip() for name in line.split(",")]
     assert tuple(names) == _lib.CALL_FIELDS and _lib.library().rch_call_size() == 8 * len(names)
     defines = {name: int(value) for name, value in re.findall(r"#define (RCH_CALL_[A-Z_]+) (\d+)\b", text)}
-    assert defines == {"RCH_CALL_JOB_WORDS": 10, "RCH_CALL_LAUNCH_WORDS": _lib.CALL_LAUNCH_WORDS,
+    assert defines == {"RCH_CALL_JOB_WORDS": 11, "RCH_CALL_LAUNCH_WORDS": _lib.CALL_LAUNCH_WORDS,
                        "RCH_CALL_PACK": _lib.CALL_PACK, "RCH_CALL_UNPACK": _lib.CALL_UNPACK,
                        "RCH_CALL_DENSE": _lib.CALL_DENSE, "RCH_CALL_RESTORE": _lib.CALL_RESTORE,
                        "RCH_CALL_PAIR": _lib.CALL_PAIR}
