@@ -534,7 +534,7 @@ class _Layout:
     def run_program(self, descs, dst, src, bases, pictures, device, stream, keepalive):
         """Fill, upload and launch one call through the native program."""
         buffer = torch.empty(self.buffer_bytes, dtype=torch.uint8, device=device)
-        codes, code_rows = self._code_rows(len(descs), device)
+        codes, code_rows = self._code_rows(device) if self.unpacked else (None, self.no_code_rows)
         host = _pinned_host(self.template.size)
         tables: dict = {}
         words = []
@@ -557,14 +557,12 @@ class _Layout:
         del codes
         return self.program_launches
 
-    def _code_rows(self, count, device):
+    def _code_rows(self, device):
         """The call's area of unpacked code rows, and each job's address in it (0: none).  The area is
         allocated on the launch stream (the current one) and dropped by the caller once the launches
         are enqueued: the allocator hands it to later work of that stream only, which runs after them.
         So the calls of a stream, or of a captured graph, share one area instead of holding one each."""
-        addresses = [0] * count
-        if not self.unpacked:
-            return None, addresses
+        addresses = list(self.no_code_rows)
         codes = torch.empty(self.codes_bytes, dtype=torch.uint8, device=device)
         base = codes.data_ptr()
         for index, at in self.unpacked.items():
@@ -587,7 +585,7 @@ class _Layout:
         tables; its rows and ``kinds`` entry become those of an aligned uint8 source.  Rows beyond
         ``_UNPACK_BYTES`` go in passes over one area, each unpacked once the pass before is restored."""
         self.unpacked, self.codes_bytes, self.unpack_passes = {}, 0, []  # unpacked: job -> offset in the area
-        self.pass_of = {}
+        self.pass_of, self.no_code_rows = {}, (0,) * len(descs)
         config, precision = self.config, self.precision
         limit = _FAST_MAX_KSTEPS[precision] if precision in _FAST_MAX_KSTEPS else 0
         if (self.staged or self.static or not limit or not _config_value(config, "fast_variant")
@@ -901,7 +899,7 @@ class _Layout:
         count = len(descs)
         rows[:count, _C_DST_PTR] = dst
         rows[:count, _C_SRC_PTR] = src
-        codes, code_rows = self._code_rows(count, device)
+        codes, code_rows = self._code_rows(device) if self.unpacked else (None, self.no_code_rows)
         for position, index in enumerate(self.unpacked):  # the restore reads the rows that the unpack row writes
             rows[count + position, _C_SRC_PTR] = src[index]
             rows[count + position, _C_DST_PTR] = rows[index, _C_SRC_PTR] = code_rows[index]
