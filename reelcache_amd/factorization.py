@@ -199,9 +199,12 @@ def project_onto_basis(tensor: torch.Tensor, basis: torch.Tensor, *, rank: int |
                        _work: dict | None = None) -> Projection:
     """Project once onto the stored FP16 basis and measure the direct residual in FP64.
 
-    Everything is enqueued before the one host read: the finite scans of the basis and of the matrix
-    (absmax keys), the condition terms, the projection with its column extrema and the energies.  The
-    checks then run on the host values in their order (basis, condition, matrix, overflow, energies)."""
+    Up to the native kernels' rank and with the condition bound not given, everything is enqueued before
+    the one host read: the finite scans of the basis and of the matrix (absmax keys), the condition terms,
+    the projection with its column extrema and the energies.  The checks then run on the host values in
+    their order (basis, condition, matrix, overflow, energies).  Otherwise the basis and its condition are
+    read and checked first.  ``condition_seconds`` is the time until the condition terms are done on the
+    device, ``coefficient_seconds`` the rest up to the read, either way."""
     started = time.perf_counter()
     _check_projection_input(tensor)
     _check_stored_basis(basis, tensor.shape[1])
@@ -221,10 +224,14 @@ def project_onto_basis(tensor: torch.Tensor, basis: torch.Tensor, *, rank: int |
         raise
     view = stored[:rank].to(device=tensor.device)
     condition_started = time.perf_counter()
-    condition, terms, basis_keys = _condition_bound, None, None
+    condition, terms, basis_keys, marks = _condition_bound, None, None, None
     if condition is None and rank <= fit_kernels.CHOLESKY_MAX_K and stored.device == tensor.device:
+        # The wait for the terms comes with the one read: events tell the condition's share of it.
+        marks = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        marks[0].record(torch.cuda.current_stream(tensor.device))
         basis_keys = fit_kernels.absmax([stored])
         terms = fit_kernels.span_terms([view], [rank])
+        marks[1].record(torch.cuda.current_stream(tensor.device))
     else:
         validate_stored_basis(basis, tensor.shape[1])
         if condition is None:
@@ -249,6 +256,10 @@ def project_onto_basis(tensor: torch.Tensor, basis: torch.Tensor, *, rank: int |
         condition = _terms_condition([float(v) for v in host[4 + 2 * rank:]])
         _check_condition(condition, max_condition)
     coefficient_seconds = time.perf_counter() - coefficient_started
+    if marks is not None:
+        total = condition_seconds + coefficient_seconds
+        condition_seconds = min(total, marks[0].elapsed_time(marks[1]) * 1e-3)
+        coefficient_seconds = total - condition_seconds
     if bits >= fit_kernels.NONFINITE_BITS:
         raise ConfigurationError("projection requires a nonempty finite FP32-compatible matrix")
     if not (math.isfinite(low) and math.isfinite(high)):

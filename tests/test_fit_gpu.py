@@ -483,6 +483,30 @@ def test_projection_reports_its_first_fault(device):
         fa.project_onto_basis(infinite, singular)
 
 
+def test_projection_times_its_condition(device):
+    """condition_seconds covers the condition's device work, though the wait for it comes with the read
+    that ends the coefficients; the parts of the time do not exceed the whole."""
+    from reelcache_amd import factorization as fa
+
+    channels, rank = 1 << 17, 128  # the basis Gram alone takes about a millisecond
+    generator = torch.Generator(device=device).manual_seed(7)
+    basis = (torch.randn(rank, channels, device=device, generator=generator) / channels ** 0.5).to(torch.float16)
+    x = torch.randn(rank, channels, device=device, generator=generator).to(torch.bfloat16)
+    fa.project_onto_basis(x, basis)
+    marks = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    torch.cuda.synchronize(device)
+    marks[0].record()
+    for _ in range(4):
+        fk.span_terms([basis], [rank])
+    marks[1].record()
+    marks[1].synchronize()
+    terms = marks[0].elapsed_time(marks[1]) * 1e-3 / 4
+    projection = fa.project_onto_basis(x, basis)
+    assert terms > 5e-4 and projection.condition_seconds >= 0.5 * terms
+    assert projection.coefficient_seconds > 0
+    assert projection.condition_seconds + projection.coefficient_seconds + projection.guard_seconds <= projection.seconds
+
+
 @pytest.mark.parametrize("rows,cols,stride", [(1, 1, 1), (17, 3, 5), (64, 96, 96), (65, 130, 132), (130, 63, 64)])
 def test_extrema_and_codes_at_tile_edges(device, rows, cols, stride):
     """Column extrema and codes of strided matrices around the kernels' row tiles, column lanes and
