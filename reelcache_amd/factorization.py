@@ -143,10 +143,10 @@ def _canonical_signs(basis: torch.Tensor) -> torch.Tensor:
 @torch.no_grad()
 def basis_condition_bound(basis: torch.Tensor) -> float:
     """Infinity-norm condition bound ||G|| ||G^-1|| of G = B B^T in FP64 via Cholesky
-    (inf for a singular basis).  FP16 rows on a GPU, up to the native kernels' order, take one native
-    call and one read; others the library's factorization."""
+    (inf for a singular basis).  FP16 rows on a GPU, up to the native kernels' order and channels, take
+    one native call and one read; others the library's factorization."""
     if (basis.device.type == "cuda" and basis.dtype == torch.float16 and basis.ndim == 2
-            and 1 <= basis.shape[0] <= fit_kernels.CHOLESKY_MAX_K and basis.shape[1] >= 1):
+            and 1 <= basis.shape[0] <= fit_kernels.CHOLESKY_MAX_K and 1 <= basis.shape[1] <= fit_kernels.MAX_CHANNELS):
         return _terms_condition(fit_kernels.span_terms([basis], [int(basis.shape[0])])[0].tolist())
     rounded = basis.to(dtype=torch.float64)
     gram = rounded @ rounded.T

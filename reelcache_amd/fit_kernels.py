@@ -23,6 +23,13 @@ NONFINITE_BITS = 0x7F800000
 _ROW_TILE, _ROW_PARTS = 16, 16  # rows of a partial energy, most channel parts of one (RCH_RESIDUAL_PARTS)
 
 
+#: Most (padded) channels of the fit kernels (csrc/fit.hip: check_matrices).
+MAX_CHANNELS = 1 << 20
+# The kernels address the rows of a tile (of X) or of a whole basis view by 32-bit offsets below 2 GiB: larger
+# strides are read through a copy.
+_OFFSET_LIMIT, _TILE_ROWS = 1 << 31, 32
+
+
 def _device(tensors) -> torch.device:
     devices = {tensor.device for tensor in tensors}
     if len(devices) != 1:
@@ -46,7 +53,8 @@ def _aligned(x: torch.Tensor, channels: int) -> torch.Tensor:
     """``x`` when the kernels can read it in place, else a copy into a zero-padded buffer."""
     size = x.element_size()
     if (x.shape[1] == channels and x.stride(1) == 1 and x.stride(0) >= channels
-            and (x.stride(0) * size) % 16 == 0 and x.data_ptr() % 16 == 0):
+            and (x.stride(0) * size) % 16 == 0 and x.data_ptr() % 16 == 0
+            and x.stride(0) * size * _TILE_ROWS < _OFFSET_LIMIT):
         return x
     out = torch.zeros((x.shape[0], channels), dtype=x.dtype, device=x.device)
     out[:, :x.shape[1]].copy_(x)
@@ -75,7 +83,9 @@ def _check_sources(sources) -> tuple[list[torch.Tensor], int, int]:
     for x in sources:
         stride = x.stride()
         # _aligned's in-place rule (the channel count is c8 here).
-        if stride[1] == 1 and stride[0] >= c8 and (stride[0] * size) % 16 == 0 and x.data_ptr() % 16 == 0:
+        pitch = stride[0] * size
+        if (stride[1] == 1 and stride[0] >= c8 and pitch % 16 == 0 and x.data_ptr() % 16 == 0
+                and pitch * _TILE_ROWS < _OFFSET_LIMIT):
             aligned.append(x)
         else:
             aligned.append(_aligned(x, c8))
@@ -157,9 +167,11 @@ def _basis_rows(basis: torch.Tensor, rank: int, c8: int, keep: list) -> tuple[in
         raise ConfigurationError("the stored basis must be float16")
     stride = basis.stride()
     address = basis.data_ptr()
-    if basis.shape[1] == c8 and stride[1] == 1 and stride[0] >= c8 and (stride[0] * 2) % 16 == 0 and address % 16 == 0:
+    if (basis.shape[1] == c8 and stride[1] == 1 and stride[0] >= c8 and (stride[0] * 2) % 16 == 0 and address % 16 == 0
+            and 2 * stride[0] * rank < _OFFSET_LIMIT):
         return address, stride[0]
-    q = _aligned(basis[:rank], c8)
+    q = torch.zeros((rank, c8), dtype=basis.dtype, device=basis.device)
+    q[:, :basis.shape[1]].copy_(basis[:rank])
     keep.append(q)
     return q.data_ptr(), q.stride(0)
 

@@ -483,6 +483,29 @@ def test_projection_reports_its_first_fault(device):
         fa.project_onto_basis(infinite, singular)
 
 
+def test_condition_bound_beyond_the_native_addressing(device):
+    """basis_condition_bound takes what it took before it had a native path: rows 2 GiB apart in all (the
+    kernels' 32-bit offsets end there, so they are read through a copy), also through the projection and
+    as a source, and more channels than the fit kernels take."""
+    from reelcache_amd import factorization as fa
+
+    rank, channels, pitch = 128, 256, 9 << 20
+    generator = torch.Generator(device=device).manual_seed(8)
+    rows = torch.linalg.qr(torch.randn(channels, rank, device=device, generator=generator)).Q.T.contiguous().to(torch.float16)
+    storage = torch.empty((rank - 1) * pitch + channels, dtype=torch.float16, device=device)
+    apart = storage.as_strided((rank, channels), (pitch, 1))
+    apart.copy_(rows)
+    assert fa.basis_condition_bound(apart) == fa.basis_condition_bound(rows) < 1.5
+    x, _ = _source(np.random.default_rng(3), rank, channels, "bfloat16", device)
+    assert torch.equal(fk.project([x], [apart], [rank])[0][0], fk.project([x], [rows], [rank])[0][0])
+    far = storage.as_strided((32, channels), (4 * pitch, 1))
+    assert torch.equal(fk.project([far], [rows], [rank])[0][0], fk.project([far.contiguous()], [rows], [rank])[0][0])
+    wide = torch.randn(2, (1 << 20) + 8, device=device, generator=generator).to(torch.float16)
+    gram = wide.double() @ wide.double().T
+    want = float(gram.abs().sum(1).max() * torch.linalg.inv(gram).abs().sum(1).max())
+    assert fa.basis_condition_bound(wide) == pytest.approx(want, rel=1e-9)
+
+
 def test_projection_times_its_condition(device):
     """condition_seconds covers the condition's device work, though the wait for it comes with the read
     that ends the coefficients; the parts of the time do not exceed the whole."""
