@@ -21,6 +21,7 @@ many layers of one model):
 
 from __future__ import annotations
 
+import itertools
 import math
 import threading
 from array import array
@@ -311,7 +312,7 @@ class _JobDesc:
         pictures = None if self.pictures is None else (len(source.pictures), len(source.pictures[0]))
         self.key = (row.tobytes(), self.kind, self.dtype, self.out_dtype, self.head_dim, self.channels, self.rope_kind,
                     self.basis_key, self.host_bound is None, pictures, self.section_pairs)
-        self.key_id = _KEY_IDS.setdefault(self.key, len(_KEY_IDS))
+        self.key_id = _KEY_IDS.setdefault(self.key, next(_KEY_NUMBERS))
 
     def _destination(self, row, view, tensor):
         size = tensor.element_size()
@@ -383,8 +384,11 @@ class _JobDesc:
         self.exponent = _prescale_exponent(_coefficient_bound(scale, offset))
 
 
-# Distinct job geometries (descriptor keys) seen by this process, numbered for cheap call keys.
+# Distinct job geometries (descriptor keys) seen by this process, numbered for cheap call keys.  A number
+# is drawn once, so threads that meet new geometries at the same time never share one (a shared number
+# would give one call the other's layout); a number may go unused.
 _KEY_IDS: dict = {}
+_KEY_NUMBERS = itertools.count()
 
 
 def job_desc(job):

@@ -229,3 +229,19 @@ def test_replaced_staging_slab_stays_alive(monkeypatch):
     unused = rp._STAGING["slab"][0]
     rp.reserve_capture_staging(1 << 21)
     assert not any(kept is unused for kept in rp._RETIRED_SLABS)
+
+
+def test_geometries_met_at_the_same_time_get_their_own_numbers(monkeypatch):
+    """Two threads that number a new geometry each, with the table's size read by both before either adds
+    its entry, must not share a number: call layouts are kept by these numbers."""
+    class Interleaved(dict):
+        def __len__(self):
+            return 0  # as read before the other thread's entry
+
+    monkeypatch.setattr(rp, "_KEY_IDS", Interleaved())
+    rng = np.random.default_rng(5)
+    jobs = [make_case(rng, grid=(1, 4, 5), heads=2, head_dim=32, rank=rank).job for rank in (8, 12)]
+    first, second = (rp.job_desc(job).key_id for job in jobs)
+    assert first != second
+    again = make_case(rng, grid=(1, 4, 5), heads=2, head_dim=32, rank=8).job
+    assert rp.job_desc(again).key_id == first
