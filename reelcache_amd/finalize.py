@@ -182,8 +182,9 @@ def _rank_terms(coefficients, rows):
         products = torch.stack([c.double().T @ c.double() for c in coefficients])
     q64 = q.double()
     gram = torch.bmm(q64, q64.mT)
-    factor, info = torch.linalg.cholesky_ex(gram)
-    traces = torch.cholesky_solve(products, factor).diagonal(dim1=1, dim2=2).sum(-1)
+    # G = R^T R, X = R^-1: trace(G^-1 C) = trace(X^T C X) = sum X * (C X).
+    inverse, info = fit_kernels.factor_inverse(gram)
+    traces = (inverse * torch.bmm(products, inverse)).sum((1, 2))
     q32 = q.float()
     gram32 = torch.bmm(q32, q32.mT)
     largest = gram32.diagonal(dim1=1, dim2=2).abs().amax(-1)

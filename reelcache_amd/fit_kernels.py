@@ -321,6 +321,38 @@ def cholesky_inverse(gram: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     return inverse, info
 
 
+def factor_inverse(gram: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    """:func:`cholesky_inverse` of a batch of any order, in block rows of equal orders up to
+    :data:`CHOLESKY_MAX_K`: per block its own factor and inverse in one launch, FP64 products for the rows
+    of R beside it, the trailing update and the inverse's column above it.
+
+    torch's batched Cholesky does not serve here: its results changed after the call when other work of
+    the stream followed without a host wait (relative error 1e-6 of a span trace at orders 144 to 192,
+    spurious failures), and it has ended in a launch failure."""
+    k = gram.shape[-1]
+    if k <= CHOLESKY_MAX_K:
+        return cholesky_inverse(gram)
+    blocks = -(-k // CHOLESKY_MAX_K)
+    step = -(-k // (16 * blocks)) * 16
+    trailing = gram.clone()
+    inverse, factor = torch.zeros_like(trailing), torch.zeros_like(trailing)
+    info = torch.zeros(gram.shape[0], dtype=torch.int32, device=gram.device)
+    for first in range(0, k, step):
+        end = min(k, first + step)
+        own, failed = cholesky_inverse(trailing[:, first:end, first:end])
+        info = torch.where((info == 0) & (failed != 0), failed + first, info)
+        inverse[:, first:end, first:end] = own
+        if first:
+            above = torch.bmm(inverse[:, :first, :first], factor[:, :first, first:end])
+            inverse[:, :first, first:end] = -torch.bmm(above, own)
+        if end < k:
+            beside = torch.bmm(own.mT, trailing[:, first:end, end:])
+            factor[:, first:end, end:] = beside
+            trailing[:, end:, end:] -= torch.bmm(beside.mT, beside)
+    identity = torch.eye(k, dtype=gram.dtype, device=gram.device)
+    return torch.where((info != 0)[:, None, None], identity, inverse), info
+
+
 _SPAN_SPLITS = 64  # RCH_SPAN_SPLITS
 
 

@@ -79,6 +79,34 @@ def test_finalize_chunk_matches_oracle(device):
         np.testing.assert_array_equal(tile.gram, rows.astype(np.float64) @ rows.astype(np.float64).T)
 
 
+@pytest.mark.parametrize("ranks", [[32, 192, 96, 256, 128, 192, 129], [192, 144, 192]])
+def test_finalize_ranks_on_both_sides_of_the_native_order(device, ranks):
+    """Ranks up to 128 take the native span kernels and larger ones the library's products and
+    factorization per rank: interleaved in one batch, and all above, each tile's energies, span energy,
+    condition, codes and affine are its own, as in the chunk test, and as it has them alone."""
+    rng = np.random.default_rng(92)
+    generator = torch.Generator(device=device).manual_seed(92)
+    items = [_item(rng, generator, device, index, rank) for index, rank in enumerate(ranks)]
+    results = npk.finalize_tiles(items, tile_rows=1024, keep_coefficients=True)
+    for item, (tile, pixels) in zip(items, results):
+        rows, host, p = item.host_rows.numpy(), item.matrix.float().cpu().numpy(), tile.coefficients
+        assert tile.entry == item.entry and p.shape == (TOKENS, item.spec.rank)
+        scale, source, error = of.energies(host, rows, p)
+        assert abs(tile.stored_energy - (1.0 - error / source)) <= 1e-12
+        source_energy = source * scale ** 2
+        assert abs(tile.source_energy - source_energy) <= 1e-12 * source_energy
+        assert abs(tile.ideal_energy - min(1.0, of.span_energy(p, rows, source_energy))) <= 1e-12
+        assert basis_condition_bound(item.rows16) <= tile.condition_bound < 1.5
+        codes, affine, _ = oq.quantize(p, item.spec.normalization, item.spec.protected_fraction)
+        np.testing.assert_array_equal(pixels.cpu().numpy(), codes)
+        assert tile.affine == affine.astype("<f4").tobytes()
+        (alone, alone_pixels), = npk.finalize_tiles([item], tile_rows=1024)
+        assert torch.equal(alone_pixels, pixels)
+        assert alone.stored_energy == tile.stored_energy and alone.source_energy == tile.source_energy
+        if item.spec.rank <= 128:  # the library's batched products may round by the batch
+            assert alone.ideal_energy == tile.ideal_energy and alone.condition_bound == tile.condition_bound
+
+
 def test_finalize_targets_zero_input_and_canvas(device):
     rng = np.random.default_rng(91)
     generator = torch.Generator(device=device).manual_seed(91)

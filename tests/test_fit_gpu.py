@@ -292,6 +292,33 @@ def test_cholesky_inverse_matches_fp64_factorization(device, k):
         assert (np.tril(got, -1) == 0).all()
 
 
+@pytest.mark.parametrize("k", [100, 129, 144, 192, 256, 257, 300, 512])
+def test_factor_inverse_of_any_order(device, k):
+    """Orders beyond one launch go in block rows: the triangular inverse against numpy's FP64 factorization
+    (relative 1e-11: condition 900, up to four blocks), zeros below the diagonal, LAPACK's info in the first,
+    a later and the last block, NaN at order 1; the same bits again with other work queued behind it."""
+    from scipy.linalg import solve_triangular
+
+    rng = np.random.default_rng(61 + k)
+    batch = []
+    for _ in range(3):
+        q, _ = np.linalg.qr(rng.standard_normal((k, k)))
+        batch.append((q * rng.uniform(1.0, 30.0, k)) @ q.T)
+    early, late, nan = batch[0].copy(), batch[1].copy(), batch[2].copy()
+    early[4, 4], late[k - 1, k - 1], nan[0, 0] = -1.0, -1.0, np.nan
+    a = torch.from_numpy(np.stack(batch + [early, late, nan])).to(device)
+    inverse, info = fk.factor_inverse(a)
+    behind = [torch.full((1 << 20,), 1.0, dtype=torch.float64, device=device) * 2 for _ in range(4)]
+    again, _ = fk.factor_inverse(a)
+    assert info.cpu().tolist() == [0, 0, 0, 5, k, 1] and torch.equal(inverse, again) and len(behind) == 4
+    inverse = inverse.cpu().numpy()
+    for member, got in zip(batch, inverse):
+        want = solve_triangular(np.linalg.cholesky(member).T, np.eye(k), lower=False)
+        assert np.abs(got - want).max() <= 1e-11 * np.abs(want).max()
+        assert (np.tril(got, -1) == 0).all()
+    assert (inverse[3:] == np.eye(k)).all()
+
+
 def test_cholesky_inverse_flags_indefinite_members(device):
     """LAPACK's info convention: j + 1 for the first leading minor that is not positive definite
     (a negative pivot at order 4, a NaN at order 1); such members come back as the identity and
@@ -445,6 +472,68 @@ def test_span_terms_flag_singular_views(device):
     terms = fk.span_terms([zero, good, nan], [20, 20, 20]).cpu().numpy()
     assert terms[:, 1].tolist() == [18.0, 0.0, 1.0]
     assert np.isinf(terms[0, 5]) and np.isinf(terms[2, 5]) and np.isfinite(terms[1]).all()
+
+
+@pytest.mark.parametrize("rank", [12, 33, 128])
+def test_span_terms_of_ill_conditioned_views(device, rank):
+    """Rows near one direction (condition of G about 1e6): the trace and both norms against extended
+    precision, within the forward error of a Cholesky solve, 8 k eps cond(G)."""
+    rng = np.random.default_rng(103)
+    channels, tokens = 512, 300
+    common = rng.standard_normal(channels) / channels ** 0.5
+    rows = (common + 0.02 * rng.standard_normal((rank, channels)) / channels ** 0.5).astype(np.float16)
+    p = rng.standard_normal((tokens, rank)).astype(np.float32)
+    got = fk.span_terms([torch.from_numpy(rows).to(device)], [rank], [torch.from_numpy(p).to(device)]).cpu().numpy()[0]
+    q = rows.astype(np.longdouble)
+    gram, c = q @ q.T, p.astype(np.longdouble).T @ p.astype(np.longdouble)
+    work = np.concatenate([gram, c, np.eye(rank, dtype=np.longdouble)], axis=1)
+    for j in range(rank):  # Gauss-Jordan without pivoting (G is positive definite)
+        work[j] /= work[j, j]
+        others = np.arange(rank) != j
+        work[others] -= work[others, j][:, None] * work[j]
+    solved, inverse = work[:, rank:2 * rank], work[:, 2 * rank:]
+    condition = float(np.linalg.cond(gram.astype(np.float64)))
+    assert 1e4 < condition < 1e8 and got[1] == 0
+    bound = 8 * rank * 2.0 ** -52 * condition
+    assert got[0] == pytest.approx(float(np.trace(solved)), rel=bound)
+    assert got[4] == pytest.approx(float(np.abs(gram).sum(1).max()), rel=1e-12)
+    assert got[5] == pytest.approx(float(np.abs(inverse).sum(1).max()), rel=bound)
+
+
+@pytest.mark.parametrize("rank", [129, 192])
+def test_projection_above_the_native_order(device, rank):
+    """Ranks above the span kernels' order read and check the basis and its condition first, then project:
+    coefficients, residual and condition against FP64, and the faults in their order."""
+    from reelcache_amd import factorization as fa
+    from reelcache_amd.errors import ConfigurationError
+
+    rng = np.random.default_rng(107)
+    x, host = _source(rng, 300, 256, "bfloat16", device)
+    q, q_host = _basis(rng, rank + 3, 256, device)
+    projection = fa.project_onto_basis(x, q, rank=rank)
+    p = projection.coefficients.cpu().numpy()
+    assert p.shape == (300, rank) and (p == of.project(host, q_host, rank)).mean() >= 0.999
+    _, source, error = of.energies(host, q_host, p, rank)
+    assert projection.relative_residual == pytest.approx((error / source) ** 0.5, rel=1e-12)
+    wide = np.asarray(q_host, dtype=np.float16).astype(np.float64)[:rank]
+    gram = wide @ wide.T
+    want = np.abs(gram).sum(1).max() * np.abs(np.linalg.inv(gram)).sum(1).max()
+    assert projection.condition_bound == pytest.approx(want, rel=1e-9)
+    given = fa.project_onto_basis(x, q, rank=rank, _condition_bound=1.25)
+    assert given.condition_bound == 1.25 and torch.equal(given.coefficients, projection.coefficients)
+    assert projection.condition_seconds > 0 and projection.coefficient_seconds > 0
+    bad = q.clone()
+    bad[rank + 2, 3] = float("nan")
+    infinite = x.clone()
+    infinite[0, 0] = float("inf")
+    with pytest.raises(ConfigurationError, match="stored basis must be finite"):
+        fa.project_onto_basis(infinite, bad, rank=rank)
+    singular = q.clone()
+    singular[4] = 0.0
+    with pytest.raises(ConfigurationError, match="singular or ill-conditioned"):
+        fa.project_onto_basis(infinite, singular, rank=rank)
+    with pytest.raises(ConfigurationError, match="nonempty finite"):
+        fa.project_onto_basis(infinite, q, rank=rank)
 
 
 def test_projection_reports_its_first_fault(device):
