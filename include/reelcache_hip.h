@@ -457,7 +457,7 @@ typedef struct rch_quantize_job {
 } rch_quantize_job;       /* 8 x int64 = 64 bytes */
 
 /*
- * rch_quantize over a batch of matrices in one launch (grid: 64-row tiles x jobs), e.g. the
+ * rch_quantize over a batch of matrices in one launch (grid: 16-row tiles x jobs), e.g. the
  * coefficients of every matrix of a chunk after projection.
  */
 int rch_quantize_batched(const rch_quantize_job* jobs_dev, int n_jobs, int64_t max_rows, void* stream);

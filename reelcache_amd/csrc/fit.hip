@@ -43,27 +43,6 @@ __device__ __forceinline__ float half_bits(uint32_t bits) {
     }
 }
 
-// Eight consecutive source elements as doubles.
-template <int DT>
-__device__ __forceinline__ void load8(__amdgpu_buffer_rsrc_t rsrc, uint32_t offset, double (&v)[8]) {
-    if constexpr (DT == RCH_DT_F32) {
-        const u4 a = __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset, 0, 0);
-        const u4 b = __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset + 16, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            v[i] = static_cast<double>(__uint_as_float(a[i]));
-            v[4 + i] = static_cast<double>(__uint_as_float(b[i]));
-        }
-    } else {
-        const u4 w = __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            v[2 * i] = static_cast<double>(half_bits<DT>(w[i] & 0xffffu));
-            v[2 * i + 1] = static_cast<double>(half_bits<DT>(w[i] >> 16));
-        }
-    }
-}
-
 // Order-preserving unsigned key of an fp32 value (larger value -> larger key).
 __device__ __forceinline__ uint32_t order_key(float v) {
     const uint32_t u = __float_as_uint(v);

@@ -157,10 +157,12 @@ def test_energies_match_fp64(device, dtype):
     assert source_only[0, 0] == pytest.approx(of.energies(host)[1], rel=1e-12)
 
 
-def test_energies_on_both_rank_paths(device):
-    """Ranks up to 64 keep the coefficient block in registers, larger ones stream it: a ragged batch
-    over both paths (and a rank that is not a multiple of 4) matches the FP64 oracle, and so does the
-    fp32 residual matrix X - P Q (rounded once from its FP64 value)."""
+@pytest.mark.parametrize("copies", [1, 12])
+def test_energies_and_residual_matrices_of_ragged_ranks(device, copies):
+    """Ranks beside the 16-rank steps (and one that is not a multiple of 4) in one batch, in 16-token
+    workgroups and, with the batch repeated, in the 128-token ones that share their basis operands: the
+    energies match the FP64 oracle, and so does the fp32 residual matrix X - P Q (rounded once from its
+    FP64 value)."""
     rng = np.random.default_rng(21)
     ranks = [13, 48, 64, 65, 130]
     sources, hosts, bases, host_bases = [], [], [], []
@@ -171,6 +173,7 @@ def test_energies_on_both_rank_paths(device):
         hosts.append(host)
         bases.append(q)
         host_bases.append(q_host)
+    sources, hosts, bases, host_bases, ranks = (copies * values for values in (sources, hosts, bases, host_bases, ranks))
     keys = fk.absmax(sources)
     coefficients, _ = fk.project(sources, bases, ranks)
     totals, residuals = fk.energies(sources, keys, bases=bases, ranks=ranks, coefficients=coefficients,
@@ -340,13 +343,13 @@ def test_cholesky_inverse_flags_indefinite_members(device):
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16", "float32"])
 @pytest.mark.parametrize("count,rows,channels,ranks", [
     (1, 17, 72, [1]),                   # one 16-token tile and a row of the next; channels below one step of each wave
-    (1, 4680, 264, [96]),               # channel-split projection and residual, several channel parts
-    (3, 31, 136, [16, 33, 130]),        # ragged ranks over several rank chunks
-    (70, 2000, 64, [49]),               # token-blocked shapes (32-token workgroups), 64-channel rows
-    (160, 1664, 40, [32]),              # 128-token projection workgroups
-    (350, 700, 72, [1, 33, 64]),        # shared basis operands: a last wave of 28 rows, one to four rank blocks
-    (18, 1000, 200, [16, 130, 75]),     # shared residual operands, four channel parts, ranks past a step
-    (500, 33, 72, [20, 5, 48]),         # waves of 32 rows, one row and none
+    (1, 4680, 264, [96]),               # 32-token projection, 16-token residual; several channel parts
+    (3, 31, 136, [16, 33, 130]),        # ragged ranks over several 16-rank chunks
+    (70, 2000, 64, [49]),               # 128-token workgroups of both; one residual part, one step a half
+    (160, 1664, 40, [32]),              # 128-token workgroups; a second half of one 8-channel group
+    (350, 700, 72, [1, 33, 64]),        # 128-token workgroups: a last wave of 28 rows, one to four rank blocks
+    (18, 1000, 200, [16, 130, 75]),     # 32-rank chunks beside 128-token residual workgroups, ranks past a step
+    (500, 33, 72, [20, 5, 48]),         # 128-token workgroups: waves of 32 rows, one row and none
 ])
 def test_fit_launch_shapes_match_fp64(device, dtype, count, rows, channels, ranks):
     """absmax, projection and residual energies on both sides of their launch-shape rules: maxima
