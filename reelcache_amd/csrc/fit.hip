@@ -1273,11 +1273,13 @@ __global__ void __launch_bounds__(kThreads) basis_gram_kernel(const rch_fit_matr
     const int t0 = 16 * blockIdx.x, r0 = 32 * blockIdx.y;
     if (t0 >= kp || r0 >= kp) return;  // whole workgroup
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (t0 == 0 && r0 == 0 && threadIdx.x == 0 && M->resid_ptr)  // basis_terms_kernel puts the time since in its place
+        *gout<uint64_t>(M->resid_ptr) = wall_clock64();
     if (r0 + 16 < kp) project_ranks<RCH_DT_F16, Project::kGram, 2>(M, channels, r0, t0, wave, lane, partial);
     else project_ranks<RCH_DT_F16, Project::kGram, 1>(M, channels, r0, t0, wave, lane, partial);
 }
 
-__global__ void __launch_bounds__(kCholThreads) basis_terms_kernel(const rch_fit_matrix* __restrict__ mats) {
+__global__ void __launch_bounds__(kCholThreads) basis_terms_kernel(const rch_fit_matrix* __restrict__ mats, double tick) {
     __shared__ CholeskyShared shared;
     constexpr int P = kCholPitch;
     const rch_fit_matrix* M = mats + blockIdx.x;
@@ -1372,6 +1374,10 @@ __global__ void __launch_bounds__(kCholThreads) basis_terms_kernel(const rch_fit
             out[2 + q] = v;
         }
         if (failed) out[5] = INFINITY;
+        if (M->resid_ptr) {
+            const uint64_t ticks = wall_clock64() - *gin<uint64_t>(M->resid_ptr);
+            *gout<double>(M->resid_ptr) = static_cast<double>(ticks) * tick;
+        }
     }
 }
 
@@ -1712,9 +1718,13 @@ int rch_fit_span(const rch_fit_matrix* mats_dev, int n_mats, int channels, int64
         return fail(RCH_E_CONFIG, "rch_fit_span: 1 <= max_rank <= %d and positive max_rows required", RCH_CHOLESKY_MAX_K);
     hipStream_t s = as_stream(stream);
     const unsigned n = static_cast<unsigned>(n_mats);
+    int device = 0, khz = 0;  // of the clock that the terms' time is read from
+    if (hipGetDevice(&device) != hipSuccess ||
+        hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) != hipSuccess || khz <= 0)
+        return fail(RCH_E_LAUNCH, "rch_fit_span: no device clock rate");
     hipLaunchKernelGGL(basis_gram_kernel, dim3((max_rank + 15) / 16, (max_rank + 31) / 32, n), dim3(kThreads), 0, s, mats_dev,
                        channels);
-    hipLaunchKernelGGL(basis_terms_kernel, dim3(n), dim3(kCholThreads), 0, s, mats_dev);
+    hipLaunchKernelGGL(basis_terms_kernel, dim3(n), dim3(kCholThreads), 0, s, mats_dev, 1e-3 / khz);
     if (with_coefficients) {
         const int64_t ranges = std::min<int64_t>((max_rows + kSpanRange - 1) / kSpanRange, RCH_SPAN_SPLITS);
         hipLaunchKernelGGL(span_trace_kernel, dim3(static_cast<unsigned>(ranges), n), dim3(kSpanThreads), 0, s, mats_dev);

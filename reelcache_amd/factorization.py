@@ -224,14 +224,10 @@ def project_onto_basis(tensor: torch.Tensor, basis: torch.Tensor, *, rank: int |
         raise
     view = stored[:rank].to(device=tensor.device)
     condition_started = time.perf_counter()
-    condition, terms, basis_keys, marks = _condition_bound, None, None, None
+    condition, terms, basis_keys, elapsed = _condition_bound, None, None, None
     if condition is None and rank <= fit_kernels.CHOLESKY_MAX_K and stored.device == tensor.device:
-        # The wait for the terms comes with the one read: events tell the condition's share of it.
-        marks = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
-        marks[0].record(torch.cuda.current_stream(tensor.device))
         basis_keys = fit_kernels.absmax([stored])
-        terms = fit_kernels.span_terms([view], [rank])
-        marks[1].record(torch.cuda.current_stream(tensor.device))
+        terms, elapsed = fit_kernels.span_terms([view], [rank], seconds=True)
     else:
         validate_stored_basis(basis, tensor.shape[1])
         if condition is None:
@@ -244,7 +240,7 @@ def project_onto_basis(tensor: torch.Tensor, basis: torch.Tensor, *, rank: int |
     totals = fit_kernels.energies([tensor], keys, bases=[view], ranks=[rank], coefficients=[coefficients])
     parts = [keys.double(), extrema.double().view(-1), totals.view(-1)]
     if terms is not None:
-        parts += [basis_keys.double(), terms.view(-1)]
+        parts += [basis_keys.double(), terms.view(-1), elapsed]
     host = torch.cat(parts).cpu().numpy()
     bits = int(host[0])
     low, high = fit_kernels.split_keys(host[1:1 + 2 * rank].astype(np.int64).astype(np.int32), rank)
@@ -253,13 +249,12 @@ def project_onto_basis(tensor: torch.Tensor, basis: torch.Tensor, *, rank: int |
     if terms is not None:
         if int(host[3 + 2 * rank]) >= fit_kernels.NONFINITE_BITS:
             raise ConfigurationError("stored basis must be finite")
-        condition = _terms_condition([float(v) for v in host[4 + 2 * rank:]])
+        condition = _terms_condition([float(v) for v in host[4 + 2 * rank:10 + 2 * rank]])
         _check_condition(condition, max_condition)
     coefficient_seconds = time.perf_counter() - coefficient_started
-    if marks is not None:
-        total = condition_seconds + coefficient_seconds
-        condition_seconds = min(total, marks[0].elapsed_time(marks[1]) * 1e-3)
-        coefficient_seconds = total - condition_seconds
+    if terms is not None:  # the wait for the terms came with the one read: the device timed their share of it
+        shift = min(coefficient_seconds, float(host[10 + 2 * rank]))
+        condition_seconds, coefficient_seconds = condition_seconds + shift, coefficient_seconds - shift
     if bits >= fit_kernels.NONFINITE_BITS:
         raise ConfigurationError("projection requires a nonempty finite FP32-compatible matrix")
     if not (math.isfinite(low) and math.isfinite(high)):
