@@ -19,7 +19,7 @@ The span energy uses the identity ``||L^-1 P^T||_F^2 = trace(G^-1 C)`` with ``G 
 ``C = P^T P`` (FP64) instead of an ``N x r`` triangular solve per tile: four hand-written launches
 for the batch, whatever its ranks up to 128 (``fit_kernels.span_terms``, with the fast condition
 bound's terms from the same FP64 Gram); larger ranks take, per group of one rank, one batched
-product ``C``, one batched Cholesky factorization and one batched solve.  Every scalar the host
+product ``C`` and one batched factorization in block rows (``fit_kernels.factor_inverse``).  Every scalar the host
 needs (scales, extrema, energies, traces, factorization status, condition terms) crosses in one
 transfer; the quantizer is one launch for the batch.
 """

@@ -24,8 +24,9 @@ Backends (same names as the reference, reelcache/restore_kernels.py:138):
   in its place.
 * ``fused`` -- the HIP path: one basis-packing launch and one fused kernel per
   launch group (gather/dequantize -> MFMA rank-view product -> RoPE -> cast ->
-  strided store).  ``two_pass`` selects the same kernels (pictures are gathered
-  inside the fused kernel; there is no separate unpack pass).
+  strided store).  ``two_pass`` selects the same kernels.  Pictures are gathered
+  inside the fused kernel, except at high ranks (16-bit modes, 193 or 257 to 512),
+  whose codes one launch unpacks into aligned rows first.
 * ``staged`` -- the comparison path of the reference's ``_staged_group``: a HIP
   unpack of each GEMM group's coefficients into a dense work matrix, the GPU BLAS
   library's product with FP32 output (``torch.mm``), then a HIP RoPE / cast /
