@@ -244,3 +244,27 @@ def test_sixty_matrix_chunk_matches_the_oracle_per_matrix(device):
         # degenerate eigenvectors are only fixed as a span, which the energies above pin.
         lead, head = rows[:4].astype(np.float32), reference[:4].astype(np.float32)
         np.testing.assert_allclose(lead * np.sign((lead * head).sum(axis=1))[:, None], head, atol=2e-3)
+
+
+def test_finalize_measures_what_the_planner_verified(device):
+    """The energy that a plan was accepted at is, bit for bit, what the finalize of the whole chunk
+    measures for its rows, though the planner's growth rounds measure few matrices at a time: a rank
+    verified at its target cannot miss it by the order of a sum."""
+    from reelcache_amd import node_packets as npk
+
+    model = _model(768, layers=20)
+    generator = torch.Generator(device=device).manual_seed(53)
+    sources, contexts = {}, {}
+    for index in range(40):
+        key = MatrixKey(index // 2, "KV"[index % 2])
+        sigma = torch.arange(1, 129, device=device, dtype=torch.float32) ** -(0.5 + 0.02 * index)
+        x = (torch.randn(1530, 128, device=device, generator=generator) * sigma) @ torch.randn(128, 768, device=device, generator=generator)
+        sources[key] = (x / 27.7 + 0.005 * torch.randn(1530, 768, device=device, generator=generator)).to(torch.bfloat16)
+        contexts[key] = _context(model, key, 1, 30, 51)
+    plan = _plan(_config(), device, sources, contexts)
+    assert len({p.rank_view for p in plan.plans.values()}) >= 3  # several rounds and rank classes
+    items = [npk.FinalizeItem(sources[key], p.new_rows[:p.rank_view].to(device), contexts[key],
+                              CodecSpec("svd_hevc", p.rank_view), key, p.target, False)
+             for key, p in plan.plans.items()]
+    for (tile, _), p in zip(npk.finalize_tiles(items, tile_rows=1024), plan.plans.values()):
+        assert tile.stored_energy == p.decision_energy >= p.target
