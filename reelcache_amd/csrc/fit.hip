@@ -465,7 +465,8 @@ __device__ __forceinline__ void project_ranks(const rch_fit_matrix* M, int chann
     for (int t = 0; t < TB; ++t)
 #pragma unroll
         for (int b = 0; b < NB; ++b) acc[t][b] = d4{};
-    auto products = [&](const Eight<DT> (&x)[TB], auto&& basis) __attribute__((always_inline)) {  // basis(b, s): channel s of rank block b
+    // basis(b, s): channel s of rank block b.
+    auto products = [&](const Eight<DT> (&x)[TB], auto&& basis) __attribute__((always_inline)) {
         double xv[TB][8];
 #pragma unroll
         for (int t = 0; t < TB; ++t)
@@ -652,9 +653,10 @@ __global__ void __launch_bounds__(64 * kProjectWaves<SHAPE>, 4) project_kernel(c
 // ---------------------------------------------------------------------------------------------
 // Residual energies on v_mfma_f64_16x16x4f64: D[m = token][n = channel] = sum_k P[token][k] Q[k][c].
 // Workgroup = some tokens of one matrix and every gridDim.z-th part of its 64-channel groups.  A group is
-// four 16 x 16 blocks per 16 tokens whose columns interleave: column i of block b is channel 4i + b of the group, so after the four blocks lane l (i = l % 16, g = l / 16) holds channels 4i ..
-// 4i + 3 of tokens g + 4v (v = 0..3, the f64 accumulator's row (l / 16) + 4v): X and the residual move
-// as 4-channel vectors, 16 lanes covering 64 contiguous channels of a row.  Per 16-rank step a lane
+// four 16 x 16 blocks per 16 tokens whose columns interleave: column i of block b is channel 4i + b of the
+// group, so after the four blocks lane l (i = l % 16, g = l / 16) holds channels 4i .. 4i + 3 of tokens
+// g + 4v (v = 0..3, the f64 accumulator's row (l / 16) + 4v): X and the residual move as 4-channel vectors,
+// 16 lanes covering 64 contiguous channels of a row.  Per 16-rank step a lane
 // takes P[token i][4g .. 4g + 3] (the A operand; MFMA step j takes rank 4g + j) and, for each j,
 // Q[4g + j][4i .. 4i + 3] (one 8-byte load: the B operands of the four blocks).
 //
