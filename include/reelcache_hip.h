@@ -20,7 +20,7 @@
 extern "C" {
 #endif
 
-#define RCH_ABI_VERSION 20
+#define RCH_ABI_VERSION 21
 
 /* Status codes (mapped to reelcache errors by the host). */
 #define RCH_OK 0
@@ -496,12 +496,12 @@ int rch_cholesky_inverse(const double* a_dev, double* x_dev, int32_t* info_dev, 
 
 /*
  * FP64 terms of a batch of stored basis views Q[:rank] (rank <= RCH_CHOLESKY_MAX_K, any mix), with
- * G = Q Q^T: energy_ptr gets float64 [6] = trace(G^-1 P^T P) (0 without coefficients), the Cholesky
+ * G = Q Q^T: energy_ptr gets float64 [7] = trace(G^-1 P^T P) (0 without coefficients), the Cholesky
  * status of G (0, or j + 1 as rch_cholesky_inverse), ||G - I||_inf, max |G_ii|, ||G||_inf, ||G^-1||_inf
- * (infinity when the status is not 0).  gram_ptr: float64 scratch [2, kp, kp], kp = rank rounded up to
- * 16; partial_ptr (with_coefficients): float64 scratch [RCH_SPAN_SPLITS]; resid_ptr: float64 [1] that gets
- * the seconds on the device from the start of G to the end of its terms (not of the trace), or 0.  Other
- * fields read: rows, basis_*, rank, coef_* (fp32 P).  max_rows / max_rank = the largest over the batch.
+ * (infinity when the status is not 0), and the seconds on the device from the start of G to the end of its
+ * terms (not of the trace).  gram_ptr: float64 scratch [2, kp, kp], kp = rank rounded up to
+ * 16; partial_ptr (with_coefficients): float64 scratch [RCH_SPAN_SPLITS].  Other fields read: rows, basis_*,
+ * rank, coef_* (fp32 P).  max_rows / max_rank = the largest over the batch.
  * Replaces the span energy of the final measurement (trace of the triangular solve,
  * reelcache/deferred_reads.py:682-714) and the Gram / Cholesky / inverse norms of the condition bounds
  * (reelcache/factorization.py:271-315).

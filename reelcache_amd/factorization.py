@@ -224,10 +224,10 @@ def project_onto_basis(tensor: torch.Tensor, basis: torch.Tensor, *, rank: int |
         raise
     view = stored[:rank].to(device=tensor.device)
     condition_started = time.perf_counter()
-    condition, terms, basis_keys, elapsed = _condition_bound, None, None, None
+    condition, terms, basis_keys = _condition_bound, None, None
     if condition is None and rank <= fit_kernels.CHOLESKY_MAX_K and stored.device == tensor.device:
         basis_keys = fit_kernels.absmax([stored])
-        terms, elapsed = fit_kernels.span_terms([view], [rank], seconds=True)
+        terms = fit_kernels.span_terms([view], [rank], seconds=True)
     else:
         validate_stored_basis(basis, tensor.shape[1])
         if condition is None:
@@ -240,7 +240,7 @@ def project_onto_basis(tensor: torch.Tensor, basis: torch.Tensor, *, rank: int |
     totals = fit_kernels.energies([tensor], keys, bases=[view], ranks=[rank], coefficients=[coefficients])
     parts = [keys.double(), extrema.double().view(-1), totals.view(-1)]
     if terms is not None:
-        parts += [basis_keys.double(), terms.view(-1), elapsed]
+        parts += [basis_keys.double(), terms.view(-1)]
     host = torch.cat(parts).cpu().numpy()
     bits = int(host[0])
     low, high = fit_kernels.split_keys(host[1:1 + 2 * rank].astype(np.int64).astype(np.int32), rank)

@@ -360,7 +360,7 @@ def span_terms(bases, ranks, coefficients=None, *, seconds: bool = False):
     """float64 ``[n, 6]`` of FP16 basis views ``Q = basis[:rank]`` (rank <= :data:`CHOLESKY_MAX_K`), with
     ``G = Q Q^T`` in FP64: ``trace(G^-1 P^T P)`` (0 without ``coefficients``), the Cholesky status of G
     (0 or the failing order), ``||G - I||_inf``, ``max |G_ii|``, ``||G||_inf`` and ``||G^-1||_inf``.  With
-    ``seconds`` also float64 ``[n]``: the device's time from the start of each G to the end of its terms."""
+    ``seconds`` ``[n, 7]``: also the device's time from the start of each G to the end of its terms."""
     device = _device(bases)
     ranks = [int(rank) for rank in ranks]
     if len(ranks) != len(bases) or not all(1 <= r <= min(CHOLESKY_MAX_K, b.shape[0]) for r, b in zip(ranks, bases)):
@@ -380,11 +380,8 @@ def span_terms(bases, ranks, coefficients=None, *, seconds: bool = False):
     work = torch.empty(total + n * (_SPAN_SPLITS + 7), dtype=torch.float64, device=device)
     table["gram_ptr"] = work.data_ptr() + 8 * firsts[:-1]
     table["partial_ptr"] = work.data_ptr() + 8 * (total + _SPAN_SPLITS * np.arange(n))
-    tail = work[total + n * _SPAN_SPLITS:]
-    terms = tail[:6 * n].view(n, 6)
-    table["energy_ptr"] = terms.data_ptr() + 48 * np.arange(n)
-    if seconds:
-        table["resid_ptr"] = terms.data_ptr() + 48 * n + 8 * np.arange(n)
+    terms = work[total + n * _SPAN_SPLITS:].view(n, 7)
+    table["energy_ptr"] = terms.data_ptr() + 56 * np.arange(n)
     max_rows = 0
     if coefficients is not None:
         if len(coefficients) != n or any(p.dtype != torch.float32 or p.ndim != 2 or p.shape[1] != rank or p.stride(1) != 1
@@ -398,7 +395,7 @@ def span_terms(bases, ranks, coefficients=None, *, seconds: bool = False):
     _lib.call("rch_fit_span", descriptors.data_ptr(), n, c8, max_rows, max(ranks), int(coefficients is not None),
               _stream(device))
     del keep
-    return (terms, tail[6 * n:]) if seconds else terms
+    return terms if seconds else terms[:, :6]
 
 
 def gaussian(blocks) -> None:
